@@ -437,8 +437,6 @@ __device__ __forceinline__ void load_v(const char* __restrict__ p, float (&v)[E]
     }
 }
 
-constexpr int kMergeRound = 16;  // partial blocks merged per round of loads
-
 __device__ __forceinline__ int64_t attn_part_index(int64_t t, int h, int s, int q_heads, int blocks) {
     return (t * q_heads + h) * blocks + s;
 }
@@ -546,46 +544,47 @@ __global__ __launch_bounds__(1024) void k_attention_blocks(const float* __restri
 }
 
 // Attention, pass 2: merge the blocks (of block_rows cache rows each) of one
-// (token, q head) in block order.
-template <int D>
-__global__ __launch_bounds__(D) void k_attention_merge(const float* __restrict__ part_ml, const float* __restrict__ part_acc,
-                                                       int q_heads, int blocks, int block_rows,
-                                                       const int32_t* __restrict__ position, int64_t max_positions,
-                                                       void* __restrict__ out, int odt) {
+// (token, q head). GROUPS groups of D threads take rounds of ROUND blocks in
+// turn and meet in LDS in group order. Bound by latency: every load of a round
+// is issued before any use, and the first round before the position is read
+// (block indices clamped to the grid's blocks; blocks past the position weigh
+// 0). 64 blocks of one token, 32 heads of 128: 3.6 us in eight groups, 7.1 us
+// in one (four rounds one after the other).
+template <int D, int ROUND, int GROUPS>
+__global__ __launch_bounds__(D * GROUPS) void k_attention_merge(
+    const float* __restrict__ part_ml, const float* __restrict__ part_acc, int q_heads, int blocks, int block_rows,
+    const int32_t* __restrict__ position, int64_t max_positions, void* __restrict__ out, int odt) {
     const int h = blockIdx.x;
     const int64_t t = blockIdx.y;
-    const int d = threadIdx.x;
+    const int d = threadIdx.x % D, group = threadIdx.x / D;
     const int64_t o = (t * q_heads + h) * D + d;
     const int64_t p0 = attn_part_index(t, h, 0, q_heads, blocks);
-    // Rounds of kMergeRound blocks: every load of a round is issued before any
-    // use, the first round before the position is read (block indices clamped
-    // to the grid's blocks; blocks past the position weigh 0), and rounds
-    // combine with a running max.
-    float mb[kMergeRound], lb[kMergeRound], ab[kMergeRound];
+    float mb[ROUND], lb[ROUND], ab[ROUND];
     const auto load_round = [&](const int b0, const int last) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < kMergeRound; ++i) {
+        for (int i = 0; i < ROUND; ++i) {
             const int64_t pb = p0 + (b0 + i < last ? b0 + i : last);
             mb[i] = part_ml[2 * pb];
             lb[i] = part_ml[2 * pb + 1];
             ab[i] = part_acc[pb * D + d];
         }
     };
-    load_round(0, blocks - 1);
+    const int first = group * ROUND;
+    load_round(first, blocks - 1);
     const int64_t pt = static_cast<int64_t>(position[0]) + t;
     const bool in_range = pt >= 0 && pt < max_positions;  // uniform
     const int nb = in_range ? static_cast<int>(pt / block_rows) + 1 : 1;
     float mrun = -INFINITY, lsum = 0.0f, acc = 0.0f;
-    for (int b0 = 0; b0 < nb; b0 += kMergeRound) {
-        if (b0 > 0) load_round(b0, nb - 1);
+    for (int b0 = first; b0 < nb; b0 += GROUPS * ROUND) {
+        if (b0 > first) load_round(b0, nb - 1);
         float mnew = mrun;
 #pragma unroll
-        for (int i = 0; i < kMergeRound; ++i) mnew = b0 + i < nb ? fmaxf(mnew, mb[i]) : mnew;
+        for (int i = 0; i < ROUND; ++i) mnew = b0 + i < nb ? fmaxf(mnew, mb[i]) : mnew;
         const float keep = nq::merge_exp(mrun - mnew);  // 0 in the first round
         lsum *= keep;
         acc *= keep;
 #pragma unroll
-        for (int i = 0; i < kMergeRound; ++i) {
+        for (int i = 0; i < ROUND; ++i) {
             if (b0 + i < nb) {  // a select: slots past the position may hold anything
                 const float f = nq::merge_exp(mb[i] - mnew);
                 lsum = fmaf(lb[i], f, lsum);
@@ -593,6 +592,24 @@ __global__ __launch_bounds__(D) void k_attention_merge(const float* __restrict__
             }
         }
         mrun = mnew;
+    }
+    if constexpr (GROUPS > 1) {
+        __shared__ float g_acc[GROUPS][D], g_m[GROUPS], g_l[GROUPS];
+        g_acc[group][d] = acc;
+        if (d == 0) g_m[group] = mrun, g_l[group] = lsum;
+        __syncthreads();
+        if (group > 0) return;
+        const int groups = nb < (GROUPS - 1) * ROUND + 1 ? (nb + ROUND - 1) / ROUND : GROUPS;  // that hold a block
+        float mnew = mrun;
+        for (int i = 1; i < groups; ++i) mnew = fmaxf(mnew, g_m[i]);
+        const float keep = nq::merge_exp(mrun - mnew);
+        lsum *= keep;
+        acc *= keep;
+        for (int i = 1; i < groups; ++i) {
+            const float f = nq::merge_exp(g_m[i] - mnew);
+            lsum = fmaf(g_l[i], f, lsum);
+            acc = fmaf(g_acc[i][d], f, acc);
+        }
     }
     if (!in_range) acc = 0.0f, lsum = 1.0f;
     nq::store_f32_as(out, odt, o, acc / lsum);
@@ -861,199 +878,423 @@ __global__ __launch_bounds__(kMfmaHeads * kWave) void k_decode_attention_mfma(
 }
 
 // ---------------------------------------------------------------------------
-// Prompt attention, pass 1 on MFMA (head_dim 128, four q heads per kv head,
-// 16-bit cache): workgroup (kv head g, tile of kPromptTile tokens, 64-row
-// cache block s); wave w computes q head 4g + w for the tile's tokens, the
-// same partial (m, l, acc) per (token, q head, block) as k_attention_blocks,
-// so k_attention_merge combines them unchanged.
-//   Scores S = Q K^T on v_mfma_f32_16x16x32 (bf16 / f16, the cache's type):
-//   A = the query rows (token i of the tile = row i), read from global memory
-//   and split into three 16-bit parts in registers (the rounding of q, of its
-//   remainder and of the remainder's remainder), all three accumulated into
-//   the same tile, so the product carries about 24 bits of the fp32 query; B =
-//   the block's K rows from LDS (exact). Four column tiles of 16 cache rows.
-//   Causal softmax per query row over the block (rows past the token's
-//   position weigh zero); the weights, split into three parts the same way,
-//   go through LDS into the A layout; O = P V with B = V staged transposed in
-//   LDS (one 16-byte read per lane), eight tiles of 16 dimensions.
-// Results differ from k_attention_blocks only by rounding.
-constexpr int kPromptTile = 16;                  // tokens per workgroup (A rows)
-constexpr int kPromptVStride = kSeqBlock + 8;    // halfs per transposed V row and per P row
+// Prompt attention on MFMA (16-bit cache, two tokens or more, any head_dim):
+// one pass over the cache with a running softmax, so no per-block partials
+// leave the chip. A unit is 16 tokens of one q head; a workgroup takes four
+// consecutive units of one kv head (the heads of a token tile, or, with fewer
+// than four q heads per kv head, further tiles), one wave each, which share
+// every K/V tile through LDS. HALVES = 2 adds four waves that take every
+// second tile for the same units, merged through LDS at the end.
+//   Scores are computed transposed, S^T = K Q^T on v_mfma_f32_16x16x32 (bf16 /
+//   f16, the cache's type): A = K rows from LDS (exact), B = the query, split
+//   into three 16-bit parts (the rounding of q, of its remainder and of the
+//   remainder's remainder: about 24 bits of the fp32 query) held in registers
+//   for the whole pass. Lane (kg, n) then holds token n's scores of cache rows
+//   16 ct + 4 kg + j: the softmax of a token is a reduction over a lane's
+//   registers and its three partner lanes, and the weights, split the same
+//   way, are already the B operand of O^T = V^T P^T when k slot 8 kg + e of a
+//   32-row step stands for row 16 (e / 4) + 4 kg + e % 4: they never go through LDS.
+//   V is staged transposed with its rows in that order (a thread moves 4 rows
+//   x 8 dimensions through registers), so an A fragment is one 16-byte read.
+// A tile's weighted values are summed on their own (small parts first) and
+// join the running output with one rounding: against 64 bits the output is
+// 1.1e-7 - 2.4e-7 off (rel-L2), 1.9e-7 - 4.0e-7 with per-block partials.
+// Bound by the matrix cores and the softmax beside them: 96 MFMAs (16 cycles)
+// and about 310 VALU instructions (four) per 16 tokens x 64 rows x 128
+// dimensions; 35% of the time is MFMA at 1531 tokens. Measured, 32 q heads,
+// 8 kv heads of 128, bf16 (per-block partials and a merge before): 512 tokens
+// 20 us (54), 1531 tokens after 517 cached 123 us (521), 16 / 8 heads 700
+// after 200 32 us (214), 8 / 4 heads of 256 700 tokens 51 us (181). Forming
+// the next tile's scores among this tile's softmax was slower (142 us): the
+// registers spill. So were three waves a SIMD (241 us).
+constexpr int kFlashTokens = 16;      // tokens per unit (B columns)
+constexpr int kFlashUnits = 4;        // units per workgroup
+
+// Cache rows per tile: K and V of a tile take 32 KB of registers in flight
+// over 256 threads (half that at head_dim 64).
+template <int D>
+constexpr int flash_rows() { return D == 256 ? 32 : 64; }
 
 template <int CT>
-constexpr size_t prompt_attention_mfma_lds() {
-    // K block [64][row], V transposed [128][64 + 8], weight parts [3][4 waves][16][64 + 8].
-    return static_cast<size_t>(kSeqBlock) * k_row_bytes<128, CT>() + 128 * kPromptVStride * 2 +
-           3 * kMfmaHeads * kPromptTile * kPromptVStride * 2;
+__device__ __forceinline__ uint32_t pack16(float a, float b) {
+    if constexpr (CT == NQ_DTYPE_BF16) {
+        typedef float v2f __attribute__((ext_vector_type(2)));
+        typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2b));
+    } else {
+        return to16<CT>(a) | (static_cast<uint32_t>(to16<CT>(b)) << 16);
+    }
 }
 
+// split3 of two values, part by part as packed pairs.
 template <int CT>
-__global__ __launch_bounds__(kMfmaHeads * kWave) void k_prompt_attention_mfma(
-    const float* __restrict__ q, const char* __restrict__ k_cache, const char* __restrict__ v_cache, int64_t tokens,
-    int kv_heads, const int32_t* __restrict__ position, int64_t max_positions, float scaling,
-    float* __restrict__ part_ml, float* __restrict__ part_acc) {
-    constexpr int D = 128;
-    constexpr int G = kMfmaHeads;
-    constexpr int T = kPromptTile;
-    constexpr int RB = k_row_bytes<D, CT>();  // padded K row in LDS
-    constexpr int VRB = D * 2;                // row in the cache
-    constexpr int PIECES = VRB / 16;
-    constexpr int VS = kPromptVStride;
+__device__ __forceinline__ void split3_pair(float a, float b, uint32_t (&h)[3]) {
+    h[0] = pack16<CT>(a, b);
+    a -= from16<CT>(static_cast<uint16_t>(h[0])), b -= from16<CT>(static_cast<uint16_t>(h[0] >> 16));
+    h[1] = pack16<CT>(a, b);
+    a -= from16<CT>(static_cast<uint16_t>(h[1])), b -= from16<CT>(static_cast<uint16_t>(h[1] >> 16));
+    h[2] = pack16<CT>(a, b);
+}
+
+// Max / sum over lanes n, n + 16, n + 32, n + 48 (every one of them gets it).
+__device__ __forceinline__ float column_max(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+__device__ __forceinline__ float column_sum(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+struct FlashArgs {
+    const float* q;
+    const char* k_cache;
+    const char* v_cache;
+    int64_t tokens;
+    int64_t max_positions;
+    const int32_t* position;
+    int q_heads, kv_heads;
+    int quads;             // workgroups per kv head and split
+    int tiles_per_split;
+    int splits;            // grid y; more than one leaves partials for k_attention_merge
+    float scaling;
+    void* out;
+    int odt;
+    int vec_out;           // out allows the four-element stores
+    float* part_ml;
+    float* part_acc;
+};
+
+template <int D, int CT, int HALVES>
+__global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const FlashArgs g) {
+    constexpr int R = flash_rows<D>();
+    constexpr int KB = 2 * D + 16;               // padded K row in LDS, bytes
+    constexpr int VS = R + 8;                    // 16-bit values per transposed V row
+    constexpr int kTileBytes = R * KB + D * VS * 2;
+    constexpr int kMergeBytes = HALVES == 2 ? (D / 4 + 2) * 256 * 4 : 0;
+    constexpr int kLds = HALVES * kTileBytes > kMergeBytes ? HALVES * kTileBytes : kMergeBytes;
+    constexpr int NS = D / 32;                   // 32-dimension steps of the scores
+    constexpr int NC = R / 16;                   // 16-row score tiles
+    constexpr int ND = D / 16;                   // 16-dimension output tiles
+    constexpr int KPT = R * D / 8 / 256;         // 16-byte K pieces per thread
+    constexpr int kQuads = R / 4 * (D / 8);      // V patches (4 rows x 8 dimensions)
+    static_assert(kQuads <= 256, "one V patch per thread");
     typedef typename Mfma16<CT>::v8 v8;
-    extern __shared__ float lds_raw[];
-    char* klds = reinterpret_cast<char*>(lds_raw);
-    uint16_t* vt = reinterpret_cast<uint16_t*>(klds + kSeqBlock * RB);  // [D][VS]
-    uint16_t* ps = vt + D * VS;                                         // [3][G][T][VS]
+    union Frag {
+        uint32_t u[4];
+        v8 v;
+    };
+    __shared__ __attribute__((aligned(16))) char lds[kLds];
+    __shared__ int wild[HALVES];  // a V value that is not finite, in a row some token of the tile may not see
 
-    const int q_heads = kv_heads * G;
-    const int g = static_cast<int>(blockIdx.x) % kv_heads;
-    const int64_t t0 = static_cast<int64_t>(blockIdx.x / kv_heads) * T;
-    const int s = blockIdx.y;
-    const int blocks = gridDim.y;
-    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int group = g.q_heads / g.kv_heads;
+    const int kvh = static_cast<int>(blockIdx.x) % g.kv_heads;
+    // The longest units first: what is left at the end is short.
+    const int quad = g.quads - 1 - static_cast<int>(blockIdx.x) / g.kv_heads;
+    const int split = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     const int lane = threadIdx.x & (kWave - 1);
-    const int64_t p0 = position[0];
-    const int64_t row0 = static_cast<int64_t>(s) * kSeqBlock;
-    const int64_t t_end = t0 + T < tokens ? t0 + T : tokens;
-    // Highest cache row any query of this workgroup may see.
-    int64_t last = p0 + t_end - 1;
-    if (last >= max_positions) last = max_positions - 1;
-    if (p0 < 0 || row0 > last) return;  // uniform: no query of this workgroup reaches row0
-    const int rows = static_cast<int>((last - row0 + 1) < kSeqBlock ? (last - row0 + 1) : kSeqBlock);
-
-    // Query operands: lane (kg, n) holds token row n, dimensions 32 st + 8 kg + [0, 8).
     const int n = lane & 15, kg = lane >> 4;
-    const int h = g * G + w;
-    const int64_t tq = t0 + n < tokens ? t0 + n : tokens - 1;  // rows past the last token reuse it (not stored)
-    float qf[4][8];
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-        const float4* src = reinterpret_cast<const float4*>(q + (tq * q_heads + h) * D + 32 * st + 8 * kg);
-        const float4 x0 = src[0], x1 = src[1];
-        qf[st][0] = x0.x; qf[st][1] = x0.y; qf[st][2] = x0.z; qf[st][3] = x0.w;
-        qf[st][4] = x1.x; qf[st][5] = x1.y; qf[st][6] = x1.z; qf[st][7] = x1.w;
-    }
-    // K rows [row0, row0 + rows) to LDS as stored, V transposed; rows past
-    // `rows` are zero (their weights are zero, and 0 * V must stay 0).
-    const int64_t head_row0 = static_cast<int64_t>(g) * max_positions + row0;
-    const char* kbase = k_cache + head_row0 * VRB;
-    const char* vbase = v_cache + head_row0 * VRB;
-    constexpr int PER_THREAD = kSeqBlock * PIECES / (G * kWave);
-    u32x4 kp[PER_THREAD], vp[PER_THREAD];
-#pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) {
-        const int idx = static_cast<int>(threadIdx.x) + i * G * kWave;
-        const int r = idx % kSeqBlock, c = idx / kSeqBlock;
-        const int rr = r < rows ? r : rows - 1;
-        kp[i] = *reinterpret_cast<const u32x4*>(kbase + static_cast<int64_t>(rr) * VRB + 16 * c);
-        vp[i] = *reinterpret_cast<const u32x4*>(vbase + static_cast<int64_t>(rr) * VRB + 16 * c);
-    }
-#pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) {
-        const int idx = static_cast<int>(threadIdx.x) + i * G * kWave;
-        const int r = idx % kSeqBlock, c = idx / kSeqBlock;
-        const bool keep = r < rows;
-        const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
-        *reinterpret_cast<u32x4*>(klds + r * RB + 16 * c) = keep ? kp[i] : zero;
-        const u32x4 vv = keep ? vp[i] : zero;
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            vt[(8 * c + e) * VS + r] = static_cast<uint16_t>((vv[e >> 1] >> (16 * (e & 1))) & 0xffffu);
-    }
-    v8 qa[3][4];
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-        union {
-            uint16_t h[8];
-            v8 v;
-        } part[3];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            uint16_t hh[3];
-            split3<CT>(qf[st][e], hh);
-#pragma unroll
-            for (int pp = 0; pp < 3; ++pp) part[pp].h[e] = hh[pp];
-        }
-#pragma unroll
-        for (int pp = 0; pp < 3; ++pp) qa[pp][st] = part[pp].v;
-    }
-    __syncthreads();
+    const int half = wave >> 2;
+    const int ht = threadIdx.x & 255;  // thread within the half
+    const int units = static_cast<int>((g.tokens + kFlashTokens - 1) / kFlashTokens) * group;
+    const int unit0 = quad * kFlashUnits;
+    const int unit_last = unit0 + kFlashUnits - 1 < units ? unit0 + kFlashUnits - 1 : units - 1;
+    const bool unit_ok = unit0 + (wave & 3) <= unit_last;
+    const int unit = unit_ok ? unit0 + (wave & 3) : unit_last;
+    const int h = kvh * group + unit % group;
+    const int64_t t0 = static_cast<int64_t>(unit / group) * kFlashTokens;
+    const int64_t t = t0 + n;
+    const int64_t p0 = g.position[0];
+    const int64_t pt = p0 + t;  // the last row token n sees
+    constexpr uint32_t kExp = CT == NQ_DTYPE_BF16 ? 0x7f80u : 0x7c00u;  // exponent of an infinity or NaN
+    const int64_t t_first = static_cast<int64_t>(unit0 / group) * kFlashTokens;
+    const int64_t t_end = (static_cast<int64_t>(unit_last / group) + 1) * kFlashTokens;
+    int64_t last_row = p0 + (t_end < g.tokens ? t_end : g.tokens) - 1;
+    last_row = last_row < g.max_positions ? last_row : g.max_positions - 1;
+    // The last row that any token of the workgroup sees and that every one
+    // does (the host bounds the cache below 2^22 rows).
+    const int last = static_cast<int>(last_row), first = static_cast<int>(p0 + t_first);
+    int tile = split * g.tiles_per_split;
+    int tile_end = p0 < 0 || p0 + t_first >= g.max_positions ? 0 : static_cast<int>(last / R) + 1;
+    tile_end = tile_end < tile + g.tiles_per_split ? tile_end : tile + g.tiles_per_split;
 
-    // Scores: sc[ct][j] = S[token row 4 kg + j][cache row 16 ct + n].
-    v4f_t sc[4];
-#pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-        sc[ct] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            const v8 b = *reinterpret_cast<const v8*>(klds + (16 * ct + n) * RB + 2 * (32 * st + 8 * kg));
-#pragma unroll
-            for (int pp = 0; pp < 3; ++pp) sc[ct] = mfma16<CT>(qa[pp][st], b, sc[ct]);
-        }
-    }
-    // Causal softmax per token row over this block.
-    float mrow[4], lrow[4];
-    uint16_t* pw = ps + w * T * VS;  // this wave's [T][VS] for part 0; parts are G * T * VS apart
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int i = 4 * kg + j;  // token row of the tile
-        const int64_t pt = p0 + t0 + i;
-        float sv[4];
-        float mx = -INFINITY;
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct) {
-            const int cr = 16 * ct + n;
-            const bool valid = cr < rows && row0 + cr <= pt;
-            sv[ct] = valid ? sc[ct][j] * scaling : -INFINITY;
-            mx = fmaxf(mx, sv[ct]);
-        }
-        const float m = row16_max(mx);
-        const float msafe = m == -INFINITY ? 0.0f : m;
-        float lsum = 0.0f;
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct) {
-            const float pv = sv[ct] == -INFINITY ? 0.0f : expf(sv[ct] - msafe);
-            lsum += pv;
-            uint16_t hh[3];
-            split3<CT>(pv, hh);
-#pragma unroll
-            for (int pp = 0; pp < 3; ++pp) pw[pp * G * T * VS + i * VS + 16 * ct + n] = hh[pp];
-        }
-        mrow[j] = m;
-        lrow[j] = row16_sum(lsum);
-    }
-    __syncthreads();
+    char* const klds = lds + half * kTileBytes;
+    uint16_t* const vt = reinterpret_cast<uint16_t*>(klds + R * KB);
+    const int64_t head0 = static_cast<int64_t>(kvh) * g.max_positions;
+    const char* const k_head = g.k_cache + head0 * (2 * D);
+    const char* const v_head = g.v_cache + head0 * (2 * D);
 
-    // O = P V: o[dt][j] = O[token row 4 kg + j][dimension 16 dt + n].
-    v4f_t o[8];
+    // Query operand: token n, dimensions 32 st + 8 kg + [0, 8), in three parts.
+    Frag qa[3][NS];
+    {
+        const float* qp = g.q + ((t < g.tokens ? t : g.tokens - 1) * g.q_heads + h) * D + 8 * kg;
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o[dt] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int st = 0; st < NS; ++st) {
+            const float4 a = *reinterpret_cast<const float4*>(qp + 32 * st);
+            const float4 b = *reinterpret_cast<const float4*>(qp + 32 * st + 4);
+            const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-    for (int kst = 0; kst < kSeqBlock / 32; ++kst) {
-        v8 pa[3];
+            for (int e = 0; e < 4; ++e) {
+                uint32_t hh[3];
+                split3_pair<CT>(x[2 * e], x[2 * e + 1], hh);
 #pragma unroll
-        for (int pp = 0; pp < 3; ++pp)
-            pa[pp] = *reinterpret_cast<const v8*>(pw + pp * G * T * VS + n * VS + 32 * kst + 8 * kg);
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-            const v8 b = *reinterpret_cast<const v8*>(vt + (16 * dt + n) * VS + 32 * kst + 8 * kg);
-#pragma unroll
-            for (int pp = 0; pp < 3; ++pp) o[dt] = mfma16<CT>(pa[pp], b, o[dt]);
+                for (int p = 0; p < 3; ++p) qa[p][st].u[e] = hh[p];
+            }
         }
     }
-    // Partials of the tokens that reach this block (the merge reads block s of
-    // token t only when row0 <= position + t).
+
+    // This thread's V patch: rows 4 vq + [0, 4), dimensions 8 vc + [0, 8); the
+    // rows' slots within the 32-row step t are 8 kg + 4 eh + [0, 4).
+    const int vq = ht % (R / 4), vc = ht / (R / 4);
+    const int v_slot = 32 * (vq >> 3) + 8 * (vq & 3) + 4 * ((vq >> 2) & 1);
+    const bool v_on = kQuads == 256 || ht < kQuads;
+    u32x4 kp[KPT], vp[4];
+    const auto load_tile = [&](int kt) __attribute__((always_inline)) {
+        const int row0 = kt * R;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int64_t t = t0 + 4 * kg + j;
-        const int64_t pt = p0 + t;
-        if (t >= tokens || pt < row0 || pt >= max_positions) continue;
-        const int64_t pi = attn_part_index(t, h, s, q_heads, blocks);
+        for (int i = 0; i < KPT; ++i) {
+            const int piece = ht + 256 * i;
+            const int r = row0 + piece / (D / 8);
+            kp[i] = *reinterpret_cast<const u32x4*>(
+                k_head + (static_cast<uint32_t>(r < last ? r : last) * (2 * D) + 16 * (piece % (D / 8))));
+        }
+        if (v_on) {
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) part_acc[pi * D + 16 * dt + n] = o[dt][j];
-        if (n == 0) {
-            part_ml[2 * pi] = mrow[j];
-            part_ml[2 * pi + 1] = lrow[j];
+            for (int i = 0; i < 4; ++i) {
+                const int r = row0 + 4 * vq + i;
+                vp[i] = *reinterpret_cast<const u32x4*>(
+                    v_head + (static_cast<uint32_t>(r < last ? r : last) * (2 * D) + 16 * vc));
+            }
+        }
+    };
+    // Rows past `last` are stored as zeros: their weights are zero, and 0 * V
+    // must stay 0. So are infinities and NaNs in the rows that not every token
+    // of the workgroup sees: the loop below adds those where they belong.
+    const auto store_tile = [&](int kt) __attribute__((always_inline)) {
+        const int row0 = kt * R;
+#pragma unroll
+        for (int i = 0; i < KPT; ++i) {
+            const int piece = ht + 256 * i;
+            *reinterpret_cast<u32x4*>(klds + (piece / (D / 8)) * KB + 16 * (piece % (D / 8))) = kp[i];
+        }
+        if (v_on) {
+            if (row0 + R - 1 > first) {
+                bool bad = false;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int r = row0 + 4 * vq + i;
+                    if (r > last) vp[i] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const bool lo = (vp[i][e] & kExp) == kExp, hi = ((vp[i][e] >> 16) & kExp) == kExp;
+                        bad |= r > first && (lo || hi);
+                        if (r > first) vp[i][e] &= (lo ? 0u : 0xffffu) | (hi ? 0u : 0xffff0000u);
+                    }
+                }
+                if (bad) wild[half] = 1;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+                uint2 w;
+                w.x = __builtin_amdgcn_perm(vp[1][e >> 1], vp[0][e >> 1], sel);
+                w.y = __builtin_amdgcn_perm(vp[3][e >> 1], vp[2][e >> 1], sel);
+                *reinterpret_cast<uint2*>(vt + (8 * vc + e) * VS + v_slot) = w;
+            }
+        }
+    };
+
+    if (threadIdx.x < HALVES) wild[threadIdx.x] = 0;
+    const float c = g.scaling * 1.4426950408889634f;  // weights are 2^(c s - c max)
+    v4f_t o[ND];
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) o[dt] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+    float m = -INFINITY, mc = 0.0f, l = 0.0f;  // running max of s, c * max (0 before any row), this lane's sum
+    if (tile + half < tile_end) load_tile(tile + half);
+    for (; tile < tile_end; tile += HALVES) {
+        const int kt = tile + half;
+        const bool on = kt < tile_end;  // uniform per wave
+        __syncthreads();
+        if (on) store_tile(kt);
+        __syncthreads();
+        if (kt + HALVES < tile_end) load_tile(kt + HALVES);
+        if (!on) continue;
+        const int row0 = kt * R;
+        if (row0 > p0 + t0 + kFlashTokens - 1) continue;  // uniform per wave: no token of the unit reaches the tile
+        const bool edge = row0 + R - 1 > p0 + t0;          // some token does not see every row
+        // The query's high part and its small parts in sums of their own: a
+        // score takes NS + 1 roundings at its own size instead of 3 NS.
+        // Consecutive MFMAs add to different accumulators.
+        v4f_t s[NC], lo[NC];
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) s[ct] = lo[ct] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            v8 a[NC];
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct)
+                a[ct] = *reinterpret_cast<const v8*>(klds + (16 * ct + n) * KB + 64 * st + 16 * kg);
+#pragma unroll
+            for (int p = 2; p >= 0; --p)
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct) {
+                    v4f_t& sum = p == 0 ? s[ct] : lo[ct];
+                    sum = mfma16<CT>(a[ct], qa[p][st].v, sum);
+                }
+        }
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) s[ct] += lo[ct];
+        if (edge) {
+            const int seen = static_cast<int>(pt - row0 < R ? pt - row0 : R);
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s[ct][j] = 16 * ct + 4 * kg + j <= seen ? s[ct][j] : -INFINITY;
+        }
+        float mx = m;
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[ct][j]);
+        mx = column_max(mx);
+        const float mc_new = mx == -INFINITY ? 0.0f : mx * c;
+        const float keep = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mc - mc_new);
+        m = mx;
+        mc = mc_new;
+        float lt = 0.0f;
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                s[ct][j] = __builtin_amdgcn_exp2f(fmaf(s[ct][j], c, -mc));
+                lt += s[ct][j];
+            }
+        l = fmaf(l, keep, lt);
+        Frag pa[3][R / 32];
+#pragma unroll
+        for (int ks = 0; ks < R / 32; ++ks)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t hh[3];
+                split3_pair<CT>(s[2 * ks + (e >> 1)][2 * (e & 1)], s[2 * ks + (e >> 1)][2 * (e & 1) + 1], hh);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) pa[p][ks].u[e] = hh[p];
+            }
+        // A tile's products on their own, small parts first, then one rounding
+        // into the running output.
+#pragma unroll
+        for (int d0 = 0; d0 < ND; d0 += 4) {
+            v4f_t y[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int p = 2; p >= 0; --p)
+#pragma unroll
+                for (int ks = 0; ks < R / 32; ++ks)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const v8 a = *reinterpret_cast<const v8*>(vt + (16 * (d0 + i) + n) * VS + 32 * ks + 8 * kg);
+                        y[i] = mfma16<CT>(a, pa[p][ks].v, y[i]);
+                    }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[d0 + i][j] = fmaf(o[d0 + i][j], keep, y[i][j]);
+        }
+        if (edge && wild[half]) {
+            // The values that store_tile left out, for the tokens that see their rows.
+            const int r_end = last < row0 + R - 1 ? last : row0 + R - 1;
+            for (int r = row0 > first ? row0 : first + 1; r <= r_end; ++r) {
+                const int rr = r - row0;
+                float w = 0.0f;
+#pragma unroll
+                for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) w = rr >> 4 == ct && (rr & 3) == j ? s[ct][j] : w;
+                w = __shfl(w, 16 * ((rr >> 2) & 3) + n, kWave);
+                const uint16_t* vr = reinterpret_cast<const uint16_t*>(v_head) + static_cast<uint32_t>(r) * D + 4 * kg;
+#pragma unroll
+                for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t x = vr[16 * dt + i];
+                        if (r <= pt && (x & kExp) == kExp)
+                            o[dt][i] = fmaf(w, from16<CT>(static_cast<uint16_t>(x)), o[dt][i]);
+                    }
+            }
+        }
+    }
+
+    if constexpr (HALVES == 2) {
+        // The second half's max, sum and sums join the first's, lane by lane.
+        float* const mg = reinterpret_cast<float*>(lds) + ht;
+        __syncthreads();
+        if (half == 1) {
+            mg[0] = m;
+            mg[256] = mc;
+#pragma unroll
+            for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mg[(2 + 4 * dt + i) * 256] = o[dt][i];
+        }
+        __shared__ float l_other[256];
+        if (half == 1) l_other[ht] = l;
+        __syncthreads();
+        if (half == 1) return;
+        const float m2 = mg[0], mc2 = mg[256];
+        const float mcn = m2 > m ? mc2 : mc;
+        const float f1 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mc - mcn);
+        const float f2 = m2 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mc2 - mcn);
+        l = l * f1 + l_other[ht] * f2;
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[dt][i] = o[dt][i] * f1 + mg[(2 + 4 * dt + i) * 256] * f2;
+        m = m2 > m ? m2 : m;
+        mc = mcn;
+    }
+    l = column_sum(l);
+    if (!unit_ok || t >= g.tokens) return;
+    if (g.splits > 1) {
+        if (pt < static_cast<int64_t>(split) * g.tiles_per_split * R || pt >= g.max_positions || p0 < 0) return;
+        const int64_t pi = attn_part_index(t, h, split, g.q_heads, g.splits);
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) *reinterpret_cast<v4f_t*>(g.part_acc + pi * D + 16 * dt + 4 * kg) = o[dt];
+        if (kg == 0) {
+            g.part_ml[2 * pi] = m == -INFINITY ? m : mc * 0.69314718055994531f;
+            g.part_ml[2 * pi + 1] = l;
+        }
+        return;
+    }
+    const bool in_range = p0 >= 0 && pt < g.max_positions;  // tokens outside the cache: zero
+    const int64_t out0 = (t * g.q_heads + h) * D + 4 * kg;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) {
+        v4f_t y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = in_range ? o[dt][i] / l : 0.0f;
+        const int64_t oi = out0 + 16 * dt;
+        if (g.odt == NQ_DTYPE_F32) {
+            float* const dst = static_cast<float*>(g.out) + oi;
+            if (g.vec_out) *reinterpret_cast<v4f_t*>(dst) = y;
+            else dst[0] = y[0], dst[1] = y[1], dst[2] = y[2], dst[3] = y[3];
+        } else {
+            uint16_t* const dst = static_cast<uint16_t*>(g.out) + oi;
+            uint2 w;
+            w.x = pack2(g.odt, y[0], y[1]);
+            w.y = pack2(g.odt, y[2], y[3]);
+            if (g.vec_out) {
+                *reinterpret_cast<uint2*>(dst) = w;
+            } else {
+                dst[0] = static_cast<uint16_t>(w.x), dst[1] = static_cast<uint16_t>(w.x >> 16);
+                dst[2] = static_cast<uint16_t>(w.y), dst[3] = static_cast<uint16_t>(w.y >> 16);
+            }
         }
     }
 }
@@ -1438,27 +1679,105 @@ int64_t proj_workgroups(int64_t vocab, int64_t hidden) {
 
 int attention_blocks(int64_t max_positions) { return static_cast<int>((max_positions + kSeqBlock - 1) / kSeqBlock); }
 
+// How a prompt attention of `groups` workgroups (four units each) over up to
+// `tiles` cache tiles is laid out.
+struct FlashPlan {
+    int halves;
+    int64_t splits, tiles_per_split;
+};
+
+// Fewer than 128 workgroups leave most of the chip idle: their cache goes to
+// several (two tiles each or more, up to 16 and to 512 workgroups in all) when
+// it is long enough to pay for the merge: 17 tokens after 1000 (16 workgroups)
+// 13 us split, 30 us not; 128 after 3000 (64) 39 and 75 us; 256 after 1000
+// (128) 35 us either way; 64 after none (32, 640-row cache) 10 and 9 us. Below
+// 512, eight waves share a workgroup's cache between them (17 after 1000: 30
+// us against 35 in four; 1024 tokens, 512 workgroups: 44 either way).
+FlashPlan flash_plan(int64_t groups, int64_t tiles) {
+    FlashPlan p;
+    int64_t want = groups < 128 && tiles >= 8 ? 512 / groups : 1;
+    want = want < tiles / 2 ? want : tiles / 2;
+    want = want < 16 ? want : 16;
+    want = want > 1 ? want : 1;
+    p.tiles_per_split = (tiles + want - 1) / want;
+    p.splits = (tiles + p.tiles_per_split - 1) / p.tiles_per_split;
+    p.halves = groups < 512 && p.splits == 1 ? 2 : 1;
+    return p;
+}
+
+// Prompt attention over a 16-bit cache. The grid is four units (16 tokens of a
+// q head) a workgroup.
+template <int D, int CT>
+int launch_prompt_attention(const float* q, const void* kc, const void* vc, int64_t tokens, int q_heads, int kv_heads,
+                            const int32_t* position, int64_t max_positions, float scaling, void* out, int odt,
+                            float* ws, hipStream_t st) {
+    constexpr int R = flash_rows<D>();
+    const int group = q_heads / kv_heads;
+    const int64_t units = (tokens + kFlashTokens - 1) / kFlashTokens * group;
+    const int64_t quads = (units + kFlashUnits - 1) / kFlashUnits;
+    const int64_t groups = quads * kv_heads;
+    if (groups > 0x7fffffff) return NQ_ERR_SHAPE;
+    const int64_t tiles = (max_positions + R - 1) / R;
+    const FlashPlan plan = flash_plan(groups, tiles);
+    FlashArgs a;
+    a.q = q;
+    a.k_cache = static_cast<const char*>(kc);
+    a.v_cache = static_cast<const char*>(vc);
+    a.tokens = tokens;
+    a.max_positions = max_positions;
+    a.position = position;
+    a.q_heads = q_heads;
+    a.kv_heads = kv_heads;
+    a.quads = static_cast<int>(quads);
+    a.tiles_per_split = static_cast<int>(plan.tiles_per_split);
+    a.splits = static_cast<int>(plan.splits);
+    a.scaling = scaling;
+    a.out = out;
+    a.odt = odt;
+    a.vec_out = aligned16(out) ? 1 : 0;
+    a.part_acc = ws;
+    a.part_ml = ws + tokens * q_heads * plan.splits * D;
+    const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(plan.splits));
+    if (plan.halves == 2)
+        hipLaunchKernelGGL((k_prompt_attention<D, CT, 2>), grid, dim3(512), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_prompt_attention<D, CT, 1>), grid, dim3(256), 0, st, a);
+    if (plan.splits > 1) {
+        if (hipGetLastError() != hipSuccess) return NQ_ERR_LAUNCH;
+        hipLaunchKernelGGL((k_attention_merge<D, 4, 1>), dim3(q_heads, static_cast<unsigned>(tokens)), dim3(D), 0, st,
+                           a.part_ml, a.part_acc, q_heads, a.splits, a.tiles_per_split * R, position, max_positions,
+                           out, odt);
+    }
+    return nq::launch_status();
+}
+
+// Merge of the 64-row blocks' partials. One token has few (token, head) rows,
+// so more than one round of blocks goes to several groups of threads.
+template <int D>
+int launch_merge(const float* ml, const float* acc, int64_t tokens, int q_heads, int blocks, const int32_t* position,
+                 int64_t max_positions, void* out, int odt, hipStream_t st) {
+    constexpr int kGroups = 1024 / D;
+    const dim3 grid(static_cast<unsigned>(q_heads), static_cast<unsigned>(tokens));
+    if (tokens == 1 && blocks > 16)
+        hipLaunchKernelGGL((k_attention_merge<D, 8, kGroups>), grid, dim3(D * kGroups), 0, st, ml, acc, q_heads, blocks,
+                           kSeqBlock, position, max_positions, out, odt);
+    else
+        hipLaunchKernelGGL((k_attention_merge<D, 16, 1>), grid, dim3(D), 0, st, ml, acc, q_heads, blocks, kSeqBlock,
+                           position, max_positions, out, odt);
+    return nq::launch_status();
+}
+
 template <int D, int CT>
 int launch_attention(const float* q, const void* kc, const void* vc, int64_t tokens, int q_heads, int kv_heads,
                      const int32_t* position, int64_t max_positions, float scaling, void* out, int odt, float* ml,
                      float* acc, hipStream_t st) {
+    if constexpr (CT != NQ_DTYPE_F32) {
+        if (tokens > 1)
+            return launch_prompt_attention<D, CT>(q, kc, vc, tokens, q_heads, kv_heads, position, max_positions,
+                                                  scaling, out, odt, ml, st);
+    }
     const int group = q_heads / kv_heads;
     const int blocks = attention_blocks(max_positions);
-    if constexpr (D == 128 && CT != NQ_DTYPE_F32) {
-        if (group == kMfmaHeads && tokens > 1) {
-            const int64_t qblocks = (tokens + kPromptTile - 1) / kPromptTile;
-            if (qblocks * kv_heads > 0x7fffffff) return NQ_ERR_SHAPE;
-            dim3 grid(static_cast<unsigned>(qblocks * kv_heads), static_cast<unsigned>(blocks));
-            hipLaunchKernelGGL((k_prompt_attention_mfma<CT>), grid, dim3(kMfmaHeads * kWave),
-                               prompt_attention_mfma_lds<CT>(), st, q, static_cast<const char*>(kc),
-                               static_cast<const char*>(vc), tokens, kv_heads, position, max_positions, scaling, ml,
-                               acc);
-            if (hipGetLastError() != hipSuccess) return NQ_ERR_LAUNCH;
-            hipLaunchKernelGGL(k_attention_merge<D>, dim3(q_heads, static_cast<unsigned>(tokens)), dim3(D), 0, st, ml,
-                               acc, q_heads, blocks, kSeqBlock, position, max_positions, out, odt);
-            return nq::launch_status();
-        }
-    }
     const int qt = tokens == 1 ? 1 : 16;
     const int64_t qblocks = (tokens + qt - 1) / qt;
     const size_t lds = attention_lds<D, CT>(group);
@@ -1469,9 +1788,7 @@ int launch_attention(const float* q, const void* kc, const void* vc, int64_t tok
                        static_cast<const char*>(kc), static_cast<const char*>(vc), tokens, q_heads, kv_heads, qt,
                        position, max_positions, scaling, ml, acc);
     if (hipGetLastError() != hipSuccess) return NQ_ERR_LAUNCH;
-    hipLaunchKernelGGL(k_attention_merge<D>, dim3(q_heads, static_cast<unsigned>(tokens)), dim3(D), 0, st, ml, acc,
-                       q_heads, blocks, kSeqBlock, position, max_positions, out, odt);
-    return nq::launch_status();
+    return launch_merge<D>(ml, acc, tokens, q_heads, blocks, position, max_positions, out, odt, st);
 }
 
 template <int D>
@@ -1533,9 +1850,7 @@ int launch_decode_attention_g(const float* q, const float* k, const float* v, in
     }
     if (hipGetLastError() != hipSuccess) return NQ_ERR_LAUNCH;
     if (!merge) return NQ_OK;  // the partials stay in the workspace
-    hipLaunchKernelGGL(k_attention_merge<D>, dim3(kv_heads * G, 1), dim3(D), 0, st, ml, acc, kv_heads * G, blocks,
-                       kSeqBlock, position, max_positions, out, odt);
-    return nq::launch_status();
+    return launch_merge<D>(ml, acc, 1, kv_heads * G, blocks, position, max_positions, out, odt, st);
 }
 
 template <int D, int CT>

@@ -149,7 +149,7 @@ def reference_attention(q, kc, vc, start, scaling):
         (37, 5, 32, 8, 128, torch.bfloat16),
         (512, 0, 32, 8, 128, torch.bfloat16),
         (100, 27, 8, 1, 64, torch.float32),
-        # MFMA prompt path (head_dim 128, four q heads per kv head, 16-bit cache):
+        # MFMA prompt path (16-bit cache, two tokens or more):
         # tile edges, the last cache rows, f16, other kv head counts
         (16, 0, 32, 8, 128, torch.bfloat16),
         (17, 63, 32, 8, 128, torch.bfloat16),
@@ -174,6 +174,83 @@ def test_attention(tokens, start, q_heads, kv_heads, head_dim, cache_dtype):
     again = ops.launch_attention(q.to(DEV), kc.to(DEV), vc.to(DEV), position=position, scaling=scaling,
                                  out_dtype=torch.float32)
     assert torch.equal(out, again)
+
+
+@pytest.mark.parametrize("cache_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "tokens,start,q_heads,kv_heads,head_dim,max_pos",
+    [
+        # fewer and more q heads per kv head than a workgroup's four units, ragged counts among them
+        (2, 0, 4, 4, 64, 2),
+        (15, 1, 4, 4, 64, 40),
+        (65, 62, 2, 2, 64, 130),
+        (31, 33, 16, 8, 128, 64),
+        (49, 500, 6, 2, 128, 549),
+        (17, 3, 10, 2, 64, 33),
+        (33, 31, 8, 1, 128, 640),
+        (129, 0, 16, 1, 64, 129),
+        # 32-row tiles
+        (16, 16, 8, 4, 256, 32),
+        (47, 18, 8, 4, 256, 65),
+        # one wave half without a tile, split cache with a merge, splits past the position
+        (20, 0, 32, 8, 128, 4096),
+        (17, 1000, 16, 4, 128, 1200),
+        (18, 2100, 8, 2, 256, 2200),
+        # enough tokens for one half per workgroup
+        (1040, 37, 32, 8, 128, 1077),
+        (1030, 5, 16, 16, 64, 1050),
+    ],
+)
+def test_prompt_attention_tiles(tokens, start, q_heads, kv_heads, head_dim, max_pos, cache_dtype):
+    """The one-pass prompt attention against fp32 at the edges of its units,
+    tiles and splits; a second call gives the same bits, a misaligned output too."""
+
+    g = _g(14)
+    kc = torch.randn(kv_heads, max_pos, head_dim, generator=g).to(cache_dtype)
+    vc = torch.randn(kv_heads, max_pos, head_dim, generator=g).to(cache_dtype)
+    q = 2 * torch.randn(tokens, q_heads, head_dim, generator=g)
+    position = torch.tensor([start], dtype=torch.int32, device=DEV)
+    call = dict(position=position, scaling=head_dim**-0.5)
+    qd, kd, vd = q.to(DEV), kc.to(DEV), vc.to(DEV)
+    out = ops.launch_attention(qd, kd, vd, out_dtype=torch.float32, **call)
+    assert relative_l2(out.cpu(), reference_attention(q, kc, vc, start, call["scaling"])) < 1e-5
+    store = torch.empty(out.numel() + 1, dtype=torch.float32, device=DEV)[1:]
+    assert torch.equal(ops.launch_attention(qd, kd, vd, out=store, **call).view_as(out), out)
+    half = torch.empty(out.numel() + 1, dtype=torch.bfloat16, device=DEV)[1:]
+    assert torch.equal(ops.launch_attention(qd, kd, vd, out=half, **call).view_as(out), out.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(8, 2, 128), (4, 4, 64)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_prompt_attention_non_finite_value_is_causal(q_heads, kv_heads, head_dim, value):
+    """A value row that is not finite reaches the tokens that see it and no other."""
+
+    g = _g(15)
+    tokens, start, max_pos, row, dim = 70, 11, 96, 50, 37
+    kc = torch.randn(kv_heads, max_pos, head_dim, generator=g).to(torch.bfloat16).to(DEV)
+    vc = torch.randn(kv_heads, max_pos, head_dim, generator=g).to(torch.bfloat16).to(DEV)
+    q = 2 * torch.randn(tokens, q_heads, head_dim, generator=g).to(DEV)
+    call = dict(position=torch.tensor([start], dtype=torch.int32, device=DEV), scaling=head_dim**-0.5,
+                out_dtype=torch.float32)
+    base = ops.launch_attention(q, kc, vc, **call).view(tokens, q_heads, head_dim)
+    vc[1, row, dim] = value
+    out = ops.launch_attention(q, kc, vc, **call).view(tokens, q_heads, head_dim)
+    group = q_heads // kv_heads
+    hit = torch.zeros_like(base, dtype=torch.bool)
+    hit[row - start:, group:2 * group, dim] = True
+    assert torch.equal(out[~hit], base[~hit])
+    assert not torch.isfinite(out[hit]).any()
+
+
+def test_prompt_attention_tokens_outside_the_cache_are_zero():
+    g = _g(16)
+    kc = torch.randn(2, 40, 128, generator=g).to(torch.bfloat16).to(DEV)
+    q = torch.randn(30, 8, 128, generator=g).to(DEV)
+    position = torch.tensor([25], dtype=torch.int32, device=DEV)
+    out = ops.launch_attention(q, kc, kc, position=position, scaling=0.1, out_dtype=torch.float32)
+    expected = reference_attention(q.cpu()[:15], kc.cpu(), kc.cpu(), 25, 0.1)
+    assert relative_l2(out[:15].cpu(), expected) < 1e-5
+    assert (out[15:] == 0).all()
 
 
 @pytest.mark.parametrize(
