@@ -69,12 +69,14 @@ typedef enum nq_decode_launch {
     NQ_DECODE_FUSED = 1
 } nq_decode_launch;
 
-/* Operands of the prefill path's fp16 MFMA GEMMs (tokens > 16).
- *   NQ_PREFILL_FP16: the row-scaled activations and the rank intermediate
- *     rounded to fp16 (11 bits; about 3e-4 rel-L2 against the fp32 forward).
- *   NQ_PREFILL_FP16_SPLIT: each as an fp16 high part plus an fp16 part of the
- *     remainder (about 22 bits), two MFMAs per product, for callers whose
- *     errors compound (a decoder's prompt pass).
+/* Operands of the prefill path's MFMA GEMMs (tokens > 16): the activations
+ * and the rank intermediate as sums of 6-bit planes of five bits each, with one
+ * exponent for 32 columns of a row.
+ *   NQ_PREFILL_FP16: three planes, an error of at most 2^-14 of the largest of
+ *     the 32 values (about 6e-5 rel-L2 against the fp32 forward; never more
+ *     than fp16 operands have, hence the name).
+ *   NQ_PREFILL_FP16_SPLIT: five planes (about 1e-7), for callers whose errors
+ *     compound (a decoder's prompt pass).
  * Batch members must agree. No reference counterpart (the reference's
  * kernels compute in the activation dtype, cuda_kernels.py:65-162). */
 typedef enum nq_prefill_operands {
@@ -230,7 +232,9 @@ int nq_linear(const nq_linear_desc* desc, const void* x, int32_t x_dtype,
  * file-scope device array of NQ_STATIC_SCRATCH_BYTES per GPU, held until the
  * process ends; calls whose nq_linear_workspace_bytes exceeds it return
  * NQ_ERR_SCRATCH (decode token counts fit any Qwen3/Llama-sized layer;
- * larger prefill calls need nq_linear). Allocates nothing itself. All calls
+ * larger prefill calls need nq_linear). The limit counts a prefill call's
+ * operands as 16-bit values of the call's rows; where whole groups of 32 rows
+ * make nq_linear_workspace_bytes larger than that, the array holds them too. Allocates nothing itself. All calls
  * on one GPU share the array: calls that overlap in time on one GPU race and
  * must not be issued (one stream, or streams ordered by the caller). */
 int nq_linear_static(const nq_linear_desc* desc, const void* x, int32_t x_dtype,

@@ -398,19 +398,24 @@ int validate(const nq_linear_desc* d) {
     return NQ_OK;
 }
 
-// Workspace carve-up: [lm: tokens*rank f32][patch tmp: tokens*p f32][decode scratch].
+// Workspace carve-up: [patch tmp: tokens*p f32][lm: tokens*rank f32][decode scratch],
+// the prefill path's scratch from lm on.
 struct WorkspaceLayout {
     int64_t lm_offset, patch_offset, decode_offset, total;
+    int64_t reserved;  // what nq_linear_static holds against its limit
 };
 
 WorkspaceLayout workspace_layout(const nq_linear_desc* d, int64_t tokens) {
     WorkspaceLayout w{};
-    w.lm_offset = 0;
-    w.patch_offset = align256(tokens * d->rank * 4);
-    w.decode_offset = w.patch_offset + align256(tokens * d->patch_rank * 4);
-    const int64_t tiled = nq::decode_path_applies(d, tokens) ? nq::decode_scratch_bytes(d, tokens)
-                                                             : nq::prefill_scratch_bytes(d, tokens);
-    w.total = w.decode_offset + tiled;
+    w.patch_offset = 0;
+    w.lm_offset = align256(tokens * d->patch_rank * 4);
+    w.decode_offset = w.lm_offset + align256(tokens * d->rank * 4);
+    if (nq::decode_path_applies(d, tokens)) {
+        w.total = w.reserved = w.decode_offset + nq::decode_scratch_bytes(d, tokens);
+    } else {
+        w.total = w.lm_offset + nq::prefill_scratch_bytes(d, tokens);
+        w.reserved = w.lm_offset + nq::prefill_reserved_bytes(d, tokens);
+    }
     return w;
 }
 
@@ -470,6 +475,11 @@ extern "C" int64_t nq_linear_workspace_bytes(const nq_linear_desc* desc, int64_t
     return workspace_layout(desc, tokens).total;
 }
 
+int64_t nq::linear_reserved_bytes(const nq_linear_desc* desc, int64_t tokens) {
+    if (validate(desc) != NQ_OK || tokens <= 0) return -1;
+    return workspace_layout(desc, tokens).reserved;
+}
+
 extern "C" int nq_linear(const nq_linear_desc* d, const void* x, int32_t x_dtype, int64_t tokens,
                          void* y, int32_t y_dtype, void* workspace, int64_t workspace_bytes,
                          void* stream) {
@@ -489,7 +499,7 @@ extern "C" int nq_linear(const nq_linear_desc* d, const void* x, int32_t x_dtype
         st = nq::launch_decode(d, x, x_dtype, tokens, y, y_dtype, ws + wl.decode_offset, s);
         if (st != NQ_OK) return st;
     } else if (nq::prefill_path_applies(d, tokens)) {
-        st = nq::launch_prefill(d, x, x_dtype, tokens, y, y_dtype, ws + wl.decode_offset, s);
+        st = nq::launch_prefill(d, x, x_dtype, tokens, y, y_dtype, ws + wl.lm_offset, s);
         if (st != NQ_OK) return st;
     } else {
         float* lm = reinterpret_cast<float*>(ws + wl.lm_offset);
@@ -558,7 +568,7 @@ extern "C" int nq_linear_batch(const nq_linear_desc* const* descs, int32_t count
         }
         const WorkspaceLayout wl = workspace_layout(d, tokens);
         if (!workspaces[i] || workspace_bytes[i] < wl.total) return NQ_ERR_WORKSPACE;
-        scratch[i] = static_cast<char*>(workspaces[i]) + wl.decode_offset;
+        scratch[i] = static_cast<char*>(workspaces[i]) + (decode ? wl.decode_offset : wl.lm_offset);
     }
     auto s = static_cast<hipStream_t>(stream);
     int st = decode ? nq::launch_decode_batch(descs, count, xs, x_dtype, tokens, ys, y_dtype, scratch, s)

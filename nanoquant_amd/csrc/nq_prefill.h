@@ -6,8 +6,18 @@
 
 namespace nq {
 
-// Workspace bytes the prefill path needs for `tokens` slots.
+// Workspace bytes of a call above the decode kernel's token counts, the general
+// path's fp32 rank intermediate among them (all of it without tiles).
 int64_t prefill_scratch_bytes(const nq_linear_desc* d, int64_t tokens);
+
+// The size that nq_linear_static's limit is held against (at most
+// prefill_scratch_bytes, and at least 1 / kPrefillOverReserve of it).
+int64_t prefill_reserved_bytes(const nq_linear_desc* d, int64_t tokens);
+constexpr int kPrefillOverReserve = 3;
+
+// The whole call's reserved bytes (nq_linear_workspace_bytes with
+// prefill_reserved_bytes in place of prefill_scratch_bytes), or -1.
+int64_t linear_reserved_bytes(const nq_linear_desc* d, int64_t tokens);
 
 // True when desc->tiles is set and tokens exceed the decode kernel's range.
 bool prefill_path_applies(const nq_linear_desc* d, int64_t tokens);

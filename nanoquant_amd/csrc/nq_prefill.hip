@@ -1,372 +1,264 @@
 // Prefill path (tokens > 16) for the packed binary low-rank linear on gfx950:
-// two dense sign GEMMs on v_mfma_f32_32x32x16_f16.
+// two dense sign GEMMs on v_mfma_scale_f32_32x32x64_f8f6f4 (activations as
+// fp6, signs as fp4).
 //
-//   k_prep_rows:  xs16[t, :] = fp16(x[t, :] * s_in * 2^e_t)       (exact power of
-//                 two per row from max |x * s_in|, so fp16 cannot overflow),
-//                 and 2^f_t from the bound |lm[t, r]| <= max|s_mid| * Σ_i |x s_in|
-//   GEMM 1:       lm16[t, r] = fp16(2^f_t * s_mid[r] * (xs16 · V±1ᵀ)[t, r] / 2^e_t)
-//   GEMM 2:       y[t, o]    = s_out[o] * (lm16 · U±1ᵀ)[t, o] / 2^f_t
-//                              + Σ_k x[t, idx_k] W_sal[o, k] (* scale_k) + bias[o]
+//   k_prep_rows:  planes of x * s_in                 (6-bit values, below)
+//   GEMM 1:       planes of lm[t, r] = s_mid[r] * (x s_in · V±1ᵀ)[t, r]
+//   GEMM 2:       y[t, o] = s_out[o] * (lm · U±1ᵀ)[t, o]
+//                           + Σ_k x[t, idx_k] W_sal[o, k] (* scale_k) + bias[o]
 //
-// The bound puts every lm16 value at or below 2^14, inside the fp16 range,
-// and values far below the bound keep fp16's relative precision down to
-// 2^-14 (they lie within a few binades of it for any real row), so the
-// rank intermediate never takes a pass of its own.
+// Activation operands. A group of 32 columns of a row shares a power of two
+// 2^e (its largest value lies in [2, 4) of it); a value is the sum of P fp6
+// (e2m3) numbers, each the rounding of what the ones before left over, plane p
+// in units of 2^(e - 5p). A plane takes a value below 4 to a remainder of at
+// most 1/8, which the next plane, 32 times finer, sees below 4 again, so every
+// plane adds five bits: P = 3 holds 16 bits below the group's largest value
+// (half a unit is 2^-14 of 4: 4e-5 rel-L2 on normal rows, where single fp16
+// operands have 2e-4 to 3e-4), P = 5 all 24 bits of an fp32 value of the
+// group's largest binade (split operands: NQ_PREFILL_FP16_SPLIT). The group's
+// exponent is the MFMA's A scale and the plane's 2^-5p its B scale, so no
+// pass over the row is needed for a scale of its own, the rank intermediate is
+// formed from its own values (no bound), and the sums come out unscaled. A
+// group that holds a NaN or an infinity has the NaN scale: every output of the
+// token is NaN, as the reference's fp32 forward yields (a non-finite
+// activation reaches every rank value with both signs; reference.py:208-217).
 //
-// The sign operand comes straight from the decode tile layout (16-row tiles;
-// in 128-column block kb = 4c + d a lane's word d of chunk c holds, at bit
-// 8b + m, column 128kb + 16m + 4g + b for lane group g). A 32 x 32 x 16 MFMA
-// over 16-column slice m takes, in lane 32h + r, the 8 k slots of B column r
-// (sign row r of a 32-row pair of tiles) for columns 16m + 8h + [0, 8): the
-// words of lane groups 2h and 2h + 1 of row r hold exactly those columns, so
-// each lane loads two words per tile pair and 128-column block and expands
-// them in registers (one shift and one and_or per fp16 pair). k_prep_rows
-// stores activation rows with columns 1 and 2 of every group of four swapped,
-// which puts the A operand's 8 k slots in the same order: one 16-byte LDS
-// read per A fragment. Each expanded B fragment serves two A fragments and
-// each A fragment two B fragments.
+// Why fp6 planes. The signs are exact in fp4 (+-1), the products exact, and
+// the matrix cores take fp6 x fp4 at four times the fp16 rate (register-only
+// loops on this chip: 4.1 - 6.7 PFLOP/s against 1.28 - 1.85, held down by
+// power either way), so three planes cost 3/4 of one fp16 pass and five planes
+// 5/8 of the two of split fp16 operands. Expanding signs costs one shift and
+// one and-or for eight of them instead of three instructions for four.
 //
-// Block tile 128 (tokens) x 128 (sign rows), 4 waves in a 2 x 2 grid, each
-// wave 64 x 64 = 2 x 2 MFMA tiles of 32 x 32 accumulated in fp32 (or 128 x
-// 256, waves side by side, for large GEMMs). The activation tile (128 x 128
-// fp16, 16-byte chunks XOR-swizzled by row) is double-buffered in LDS and
-// moved there by global_load_lds_dwordx4, so the next 128-column block is in
-// flight during the current block's MFMAs without holding registers; one
-// barrier per block orders the buffer swap. Within a block the eight
-// 16-column slices are software-pipelined: slice m's MFMAs issue while slice
-// m + 1's A fragments are read and its signs expanded.
+// Sign operand, straight from the decode tile layout (16-row tiles; in
+// 128-column block kb = 4c + d a lane's word d of chunk c holds, at bit 8b + m,
+// column 128kb + 16m + 4g + b for lane group g). A 32 x 32 x 64 MFMA takes, in
+// lane 32h + r, 32 k slots of B column r: exactly one word, that of lane group
+// g = 2 step + h for 64-column step `step`. Slot 8s + j is the nibble j of
+// dword s, sign bit 4j + s of the word: column 16 (4 (j & 1) + s) + 4g + (j >> 1).
+// The columns of one word are the 32-column group that shares a scale.
 //
-// Split operands (nq_linear_desc.prefill_operands = NQ_PREFILL_FP16_SPLIT):
-// every prepared row and the rank intermediate carry, per 128-column block,
-// the fp16 values hi = fp16(v) and then the fp16 remainders lo = fp16(v - hi)
-// (v - hi is exact in fp32), so a row of K columns is 2K fp16 wide. Each K
-// step then moves both 128-column planes into LDS and issues every MFMA
-// twice, hi then lo into the same accumulator: about 22 bits per operand
-// instead of 11, against twice the MFMA and activation work (the signs are
-// expanded once).
+// Activation operand in memory, in the order the MFMA and LDS want it: per
+// 128-column block kb and group of 32 rows, for each 64-column step and plane
+// the 64 lanes' first 16 bytes and then their last 8 (1536 bytes): a K step of
+// a block tile is one run of bytes, moved into LDS linearly by
+// global_load_lds_dwordx4 and read back without bank conflicts. Exponents:
+// [kb][row group][lane][step], one byte each, read from global memory.
+//
+// Block tile up to 128 (tokens) x 256 (sign rows), four waves in a 2 x 2 grid
+// of 64 x 128 (each expanded sign fragment feeds 2 x P MFMAs, each A fragment
+// four). The next 128-column step moves into the idle LDS buffer during the
+// current one's MFMAs; one barrier per step orders the swap. Within a step the
+// 2 P (64-column step, plane) phases are software-pipelined.
 //
 // Split K: when a GEMM has too few (token, sign-row) tiles to fill the GPU,
-// its K blocks are split into slices of at least two, each workgroup writes
-// its raw fp32 accumulators to partial[slice][t][n], and k_reduce_splits, one
-// thread per output element, sums them in slice order (deterministic) and
-// applies the epilogue. A batched call runs up to eight GEMMs of one phase in
-// one launch, their (column block, slice) ranges concatenated along grid x.
+// its K blocks are split into slices, each workgroup writes its raw fp32
+// accumulators to partial[slice][t][n], and a reduction sums them in slice
+// order (deterministic) and applies the epilogue. A batched call runs up to
+// eight GEMMs of one phase in one launch, their (column block, slice) ranges
+// concatenated along grid x.
+#include <utility>
+
 #include "nq_prefill.h"
 
 namespace {
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef uint32_t v6u __attribute__((ext_vector_type(6)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
 
 constexpr int kBlock = 256;
-constexpr int kBM = 128;
-constexpr int kBN = 128;
-constexpr int kBK = 128;                 // one superchunk per K step
+constexpr int kBK = 128;                 // columns per K step
 constexpr int kTileRows = 16;
+constexpr int kRows = 32;                // rows of an operand group
+constexpr int kPlaneBytes = 1536;        // 32 rows x 64 columns of 6 bits
+constexpr int kPlaneBits = 5;            // what a plane adds
 constexpr int kPrefillBatch = 8;         // members of one batched call
-// s_waitcnt vmcnt(0) expcnt(7) lgkmcnt(15): wait for this wave's vector
-// memory operations only (gfx9 encoding), as a builtin the compiler's own
-// wait tracking takes into account.
-constexpr int kWaitVmcnt0 = 0x0F70;
+constexpr int kPlanes = 3, kPlanesSplit = 5;
+constexpr int64_t kRowsPerGridZ = 65535;  // grid y's limit; rows beyond it go to grid z
+// s_waitcnt vmcnt(n) expcnt(7) lgkmcnt(15): wait until this wave has at most n
+// vector memory operations in flight (gfx9 encoding), as a builtin the
+// compiler's own wait tracking takes into account.
+constexpr int wait_vmcnt(int n) { return (n & 15) | 0x0F70 | (n >> 4) << 14; }
+constexpr int kWaitVmcnt0 = wait_vmcnt(0);
 
 __device__ __forceinline__ float exp2i(int e) { return __uint_as_float(static_cast<uint32_t>(e + 127) << 23); }
 
-__device__ __forceinline__ float range_scale(float bound) {
-    if (!(bound > 0.0f)) return 1.0f;
-    int e = static_cast<int>((__float_as_uint(bound) >> 23) & 0xff) - 127;
-    e = 13 - (e < -126 ? -126 : e);
-    e = e > 100 ? 100 : (e < -100 ? -100 : e);
-    return exp2i(e);
-}
+// An activation matrix as fp6 planes: rows in groups of 32 (row_groups of
+// them; the rows past the last token hold anything), nkb 128-column blocks.
+struct Operand {
+    uint8_t* planes;     // [nkb][row_groups][2][P][1536]
+    uint8_t* exps;       // [nkb][row_groups][64][2]
+    int64_t row_groups;
+};
 
-// Scale of a prepared row from its max |a s| and its sum of |a s|. The sum
-// is NaN or +Inf exactly when the row holds a NaN or an infinity (fmaxf
-// drops NaN, a sum does not); such a row is scaled by NaN, so every output of
-// the token is NaN, as the reference's fp32 forward yields (a non-finite
-// activation reaches every rank value with both signs; reference.py:208-217).
-__device__ __forceinline__ float prep_scale(float max_abs, float sum_abs) {
-    return sum_abs <= 3.402823466e38f ? range_scale(max_abs) : __builtin_nanf("");
-}
-
-// Position of column c in a prepared row: columns 1 and 2 of every group of
-// four are swapped (the order the sign operand's fp16 pairs come in).
-__device__ __forceinline__ int64_t swizzle4(int64_t c) { return (c & ~int64_t(3)) | ((c & 1) << 1) | ((c >> 1) & 1); }
-
-// fp32 values of elements [c, c + 8) of a row (c % 8 == 0): one 16-byte (or
-// two, for fp32) vector load when `vec` (the host checked alignment and
-// cols % 8 == 0), bounds-checked element loads otherwise.
-__device__ __forceinline__ void load8(const void* __restrict__ p, int dtype, bool vec, int64_t base, int64_t c,
-                                      int64_t cols, float (&v)[8]) {
-    if (vec) {
-        if (dtype == NQ_DTYPE_F32) {
-            const float4* q = reinterpret_cast<const float4*>(static_cast<const float*>(p) + base + c);
-            const float4 a = q[0], b = q[1];
-            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-            v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-        } else {
-            const uint4 q = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + base + c);
-            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+// Columns 4g + b + 16m of 128-column block kb of a row, a = m in [0, 4) (four
+// b each) and c = m in [4, 8), as P planes.
+template <int P>
+__device__ __forceinline__ void store_group(const Operand& op, int64_t row, int64_t kb, int g, v16f a, v16f c) {
+    uint32_t top = 0;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (dtype == NQ_DTYPE_BF16) {
-                    v[2 * i] = __uint_as_float(w[i] << 16);
-                    v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-                } else {
-                    union {
-                        uint32_t u;
-                        _Float16 h[2];
-                    } h;
-                    h.u = w[i];
-                    v[2 * i] = static_cast<float>(h.h[0]);
-                    v[2 * i + 1] = static_cast<float>(h.h[1]);
-                }
-            }
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = c + i < cols ? nq::load_f32(p, dtype, base + c + i) : 0.0f;
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t x = __float_as_uint(a[i]) & 0x7fffffffu, y = __float_as_uint(c[i]) & 0x7fffffffu;
+        top = top > x ? top : x;
+        top = top > y ? top : y;
     }
+    const bool finite = top < 0x7f800000u;
+    int e = static_cast<int>(top >> 23) - 128;  // 2^e: half the largest value's binade
+    e = e < -100 ? -100 : (finite ? e : 0);
+    const int64_t at = kb * op.row_groups + (row >> 5);
+    const int lane = 32 * (g & 1) + static_cast<int>(row & 31);
+    uint8_t* const dst = op.planes + (at * 2 + (g >> 1)) * (P * kPlaneBytes);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const float unit = exp2i(e - kPlaneBits * p);
+        v6u w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, c, unit);
+        // The conversion's operands outlive it, or the compiler lets its result
+        // overlap them, and what is written first is read again (seen in the
+        // last plane: 5.7e-6 rel-L2 with five).
+        asm volatile("" : "+v"(w) : "v"(a), "v"(c), "v"(unit));
+        *reinterpret_cast<uint4*>(dst + p * kPlaneBytes + 16 * lane) = make_uint4(w[0], w[1], w[2], w[3]);
+        *reinterpret_cast<uint2*>(dst + p * kPlaneBytes + 1024 + 8 * lane) = make_uint2(w[4], w[5]);
+        if (p + 1 < P) {
+            v32f got = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(w, unit);
+            asm volatile("" : "+v"(got) : "v"(w), "v"(unit));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) a[i] -= got[2 * i], c[i] -= got[2 * i + 1];  // exact
+        }
+    }
+    op.exps[(at * 64 + lane) * 2 + (g >> 1)] = static_cast<uint8_t>(finite ? e + 127 : 255);
 }
 
-// Row pass of one member of a batched call (grid y = member, x = token).
+// Four elements of a buffer as fp32: one load (the host checked alignment).
+template <int DT>
+__device__ __forceinline__ v4f load4_as(const void* __restrict__ p, int64_t i) {
+    if constexpr (DT == NQ_DTYPE_F32) return *reinterpret_cast<const v4f*>(static_cast<const float*>(p) + i);
+    const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p) + i);
+    v4f v;
+    if constexpr (DT == NQ_DTYPE_BF16) {
+        v[0] = __uint_as_float(w.x << 16), v[1] = __uint_as_float(w.x & 0xffff0000u);
+        v[2] = __uint_as_float(w.y << 16), v[3] = __uint_as_float(w.y & 0xffff0000u);
+    } else {
+        v[0] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w.x)));
+        v[1] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w.x >> 16)));
+        v[2] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w.y)));
+        v[3] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w.y >> 16)));
+    }
+    return v;
+}
+
+// Row pass of one member of a batched call.
 struct PrepArgs {
-    const void* act;                 // [tokens, ld] activations
-    int64_t ld;
-    const void* colscale;            // [cols] s_in, or null
-    int colscale_dtype;
-    int vec;                         // 16-byte loads allowed (generic kernel)
-    int64_t cols, cols_pad;
-    _Float16* out16;                 // [tokens, cols_pad], or [tokens, 2 cols_pad] with split
-    int split;                       // split operands: hi and lo planes per 128-column block
-    float* scale_out;                // [tokens]
-    const uint32_t* max_mid_bits;    // fp32 bits of max|s_mid|, or null
-    float* bound_scale_out;          // [tokens]
+    const void* act;                 // [tokens, cols] activations
+    const void* colscale;            // [cols] s_in
+    int act_dtype, colscale_dtype;
+    int64_t tokens, cols, nkb;
+    Operand out;
 };
 
 struct PrepBatch {
     PrepArgs p[kPrefillBatch];
 };
 
-// Stores columns [c, c + 8) (c % 8 == 0) of prepared row t, v times `scale`,
-// into a buffer of rows of cols_pad columns: fp16 with columns 1 and 2 of
-// every group of four exchanged (swizzle4), one 16-byte store; with `split`
-// the rows are 2 cols_pad wide, block c / 128 holding its 128 high parts and
-// then their remainders: two stores.
-__device__ __forceinline__ void store_prepped(_Float16* __restrict__ out, int64_t t, int64_t cols_pad, int64_t c,
-                                              const float (&v)[8], float scale, bool split) {
-    union {
-        _Float16 h[8];
-        uint4 u;
-    } hi, lo;
+// planes of act * colscale, zero past the last column. Grid: 16-row groups,
+// four 128-column blocks (one per wave), members; lane 16 g + r takes row r and
+// columns 16 m + 4 g + [0, 4). Bound by memory and launch: VEC reads four
+// elements per load (cols % 4 == 0, aligned), typed, all issued before the
+// first use; the generic form takes any type, alignment and width.
+// Written and read once, 2048 x 14336 bf16 moves 126 MB in 23.5 us (5.4 TB/s;
+// fp16 operands with a scale per row: 19.4 us for 117 MB); 61 x 4096 4.6 us.
+template <int ADT, int SDT, int P, bool VEC>
+__global__ __launch_bounds__(kBlock) void k_prep_rows(const PrepBatch batch) {
+    const PrepArgs& pa = batch.p[blockIdx.z];
+    const int lane = threadIdx.x & 63, g = lane >> 4;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * 16 + (lane & 15);
+    const int64_t kb = static_cast<int64_t>(blockIdx.y) * 4 + (threadIdx.x >> 6);
+    const int64_t cols = pa.cols;
+    if (kb >= pa.nkb || row >= pa.tokens) return;
+    const int64_t c0 = kb * kBK + 4 * g, at = row * cols + c0;
+    v16f half[2];
+    if constexpr (VEC) {
+        v4f x[8], s[8];
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float x = v[4 * g + (i == 1 ? 2 : (i == 2 ? 1 : i))] * scale;
-            hi.h[4 * g + i] = static_cast<_Float16>(x);
-            lo.h[4 * g + i] = static_cast<_Float16>(x - static_cast<float>(hi.h[4 * g + i]));
-        }
-    }
-    if (!split) {
-        *reinterpret_cast<uint4*>(out + t * cols_pad + c) = hi.u;
-        return;
-    }
-    _Float16* const row = out + t * 2 * cols_pad + (c >> 7) * 256 + (c & 127);
-    *reinterpret_cast<uint4*>(row) = hi.u;
-    *reinterpret_cast<uint4*>(row + 128) = lo.u;
-}
-
-// One workgroup per row: out16[t, swizzle4(c)] = fp16(a[t, c] * s[c] * scale_t)
-// for c < cols, zero for cols <= c < cols_pad; scale_out[t] = scale_t. Each
-// thread takes 8 consecutive columns per step (one 16-byte store of fp16).
-// With `max_mid_bits` (fp32 bits of max|s_mid|) it also writes
-// bound_scale_out[t], the power of two that puts max|s_mid| * Σ_c |a s| at
-// or below 2^14: the scale of the row's rank intermediate.
-__global__ __launch_bounds__(kBlock) void k_prep_rows(const PrepBatch batch, int act_dtype) {
-    const PrepArgs& pa = batch.p[blockIdx.y];
-    const void* __restrict__ act = pa.act;
-    const int64_t ld = pa.ld;
-    const void* __restrict__ colscale = pa.colscale;
-    const int colscale_dtype = pa.colscale_dtype;
-    const int64_t cols = pa.cols, cols_pad = pa.cols_pad;
-    const int vec = pa.vec;
-    _Float16* __restrict__ out16 = pa.out16;
-    float* __restrict__ scale_out = pa.scale_out;
-    const uint32_t* __restrict__ max_mid_bits = pa.max_mid_bits;
-    float* __restrict__ bound_scale_out = pa.bound_scale_out;
-    __shared__ float wmax[kBlock / 64];
-    __shared__ float wsum[kBlock / 64];
-    const int64_t t = blockIdx.x;
-    auto values = [&](int64_t c, float (&v)[8]) {
-        load8(act, act_dtype, vec != 0, t * ld, c, cols, v);
-        if (colscale) {
-            float s8[8];
-            load8(colscale, colscale_dtype, vec != 0, 0, c, cols, s8);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] *= s8[i];
+        for (int m = 0; m < 8; ++m) {
+            const int64_t back = c0 + 16 * m < cols ? 16 * m : -c0;  // past the row: its first columns, dropped below
+            x[m] = load4_as<ADT>(pa.act, at + back);
+            s[m] = load4_as<SDT>(pa.colscale, c0 + back);
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = c + i < cols ? v[i] : 0.0f;
-    };
-    float m = 0.0f, l1 = 0.0f;
-    for (int64_t c = 8 * threadIdx.x; c < cols; c += 8 * kBlock) {
-        float v[8];
-        values(c, v);
+        for (int m = 0; m < 8; ++m)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v[i])), l1 += fabsf(v[i]);
-    }
-    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off)), l1 += __shfl_xor(l1, off);
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m, wsum[threadIdx.x >> 6] = l1;
-    __syncthreads();
-    const float l1t = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
-    const float scale = prep_scale(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])), l1t);
-    if (max_mid_bits && threadIdx.x == 0) bound_scale_out[t] = range_scale(__uint_as_float(*max_mid_bits) * l1t);
-    for (int64_t c = 8 * threadIdx.x; c < cols_pad; c += 8 * kBlock) {
-        float v[8];
-        if (c < cols) values(c, v);
-        else
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = 0.0f;
-        store_prepped(out16, t, cols_pad, c, v, scale, pa.split != 0);
-    }
-    if (threadIdx.x == 0) scale_out[t] = scale;
-}
-
-// Elements [i, i + 8) of a buffer of dtype DT as fp32: one 16-byte load
-// (two for fp32), no branch.
-template <int DT>
-__device__ __forceinline__ void load8_as(const void* __restrict__ p, int64_t i, float (&v)[8]) {
-    if constexpr (DT == NQ_DTYPE_F32) {
-        const float4* q = reinterpret_cast<const float4*>(static_cast<const float*>(p) + i);
-        const float4 a = q[0], b = q[1];
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+            for (int b = 0; b < 4; ++b) half[m >> 2][4 * (m & 3) + b] = c0 + 16 * m < cols ? x[m][b] * s[m][b] : 0.0f;
     } else {
-        const uint4 q = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + i);
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if constexpr (DT == NQ_DTYPE_BF16) {
-                v[2 * j] = __uint_as_float(w[j] << 16);
-                v[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-            } else {
-                v[2 * j] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w[j])));
-                v[2 * j + 1] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w[j] >> 16)));
+        for (int m = 0; m < 8; ++m)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int64_t c = 16 * m + b;
+                half[m >> 2][4 * (m & 3) + b] = c0 + c < cols
+                                                    ? nq::load_f32(pa.act, pa.act_dtype, at + c) *
+                                                          nq::load_f32(pa.colscale, pa.colscale_dtype, c0 + c)
+                                                    : 0.0f;
             }
-        }
     }
+    store_group<P>(pa.out, row, kb, g, half[0], half[1]);
 }
 
-// k_prep_rows for rows of at most NCH * 8 * kBlock padded columns whose
-// activations and column scales allow 16-byte loads (cols % 8 == 0, aligned):
-// each thread keeps its NCH chunks of eight columns in registers, so the row
-// is read once, and every load is issued before the first use. Same
-// arithmetic and summation order as k_prep_rows, so both give identical
-// results. NCH = 2 (rows up to 4096 columns) keeps the registers low enough
-// for eight workgroups per CU.
-constexpr int kPrepChunksMax = 8;
-
-template <int ADT, int SDT, int NCH>
-__global__ __launch_bounds__(kBlock) void k_prep_rows_vec(const PrepBatch batch) {
-    const PrepArgs& pa = batch.p[blockIdx.y];
-    const void* __restrict__ act = pa.act;
-    const int64_t ld = pa.ld;
-    const void* __restrict__ colscale = pa.colscale;
-    const int64_t cols = pa.cols, cols_pad = pa.cols_pad;
-    _Float16* __restrict__ out16 = pa.out16;
-    float* __restrict__ scale_out = pa.scale_out;
-    const uint32_t* __restrict__ max_mid_bits = pa.max_mid_bits;
-    float* __restrict__ bound_scale_out = pa.bound_scale_out;
-    __shared__ float wmax[kBlock / 64];
-    __shared__ float wsum[kBlock / 64];
-    const int64_t t = blockIdx.x;
-    float v[NCH][8];
-#pragma unroll
-    for (int k = 0; k < NCH; ++k) {
-        const int64_t c = 8 * threadIdx.x + 8 * kBlock * k;
-        const int64_t cc = c < cols ? c : 0;  // chunks past the row reload its first
-        float s8[8];
-        load8_as<ADT>(act, t * ld + cc, v[k]);
-        load8_as<SDT>(colscale, cc, s8);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[k][i] *= s8[i];
-    }
-    float m = 0.0f, l1 = 0.0f;
-#pragma unroll
-    for (int k = 0; k < NCH; ++k) {
-        const bool live = 8 * threadIdx.x + 8 * kBlock * k < cols;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            v[k][i] = live ? v[k][i] : 0.0f;
-            if (live) m = fmaxf(m, fabsf(v[k][i])), l1 += fabsf(v[k][i]);
-        }
-    }
-    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off)), l1 += __shfl_xor(l1, off);
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m, wsum[threadIdx.x >> 6] = l1;
-    __syncthreads();
-    const float l1t = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
-    const float scale = prep_scale(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])), l1t);
-    if (max_mid_bits && threadIdx.x == 0) bound_scale_out[t] = range_scale(__uint_as_float(*max_mid_bits) * l1t);
-#pragma unroll
-    for (int k = 0; k < NCH; ++k) {
-        const int64_t c = 8 * threadIdx.x + 8 * kBlock * k;
-        if (c >= cols_pad) continue;
-        store_prepped(out16, t, cols_pad, c, v[k], scale, pa.split != 0);
-    }
-    if (threadIdx.x == 0) scale_out[t] = scale;
+// Signs of one word as the B operand (32 fp4 values of +-1): nibble j of dword
+// s takes sign bit 4j + s.
+__device__ __forceinline__ v8i expand_signs(uint32_t w, uint32_t mask, uint32_t one) {
+    // The masks come in registers: a VOP3 instruction cannot take two literals.
+    v8i b = {};
+    b[0] = static_cast<int>(((w << 3) & mask) | one);
+    b[1] = static_cast<int>(((w << 2) & mask) | one);
+    b[2] = static_cast<int>(((w << 1) & mask) | one);
+    b[3] = static_cast<int>((w & mask) | one);
+    return b;
 }
 
-// B operand of the 32 x 32 x 16 MFMA of 16-column slice m from the words of
-// lane groups 2h and 2h + 1 (w0, w1): at bit 8b + m they hold columns
-// 16m + 8h + b and 16m + 8h + 4 + b. The A rows are stored with columns 1 and
-// 2 of every group of four swapped, so the eight k slots of a lane are columns
-// 8h + {0, 2, 1, 3, 4, 6, 5, 7}: dword e pairs bits (m, m + 16) or
-// (m + 8, m + 24) of one word, which one shift moves to the fp16 sign
-// positions 15 and 31.
-__device__ __forceinline__ uint32_t sign_pair(uint32_t w, int shift, uint32_t mask, uint32_t one) {
-    // ((w << shift) & mask) | one as two instructions: the masks are kept in
-    // registers because a VOP3 instruction cannot take two literal constants.
-    return ((w << shift) & mask) | one;
+// One plane's product of a 64-column step: A fp6 (format 2) with its row
+// groups' exponents (byte STEP of `ea`), B fp4 (format 4) with the plane's.
+template <int STEP, int PL>
+__device__ __forceinline__ v16f mfma_plane(const v8i& a, const v8i& b, const v16f& c, int ea, int eb, int eb4) {
+    if constexpr (PL < 4) return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 4, STEP, ea, PL, eb);
+    else return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 4, STEP, ea, 0, eb4);
 }
 
-// 64-bit left shift as one instruction (a shift by a constant is otherwise
-// split into a 32-bit shift and an alignbit); the amount comes from an SGPR.
-__device__ __forceinline__ uint64_t shl64(uint64_t w, int s) {
-    uint64_t r;
-    asm("v_lshlrev_b64 %0, %1, %2" : "=v"(r) : "s"(s), "v"(w));
-    return r;
+// A wave-uniform value, in scalar registers.
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    return static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32))) << 32 |
+           static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
 }
 
-// The two words take the same shifts, so each shift moves both as one 64-bit
-// value (w1:w0): a shift s <= 15 carries bits of w0 only into bits below s of
-// the high half, never into its sign positions 15 and 31.
-__device__ __forceinline__ v8h expand_signs32(uint32_t w0, uint32_t w1, int m, uint32_t mask, uint32_t one) {
-    union {
-        uint32_t u[4];
-        v8h v;
-    } x;
-    const uint64_t w = (static_cast<uint64_t>(w1) << 32) | w0;
-    const uint64_t hi = shl64(w, 15 - m), lo = shl64(w, 7 - m);
-    x.u[0] = (static_cast<uint32_t>(hi) & mask) | one;
-    x.u[1] = (static_cast<uint32_t>(lo) & mask) | one;
-    x.u[2] = (static_cast<uint32_t>(hi >> 32) & mask) | one;
-    x.u[3] = (static_cast<uint32_t>(lo >> 32) & mask) | one;
-    return x.v;
+template <typename F, int... I>
+__device__ __forceinline__ void each(std::integer_sequence<int, I...>, const F& f) {
+    (f(std::integral_constant<int, I>{}), ...);
 }
+
+// The LDS byte address of a shared pointer, for M0.
+__device__ __forceinline__ uint32_t lds_address(char* p) {
+    typedef __attribute__((address_space(3))) char lds_char_t;
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_char_t*)p));
+}
+
+template <int W>
+struct __attribute__((packed, aligned(4))) WordRun {
+    uint32_t w[W];
+};
 
 struct GemmArgs {
-    const _Float16* a;        // [M, kpad] fp16 activations (row-scaled); [M, 2 kpad] with split
+    Operand a;                // [m] rows of nb 128-column blocks
     int64_t m;                // tokens
-    int64_t kpad;             // nb * 128
     const uint32_t* tiles;    // sign tiles [rt][nb * 64] (chunked, see above)
     int64_t n;                // sign rows (rank or out)
     int64_t nb;               // 128-column blocks
-    const float* row_scale;   // [M]: divide accumulators by this
     const void* col_scale;    // [n] s_mid or s_out
     int col_scale_dtype;
-    // epilogue (GEMM 2 only; salient_count == 0 and bias == null for GEMM 1)
+    // GEMM 1: the rank intermediate's operand (planes set); GEMM 2: y and what joins it
+    Operand mid;
+    int64_t mid_blocks;       // 128-column blocks of `mid`
     const void* x;
     int x_dtype;
     int64_t in;
@@ -378,23 +270,21 @@ struct GemmArgs {
     int scale_dtype;
     const void* bias;
     int bias_dtype;
-    void* out;                // [M, n], or fp16 [M, out_ld] with out_scale
+    void* out;                // [M, n]
     int out_dtype;
-    const float* out_scale;   // [M] or null: write fp16(v * out_scale[t]) at column
-                              // swizzle4(c) of an out_ld-wide row, zero for n <= c < out_ld
-                              // (split: rows 2 out_ld wide, the prepared-row layout)
-    int64_t out_ld;
-    int split;                // split operands (A, and the rank intermediate written)
     int64_t k_per_split;      // K blocks per K slice
     int64_t splits;           // K slices (1: no split)
     int64_t col_blocks;       // column blocks at the launch's block width
-    float* partial;           // [splits][M][n] raw accumulators, or null (direct epilogue)
+    float* partial;           // [splits][M][part_ld(n)] raw accumulators, or null (direct epilogue)
 };
+
+// Floats per row of the partials: rows begin at multiples of 16 bytes.
+__host__ __device__ constexpr int64_t part_ld(int64_t n) { return (n + 3) & ~int64_t(3); }
 
 // Up to kPrefillBatch GEMMs of one phase (the members of a batched call share
 // the token count) in one launch. Grid x concatenates the members' ranges:
 // member i owns [begin[i], begin[i + 1]) (k_sign_gemm: col_blocks * splits
-// workgroups, slice-major; k_reduce_splits: its column blocks, none for a
+// workgroups, slice-major; the reductions: their column blocks, none for a
 // member without a split); begin[i] = INT32_MAX past the last member.
 struct GemmBatch {
     int32_t begin[kPrefillBatch];
@@ -411,24 +301,38 @@ __device__ __forceinline__ int batch_member(const GemmBatch& b, int x) {
 }
 
 // Block shapes, as (WR wave rows, II 32-row A fragments and JJ 32-column B
-// fragments per wave): (2, 2, 2): the four waves form a 2 x 2 grid of 64 x 64
-// tiles (block tile 128 x 128). (1, 4, 2): they sit side by side, each
-// 128 x 64 (block tile 128 x 256): every expanded sign fragment then serves
-// four A fragments instead of two, for GEMMs with enough blocks to fill the
-// GPU at that size. (1, 2, 1): side by side, each 64 x 32 (block tile
-// 64 x 128), for at most 64 tokens: no MFMA or A read is spent on rows past
-// the last token.
-template <int WR, int II, int JJ, bool SPLIT>
-__global__ __launch_bounds__(kBlock, JJ == 1 ? 4 : 2) void k_sign_gemm(const GemmBatch batch) {
-    constexpr int BM = WR * 32 * II;      // token rows per block
-    constexpr int BN = (4 / WR) * 32 * JJ;  // sign rows per block
-    constexpr int NJ = BM / 16;           // 1-KB LDS transfers per wave per K step and plane
-    constexpr int kABytes = BM * kBK * 2;   // one activation plane, rows of 256 bytes
-    constexpr int kPlanes = SPLIT ? 2 : 1;  // split operands: the hi plane, then the lo plane
-    constexpr int kBufBytes = kPlanes * kABytes;
-    constexpr int kParkStride = 32 * JJ + 1;  // floats per parked accumulator row
-    constexpr int kParkBytes = 4 * 64 * kParkStride * 4;
-    constexpr int kLds = 2 * kBufBytes > kParkBytes ? 2 * kBufBytes : kParkBytes;  // double-buffered A
+// fragments per wave): WR = 2: the four waves form a 2 x 2 grid; WR = 1: they
+// sit side by side. P planes.
+template <int WR, int II, int JJ, int P>
+__global__ __launch_bounds__(kBlock, 2) void k_sign_gemm(const GemmBatch batch) {
+    constexpr int RG = WR * II;                  // row groups per block
+    constexpr int BM = kRows * RG;               // token rows per block
+    constexpr int BN = (4 / WR) * 32 * JJ;       // sign rows per block
+    constexpr int kGroupBytes = 2 * P * kPlaneBytes;  // a row group's K step
+    // In LDS a group is 64 bytes longer: the compiler would pair two groups'
+    // 8-byte reads (their distance a multiple of 512), which puts them in
+    // registers the MFMA cannot take and costs four moves a phase.
+    constexpr int kGroupLds = kGroupBytes + 64;
+    constexpr int kStepBytes = RG * kGroupLds;
+    constexpr int NI = RG * kGroupBytes / 1024;  // LDS transfers per K step (64 lanes x 16 bytes)
+    constexpr int NL = (NI + 3) / 4;             // and per wave
+    constexpr int kParkStride = BN + 16;         // floats per parked row (GEMM 1's epilogue)
+    constexpr int kParkBytes = WR * kRows * kParkStride * 4;
+    // Blocks of 32 and 64 rows (JJ = 1) have little work per step, so they keep
+    // NB - 1 steps in flight and move sign words and exponents through LDS
+    // too: a load the compiler tracks would be waited for together with every
+    // transfer issued before it.
+    constexpr bool kRing = JJ == 1;
+    constexpr int NB = !kRing ? 2 : (RG == 1 ? 4 : (P == kPlanes ? 3 : 2));
+    constexpr int kExpBytes = kRing ? 256 : 0;
+    constexpr int kWordBytes = kRing ? BN / kTileRows * 1024 : 0;  // a four-block chunk of the block's tiles
+    constexpr int kRingBytes = NB * (kStepBytes + kExpBytes) + 2 * kWordBytes;
+    constexpr int kLds = kRingBytes > kParkBytes ? kRingBytes : kParkBytes;
+    static_assert(!kRing || RG <= 2, "one transfer moves the exponents");
+    constexpr int kSalient = 8;                  // salient columns staged at a time
+    constexpr int W = JJ == 4 ? 2 : 4;           // blocks whose sign words one load moves
+    constexpr bool kSignsAhead = JJ < 4;         // both by the registers JJ = 4 leaves
+    static_assert(BN % 128 == 0 && kSalient * BM * 4 <= kLds, "epilogue tiles");
     const int member = batch_member(batch, static_cast<int>(blockIdx.x));
     const GemmArgs& g = batch.p[member];
     const int local = static_cast<int>(blockIdx.x) - batch.begin[member];
@@ -440,304 +344,416 @@ __global__ __launch_bounds__(kBlock, JJ == 1 ? 4 : 2) void k_sign_gemm(const Gem
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int wm = WR == 2 ? wave >> 1 : 0;  // wave row
     const int wn = WR == 2 ? wave & 1 : wave;  // wave column
-    const int h = lane >> 5;   // K half of the 32 x 32 x 16 operands
+    const int h = lane >> 5;   // K half of the operands
     const int r = lane & 31;   // A row / B column within a 32-wide fragment
-    const int64_t m0 = static_cast<int64_t>(blockIdx.y) * BM;
+    const int64_t row_block = static_cast<int64_t>(blockIdx.z) * kRowsPerGridZ + blockIdx.y;
+    const int64_t m0 = row_block * BM;
+    if (m0 >= g.m) return;  // uniform
     const int64_t n0 = static_cast<int64_t>(col_block) * BN;
     const int64_t rt_count = (g.n + kTileRows - 1) / kTileRows;
-    // B fragment jj covers sign rows n0 + 32 JJ wn + 32 jj + [0, 32): lane r
-    // reads row r of tile (r >> 4) of that pair, from the words of lane groups
-    // 2h and 2h + 1, which hold columns 16m + 8h + [0, 8) of each 16-column slice.
-    const int64_t rt0 = n0 / kTileRows + 2 * JJ * wn + (r >> 4);
-    const int wl0 = 16 * (2 * h) + (r & 15), wl1 = wl0 + 16;
 
-    v16f acc[II][JJ];
+    // The matrix core truncates what it adds to an accumulator. Two planes of
+    // five bits sum up exactly or nearly so within an accumulator's 24 bits, so
+    // with split operands planes 2 to 4 take one of their own (one for all
+    // five: 1.0e-7 to 3.0e-7 rel-L2 against 7.5e-8 to 9.1e-8).
+    constexpr int NA = P > 3 ? 2 : 1;
+    v16f sums[NA][II][JJ];
 #pragma unroll
-    for (int i = 0; i < II; ++i)
+    for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int j = 0; j < JJ; ++j) acc[i][j] = v16f{};
+        for (int i = 0; i < II; ++i)
+#pragma unroll
+            for (int j = 0; j < JJ; ++j) sums[a][i][j] = v16f{};
+    v16f (&acc)[II][JJ] = sums[0];
 
-    uint32_t words[JJ][2], next_words[JJ][2];
-    // Activation tile: BM rows of 128 fp16 (256 bytes) per buffer, moved
-    // from global memory straight into LDS (global_load_lds_dwordx4: lane l
-    // of an instruction writes 16 bytes at the wave's LDS address + 16 l), so
-    // the next K step's tile costs no registers while it is in flight. Wave w's
-    // instruction j fills LDS rows 4 (NJ w + j) + [0, 4); lane l writes chunk
-    // position p = l & 15 of row r, which holds the row's 16-byte column chunk
-    // p ^ (r & 15): the A-fragment reads (32 rows at one chunk per
-    // instruction) then fall on distinct banks. Every load is unconditional
-    // (no branch in the K loop): rows past M read the last valid row and sign
-    // tiles past N a valid tile; they only feed accumulators whose outputs are
-    // never stored.
-    const int64_t nsc = g.nb, lda = kPlanes * g.kpad;  // fp16 per activation row
-    const int64_t a_rows = g.m - m0;  // valid rows of this block (>= 1)
-    // Byte offsets from the block's first row (below 2^31: at most 128 rows
-    // of a padded K that the host limits), added to a wave-uniform base.
-    const char* const a_blk = reinterpret_cast<const char*>(g.a + m0 * lda);
-    uint32_t a_src[NJ];
+    // Activation steps: transfer i of a step fills LDS bytes [1024 i, + 1024).
+    // Row groups past the last one read the last (their rows are not stored).
+    // What the K loop uses of the arguments is taken once: loads from the
+    // argument segment would be repeated (and waited for) in every step.
+    const int nsc = static_cast<int>(g.nb);
+    const int64_t groups = g.a.row_groups, rg0 = row_block * RG;
+    const int rg_max = static_cast<int>(groups - rg0 < RG ? groups - rg0 : RG) - 1;
+    const int k_begin = slice * static_cast<int>(g.k_per_split);
+    const int k_end = k_begin + static_cast<int>(g.k_per_split) < nsc ? k_begin + static_cast<int>(g.k_per_split) : nsc;
+    const uint64_t plane_stride = groups * kGroupBytes, exp_stride = groups * 128;  // from block to block
+    uint64_t plane_at = uniform64(reinterpret_cast<uint64_t>(g.a.planes) + (k_begin * groups + rg0) * kGroupBytes);
+    uint64_t exp_at = uniform64(reinterpret_cast<uint64_t>(g.a.exps) + (k_begin * groups + rg0) * 128);
+    uint32_t a_src[NL];  // from the step's first row group (below 2^31: at most four groups)
+    uint32_t a_dst[NL];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int row = 4 * (NJ * wave + j) + (lane >> 4);
-        const int chunk = (lane & 15) ^ (row & 15);
-        const int64_t rr = row < a_rows ? row : a_rows - 1;
-        a_src[j] = static_cast<uint32_t>((rr * lda + 8 * chunk) * 2);
+    for (int j = 0; j < NL; ++j) {
+        // A wave without a transfer of its own repeats the last one.
+        const int i = 4 * j + wave < NI ? 4 * j + wave : NI - 1, rg = i / (kGroupBytes / 1024);
+        a_src[j] = (rg < rg_max ? rg : rg_max) * kGroupBytes + (i % (kGroupBytes / 1024)) * 1024 + 16 * lane;
+        a_dst[j] = __builtin_amdgcn_readfirstlane(lds_address(lds) + rg * 64 + i * 1024);
     }
+    // The transfer is issued as inline asm with its LDS address in M0: the
+    // compiler then does not track it, so the fragment reads of the current
+    // buffer wait only on themselves instead of on the tile in flight.
+    // Completion is this kernel's own business: a transfer only targets a
+    // buffer no wave reads in that step, and every step ends with a wait and a
+    // barrier before the next buffer is read. Steps are moved in order;
+    // `more`: there is another one (past the last, its tile is moved again).
+    const auto load_a = [&](int buf, bool more) __attribute__((always_inline)) {
+        const uint64_t base = plane_at;
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            // s_nop: one wait state between the M0 write and the LDS transfer.
+            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(a_src[j]), "s"(base),
+                         "{m0}"(a_dst[j] + buf * kStepBytes)
+                         : "memory");
+        }
+        plane_at = uniform64(more ? base + plane_stride : base);
+    };
+    // Ring form: exponents of a step (lane i: bytes 4 i of the two row groups'
+    // 256) and the sign words of a chunk (1 KB a tile: 64 lanes x 4 blocks;
+    // lanes past a narrow last chunk read its first bytes again).
+    const uint32_t exp_lds = lds_address(lds) + NB * kStepBytes, word_lds = exp_lds + NB * kExpBytes;
+    const uint32_t exp_src = ((lane >> 5) < rg_max ? (lane >> 5) : rg_max) * 128 + 4 * (lane & 31);
+    const auto load_exps_ring = [&](int buf, bool more) __attribute__((always_inline)) {
+        const uint64_t base = exp_at;
+        if (wave == 0)
+            asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(exp_src), "s"(base),
+                         "{m0}"(exp_lds + buf * kExpBytes)
+                         : "memory");
+        exp_at = uniform64(more ? base + exp_stride : base);
+    };
+    constexpr int NT = kRing ? BN / kTileRows / 4 : 1;  // sign tiles a wave moves
+    uint64_t word_at[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int64_t rt = n0 / kTileRows + 4 * j + wave;
+        word_at[j] = uniform64(reinterpret_cast<uint64_t>(g.tiles + (rt < rt_count ? rt : rt_count - 1) * nsc * 64));
+    }
+    const auto load_words_ring = [&](int chunk) __attribute__((always_inline)) {
+        const int rem = nsc - 4 * chunk;
+        const uint32_t src = 1024 * chunk + (rem >= 4 || lane < 16 * rem ? 16 * lane : 0);
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(src), "s"(word_at[j]),
+                         "{m0}"(word_lds + (chunk & 1) * kWordBytes + (4 * j + wave) * 1024)
+                         : "memory");
+    };
+    // B fragment jj covers sign rows n0 + 32 JJ wn + 32 jj + [0, 32): lane r
+    // reads row r & 15 of tile r >> 4 of that pair, the words of lane groups h
+    // and 2 + h. Tiles past the last one read it (their columns are not stored).
+    const int64_t rt0 = n0 / kTileRows + 2 * JJ * wn + (r >> 4);
+    const int wl0 = 16 * h + (r & 15), wl1 = wl0 + 32;
     const uint32_t* bt[JJ];
 #pragma unroll
     for (int jj = 0; jj < JJ; ++jj) {
         const int64_t rt = rt0 + 2 * jj < rt_count ? rt0 + 2 * jj : rt_count - 1;
         bt[jj] = g.tiles + rt * nsc * 64;
     }
-    const int64_t k_begin = static_cast<int64_t>(slice) * g.k_per_split;
-    const int64_t k_end = k_begin + g.k_per_split < nsc ? k_begin + g.k_per_split : nsc;
-    // The transfer is issued as inline asm with its LDS address in M0: the
-    // compiler then does not track it, so the A-fragment reads of the current
-    // buffer wait only on themselves (lgkmcnt(4)) instead of lgkmcnt(0) while
-    // the next tile is in flight. Completion is this kernel's own business: a
-    // transfer only targets the buffer no wave reads in that step, and every
-    // step ends with vmcnt(0) and a barrier before that buffer is read.
-    typedef __attribute__((address_space(3))) void lds_void_t;
-    const auto load_a = [&](int64_t sc, int buf) __attribute__((always_inline)) {
-        // wave-uniform: a scalar base, per-lane 32-bit offsets; plane q of
-        // block sc starts 256 q bytes after the hi plane.
-        const char* base = a_blk + sc * (2 * kBK * kPlanes);
+    uint32_t et[II];
 #pragma unroll
-        for (int q = 0; q < kPlanes; ++q)
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                lds_void_t* dst = (lds_void_t*)(lds + buf * kBufBytes + q * kABytes + (NJ * wave + j) * 1024);
-                const uint32_t lds_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst));
-                // s_nop: one wait state between the M0 write and the LDS transfer.
-                asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(a_src[j]), "s"(base + 2 * kBK * q),
-                             "{m0}"(lds_addr)
-                             : "memory");
-            }
-    };
-    const auto load_words = [&](int64_t sc) __attribute__((always_inline)) {
-        const int64_t c_ = sc >> 2;
-        const int64_t rem_ = nsc - 4 * c_;
-        const int dw_ = static_cast<int>(rem_ < 4 ? rem_ : 4);
-        const int64_t off_ = c_ * 256 + (sc & 3);
+    for (int ii = 0; ii < II; ++ii) {
+        const int rg = II * wm + ii < rg_max ? II * wm + ii : rg_max;
+        et[ii] = rg * 128 + 2 * lane;
+    }
+    // A lane's words of W consecutive blocks of a chunk lie side by side: one
+    // load moves them (a dword load costs the texture path as much as a
+    // 16-byte one here, lanes lying 16 bytes apart). Slices begin at multiples
+    // of W; a load may run past a narrow last chunk (not used; the buffer has a
+    // 256-byte tail).
+    uint32_t words[JJ][2][W], next_words[JJ][2][W];
+    int ea[II], next_ea[II];
+    const auto load_words = [&](int sc) __attribute__((always_inline)) {
+        const int rem_ = nsc - (sc & ~3);
+        const int dw_ = rem_ < 4 ? rem_ : 4;
+        const int64_t off_ = static_cast<int64_t>(sc >> 2) * 256 + (sc & 3);
 #pragma unroll
         for (int jj = 0; jj < JJ; ++jj) {
-            next_words[jj][0] = bt[jj][off_ + wl0 * dw_];
-            next_words[jj][1] = bt[jj][off_ + wl1 * dw_];
+            const WordRun<W> a = *reinterpret_cast<const WordRun<W>*>(bt[jj] + off_ + wl0 * dw_);
+            const WordRun<W> b = *reinterpret_cast<const WordRun<W>*>(bt[jj] + off_ + wl1 * dw_);
+#pragma unroll
+            for (int i = 0; i < W; ++i) next_words[jj][0][i] = a.w[i], next_words[jj][1][i] = b.w[i];
         }
     };
-    // Byte offset, within a buffer, of the A fragment of 16-column slice m
-    // for fragment row 0 (fragment ii adds 32 rows = 8192 bytes).
-    int a_off[8];
+    const auto load_exps = [&](bool more) __attribute__((always_inline)) {
+        const uint8_t* const base = reinterpret_cast<const uint8_t*>(exp_at);
 #pragma unroll
-    for (int m = 0; m < 8; ++m) a_off[m] = (32 * II * wm + r) * 256 + 16 * ((2 * m + h) ^ (r & 15));
-    // Step s computes on buffer s & 1 while the tile of step s + 1 moves into
-    // the other; a wait for this wave's transfers and one barrier per step
-    // make every wave's part of the next tile visible before it is read.
-    load_a(k_begin, 0);
-    load_words(k_begin);
-    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-    __syncthreads();
-#pragma unroll
-    for (int jj = 0; jj < JJ; ++jj) words[jj][0] = next_words[jj][0], words[jj][1] = next_words[jj][1];
-    int buf = 0;
-    uint32_t sign_mask = 0x80008000u, fp16_one = 0x3C003C00u;
-    asm volatile("" : "+v"(sign_mask), "+v"(fp16_one));  // keep them in VGPRs
-    for (int64_t sc = k_begin; sc < k_end; ++sc) {
-        const int64_t nxt = sc + 1 < k_end ? sc + 1 : sc;  // the last step reloads its tile into the idle buffer
-        load_a(nxt, buf ^ 1);
-        load_words(nxt);
-        // The sign words of the next step are issued here, ahead of the
-        // MFMAs; left to itself the scheduler sinks them to the step's end,
-        // where the wait before the barrier would take their whole latency.
-        __builtin_amdgcn_sched_barrier(0);
-        const char* a_lds = lds + buf * kBufBytes;
-        // Software pipeline over the eight 16-column slices: slice m's MFMAs
-        // issue while slice m + 1's A fragments are read from LDS and its
-        // sign fragments expanded, so no MFMA waits on a read issued just
-        // before it. Each slice is one scheduling region (sched_barrier) laid
-        // out as the reads, then MFMAs alternating with the expansion. With
-        // split operands fragment II + ii is the lo plane of fragment ii.
-        constexpr int NA = kPlanes * II;
-        v8h a_cur[NA], b_cur[JJ];
-#pragma unroll
-        for (int ai = 0; ai < NA; ++ai)
-            a_cur[ai] = *reinterpret_cast<const v8h*>(a_lds + (ai / II) * kABytes + a_off[0] + 8192 * (ai % II));
-#pragma unroll
-        for (int jj = 0; jj < JJ; ++jj) b_cur[jj] = expand_signs32(words[jj][0], words[jj][1], 0, sign_mask, fp16_one);
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            __builtin_amdgcn_sched_barrier(0);
-            v8h a_nxt[NA], b_nxt[JJ];
-            if (m < 7) {
-#pragma unroll
-                for (int ai = 0; ai < NA; ++ai)
-                    a_nxt[ai] = *reinterpret_cast<const v8h*>(a_lds + (ai / II) * kABytes + a_off[m + 1] +
-                                                              8192 * (ai % II));
-#pragma unroll
-                for (int jj = 0; jj < JJ; ++jj)
-                    b_nxt[jj] = expand_signs32(words[jj][0], words[jj][1], m + 1, sign_mask, fp16_one);
-            }
-#pragma unroll
-            for (int ai = 0; ai < NA; ++ai)
-#pragma unroll
-                for (int jj = 0; jj < JJ; ++jj)
-                    acc[ai % II][jj] =
-                        __builtin_amdgcn_mfma_f32_32x32x16_f16(a_cur[ai], b_cur[jj], acc[ai % II][jj], 0, 0, 0);
-            if (m < 7) {
-                __builtin_amdgcn_sched_group_barrier(0x100, NA, 0);  // LDS reads of slice m + 1
-#pragma unroll
-                for (int q = 0; q < NA * JJ; ++q) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);       // MFMA of slice m
-                    __builtin_amdgcn_sched_group_barrier(0x002, 8 / NA, 0);  // expansion of m + 1
-                }
-#pragma unroll
-                for (int ai = 0; ai < NA; ++ai) a_cur[ai] = a_nxt[ai];
-#pragma unroll
-                for (int jj = 0; jj < JJ; ++jj) b_cur[jj] = b_nxt[jj];
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int jj = 0; jj < JJ; ++jj) words[jj][0] = next_words[jj][0], words[jj][1] = next_words[jj][1];
-        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-        __syncthreads();
-        buf ^= 1;
-    }
-
-
-    // Epilogue through LDS: each wave parks its 64 x 64 fp32 tile (lane holds
-    // D[8 (q / 4) + 4 (lane / 32) + q % 4][lane % 32] of each 32 x 32 MFMA
-    // tile), then walks it row by row with lane = column, so every output row
-    // segment is one coalesced 64-wide store and the salient sum joins before
-    // the single rounding to the output dtype.
-    float* park = reinterpret_cast<float*>(lds) + wave * (64 * kParkStride);
-    // One 64-row half of the wave's tile (rows row0 + [0, 64)); `return`
-    // leaves only this lambda.
-    const auto emit = [&](const int64_t row0) __attribute__((always_inline)) {
-        const int64_t col = n0 + 32 * JJ * wn + lane;
-        const bool lane_ok = lane < 32 * JJ;  // lanes past the wave's columns store nothing
-        const int p_lane = lane_ok ? lane : 0;  // and read a parked column of their own row
-        const int rows = __builtin_amdgcn_readfirstlane(static_cast<int>(g.m - row0 < 64 ? g.m - row0 : 64));
-        if (rows <= 0) return;  // the whole wave is past the last token
-        const bool col_ok = lane_ok && col < g.n;
-        if (g.partial) {
-            if (!col_ok) return;
-            float* dst = g.partial + static_cast<int64_t>(slice) * g.m * g.n;
-            for (int e = 0; e < rows; ++e) dst[(row0 + e) * g.n + col] = park[e * kParkStride + p_lane];
-            return;
-        }
-        // Every lane stays active up to the stores: lane e holds values of row
-        // row0 + e that other lanes read with readlane. 1 / row_scale is exact
-        // (row_scale is a normal power of two; exponent field 254 - E), so the
-        // row loop multiplies by it and waits on no memory.
-        const int64_t col_c = col_ok ? col : g.n - 1;
-        const int lane_row = lane < rows ? lane : rows - 1;
-        const float inv_lane =
-            __uint_as_float((254u << 23) - (__float_as_uint(g.row_scale[row0 + lane_row]) & 0x7f800000u));
-        const float cs = nq::load_f32(g.col_scale, g.col_scale_dtype, col_c);
-        const float bias = g.bias ? nq::load_f32(g.bias, g.bias_dtype, col_c) : 0.0f;
-        auto inv_of = [&](int e) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv_lane), e)); };
-        const int64_t salient = g.salient_count;
-        float v[64];
-#pragma unroll
-        for (int e = 0; e < 64; ++e) v[e] = park[e * kParkStride + p_lane] * inv_of(e) * cs + bias;
-        // Salient columns (none for most layers): v[e] for the wave's 64 rows
-        // stays in registers while the columns are added in index order, eight at
-        // a time. Lane e loads x[row0 + e, idx_k] and the row loop takes it with
-        // readlane, so a batch of eight columns costs one round of loads.
-        for (int64_t k0 = 0; k0 < salient; k0 += 8) {
-            float xk[8], wk[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int64_t k = k0 + j < salient ? k0 + j : salient - 1;
-                const int64_t idx = g.salient_indices[k];
-                xk[j] = nq::load_f32(g.x, g.x_dtype, (row0 + lane_row) * g.in + idx);
-                float w = nq::load_f32(g.salient_values, g.salient_dtype, col_c * salient + k);
-                if (g.salient_scales) w *= nq::load_f32(g.salient_scales, g.scale_dtype, k);
-                wk[j] = k0 + j < salient ? w : 0.0f;
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (k0 + j < salient) {
-#pragma unroll
-                    for (int e = 0; e < 64; ++e)
-                        v[e] += wk[j] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xk[j]), e));
-                }
-            }
-        }
-        if (g.out_scale) {
-            // The rank intermediate for GEMM 2: fp16, row-scaled, swizzled, with
-            // the padding columns up to out_ld written as zeros (a 256-wide
-            // block can reach past out_ld: those lanes store nothing); split:
-            // the prepared-row layout, high parts and remainders.
-            const float os_lane = g.out_scale[row0 + lane_row];
-            const bool in_row = lane_ok && col < g.out_ld;
-            const int64_t cc = in_row ? col : 0;
-            const int64_t stride = kPlanes * g.out_ld;
-            _Float16* o = static_cast<_Float16*>(g.out) + row0 * stride + (cc >> 7) * (128 * kPlanes) +
-                          swizzle4(cc & 127);
-#pragma unroll
-            for (int e = 0; e < 64; ++e) {
-                const float os = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(os_lane), e));
-                if (e < rows && in_row) {
-                    const float x = col_ok ? v[e] * os : 0.0f;
-                    const _Float16 hi = static_cast<_Float16>(x);
-                    o[e * stride] = hi;
-                    if constexpr (SPLIT) o[e * stride + 128] = static_cast<_Float16>(x - static_cast<float>(hi));
-                }
-            }
-            return;
-        }
-        if (!col_ok) return;
-        // One switch on the output dtype, then 64 predicated stores with
-        // constant register indices.
-        const int64_t out0 = row0 * g.n + col;
-        switch (g.out_dtype) {
-            case NQ_DTYPE_F32: {
-                float* o = static_cast<float*>(g.out) + out0;
-#pragma unroll
-                for (int e = 0; e < 64; ++e)
-                    if (e < rows) o[e * g.n] = v[e];
-                break;
-            }
-            case NQ_DTYPE_F16: {
-                _Float16* o = static_cast<_Float16*>(g.out) + out0;
-#pragma unroll
-                for (int e = 0; e < 64; ++e)
-                    if (e < rows) o[e * g.n] = static_cast<_Float16>(v[e]);
-                break;
-            }
-            case NQ_DTYPE_BF16: {
-                uint16_t* o = static_cast<uint16_t*>(g.out) + out0;
-#pragma unroll
-                for (int e = 0; e < 64; ++e)
-                    if (e < rows) o[e * g.n] = nq::f32_to_bf16_bits(v[e]);
-                break;
-            }
-            default:
-                break;
-        }
+        for (int ii = 0; ii < II; ++ii) next_ea[ii] = *reinterpret_cast<const uint16_t*>(base + et[ii]);
+        exp_at = uniform64(more ? exp_at + exp_stride : exp_at);
     };
-    // Park fragments ii0 and ii0 + 1 (a 64-row half), then emit it. Written
-    // out per half rather than as a loop: the accumulators must keep constant
-    // register indices, and the compiler does not always unroll a loop around
-    // two copies of emit.
-    const auto park_half = [&](const v16f (&a0)[JJ], const v16f (&a1)[JJ]) __attribute__((always_inline)) {
+    // Ring form: the two words of block sc for this lane, from LDS.
+    const auto read_words = [&](int sc, uint32_t (&w)[2]) __attribute__((always_inline)) {
+        const int rem = nsc - (sc & ~3), dw = rem < 4 ? rem : 4;
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(lds + NB * (kStepBytes + kExpBytes) +
+                                                              ((sc >> 2) & 1) * kWordBytes) +
+                            (2 * wn + (r >> 4)) * 256 + (sc & 3);
+        w[0] = p[wl0 * dw], w[1] = p[wl1 * dw];
+    };
+    const auto take_words = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int jj = 0; jj < JJ; ++jj)
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                park[(8 * (q >> 2) + 4 * h + (q & 3)) * kParkStride + 32 * jj + r] = a0[jj][q];
-                park[(32 + 8 * (q >> 2) + 4 * h + (q & 3)) * kParkStride + 32 * jj + r] = a1[jj][q];
-            }
+            for (int i = 0; i < W; ++i)
+                words[jj][0][i] = next_words[jj][0][i], words[jj][1][i] = next_words[jj][1][i];
     };
-    park_half(acc[0], acc[1]);
-    __syncthreads();
-    emit(m0 + 32 * II * wm);
-    if constexpr (II == 4) {
-        __syncthreads();  // the first half is read out of the park area
-        park_half(acc[2], acc[3]);
+    const auto take_exps = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int ii = 0; ii < II; ++ii) ea[ii] = next_ea[ii];
+    };
+    // Step s computes on buffer s & 1 while the tile of step s + 1 moves into
+    // the other; a wait for this wave's transfers and one barrier per step
+    // make every wave's part of the next tile visible before it is read.
+    // Ring: step s computes on buffer s % NB while the next NB - 1 steps move;
+    // the wait leaves the transfers of the youngest NB - 2 in flight (counted
+    // as the fewest a wave issues per step).
+    constexpr int kInFlight = (NB - 2) * NL;
+    uint32_t ring_words[2];
+    if constexpr (kRing) {
+        load_words_ring(k_begin >> 2);
+#pragma unroll
+        for (int i = 0; i < NB - 1; ++i) {
+            load_exps_ring(i, k_begin + i + 1 < k_end);
+            load_a(i, k_begin + i + 1 < k_end);
+        }
+        __builtin_amdgcn_s_waitcnt(wait_vmcnt(kInFlight));
         __syncthreads();
-        emit(m0 + 32 * II * wm + 64);
+        read_words(k_begin, ring_words);
+    } else {
+        load_a(0, k_begin + 1 < k_end);
+        load_words(k_begin);
+        load_exps(k_begin + 1 < k_end);
+        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+        __syncthreads();
+        take_words();
+        take_exps();
+    }
+    int buf = 0;
+    uint32_t sign_mask = 0x88888888u, fp4_one = 0x22222222u;
+    // B scales 2^(-5p) of planes 0-3 (one byte each) and 4.
+    constexpr int kE = kPlaneBits;
+    int eb = 127 | (127 - kE) << 8 | (127 - 2 * kE) << 16 | (127 - 3 * kE) << 24, eb4 = 127 - 4 * kE;
+    asm volatile("" : "+v"(sign_mask), "+v"(fp4_one), "+v"(eb), "+v"(eb4));  // keep them in VGPRs
+    // One K step, block sc, word `wi` of the run.
+    const auto step = [&](int sc, auto wi_) __attribute__((always_inline)) {
+        constexpr int wi = decltype(wi_)::value;
+        const bool more = sc + NB < k_end;
+        if constexpr (kRing) {
+            if (wi == 0 && sc + W < k_end) load_words_ring((sc >> 2) + 1);
+            const int idle = buf == 0 ? NB - 1 : buf - 1;
+            load_exps_ring(idle, more);
+            load_a(idle, more);
+            words[0][0][wi] = ring_words[0], words[0][1][wi] = ring_words[1];
+#pragma unroll
+            for (int ii = 0; ii < II; ++ii)
+                ea[ii] = *reinterpret_cast<const uint16_t*>(lds + NB * kStepBytes + buf * kExpBytes + 128 * ii + 2 * lane);
+        } else {
+            load_a(buf ^ 1, more);
+            if constexpr (wi == 0) load_words(sc + W < k_end ? sc + W : sc);
+            load_exps(more);
+        }
+        // The sign words of the next steps are issued here, ahead of the
+        // MFMAs; left to itself the scheduler sinks them to the step's end,
+        // where the wait before the barrier would take their whole latency.
+        __builtin_amdgcn_sched_barrier(0);
+        const char* const a_lds = lds + buf * kStepBytes + II * wm * kGroupLds;
+        const auto read_a = [&](int phase, v8i (&a)[II]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int ii = 0; ii < II; ++ii) {
+                const char* p = a_lds + ii * kGroupLds + phase * kPlaneBytes;
+                const uint4 lo = *reinterpret_cast<const uint4*>(p + 16 * lane);
+                const uint2 hi = *reinterpret_cast<const uint2*>(p + 1024 + 8 * lane);
+                a[ii] = v8i{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z),
+                            static_cast<int>(lo.w), static_cast<int>(hi.x), static_cast<int>(hi.y), 0, 0};
+            }
+        };
+        // Software pipeline over the 2 P phases: a phase's MFMAs issue while
+        // the next one's A fragments are read and, in the first step's last
+        // phases, the second step's signs are expanded.
+        v8i a_cur[II], b_cur[JJ], b_nxt[JJ];
+        read_a(0, a_cur);
+        if constexpr (kRing) read_words(sc + 1 < k_end ? sc + 1 : sc, ring_words);  // a chunk lands within its predecessor
+#pragma unroll
+        for (int jj = 0; jj < JJ; ++jj) b_cur[jj] = expand_signs(words[jj][0][wi], sign_mask, fp4_one);
+        each(std::make_integer_sequence<int, 2 * P>{}, [&](auto phase_) __attribute__((always_inline)) {
+            constexpr int kPhase = decltype(phase_)::value, kStep = kPhase / P, kPl = kPhase % P;
+            constexpr int kSum = NA > 1 && kPl > 1 ? 1 : 0;
+            __builtin_amdgcn_sched_barrier(0);
+            v8i a_nxt[II];
+            if constexpr (kPhase + 1 < 2 * P) read_a(kPhase + 1, a_nxt);
+            if constexpr (kPhase == P - 1 && kSignsAhead) {
+#pragma unroll
+                for (int jj = 0; jj < JJ; ++jj) b_nxt[jj] = expand_signs(words[jj][1][wi], sign_mask, fp4_one);
+            }
+            if constexpr (kPhase == P && !kSignsAhead) {
+#pragma unroll
+                for (int jj = 0; jj < JJ; ++jj) b_cur[jj] = expand_signs(words[jj][1][wi], sign_mask, fp4_one);
+            }
+#pragma unroll
+            for (int ii = 0; ii < II; ++ii)
+#pragma unroll
+                for (int jj = 0; jj < JJ; ++jj)
+                    sums[kSum][ii][jj] = mfma_plane<kStep, kPl>(a_cur[ii], b_cur[jj], sums[kSum][ii][jj], ea[ii], eb, eb4);
+            if constexpr (kPhase + 1 < 2 * P) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 2 * II, 0);  // LDS reads of the next phase
+#pragma unroll
+                for (int q = 0; q < II * JJ; ++q) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // a part of the expansion
+                }
+#pragma unroll
+                for (int ii = 0; ii < II; ++ii) a_cur[ii] = a_nxt[ii];
+            }
+            if constexpr (kPhase == P - 1 && kSignsAhead) {
+#pragma unroll
+                for (int jj = 0; jj < JJ; ++jj) b_cur[jj] = b_nxt[jj];
+            }
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kRing) {
+            __builtin_amdgcn_s_waitcnt(wait_vmcnt(kInFlight));
+            __syncthreads();
+            buf = buf + 1 < NB ? buf + 1 : 0;
+        } else {
+            take_exps();
+            __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+            __syncthreads();
+            buf ^= 1;
+        }
+    };
+    for (int sc = k_begin; sc < k_end; sc += W) {
+        each(std::make_integer_sequence<int, W>{}, [&](auto wi) __attribute__((always_inline)) {
+            if (sc + decltype(wi)::value < k_end) step(sc + decltype(wi)::value, wi);  // uniform
+        });
+        if constexpr (!kRing) take_words();
+    }
+    if constexpr (kRing) {  // the transfers past the last step, before LDS is used again
+        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+        __syncthreads();
+    }
+    if constexpr (NA > 1) {
+#pragma unroll
+        for (int ii = 0; ii < II; ++ii)
+#pragma unroll
+            for (int jj = 0; jj < JJ; ++jj) acc[ii][jj] += sums[1][ii][jj];
+    }
+    // Lane (h, r) holds D[8 (q / 4) + 4 h + q % 4][r] of each 32 x 32 tile; a
+    // store is 32 columns of two rows.
+    const int64_t row_w = m0 + kRows * II * wm, col_w = n0 + 32 * JJ * wn + r;
+    const auto store = [&](auto* out, int64_t ld, auto convert) __attribute__((always_inline)) {
+        const int64_t row0 = row_w + 4 * h;
+        const bool all = row_w + kRows * II <= g.m;  // uniform per wave
+        auto* const o = out + row0 * ld + col_w;
+#pragma unroll
+        for (int jj = 0; jj < JJ; ++jj) {
+            if (col_w + 32 * jj >= g.n) continue;
+            if (all) {
+#pragma unroll
+                for (int ii = 0; ii < II; ++ii)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q)
+                        o[(kRows * ii + 8 * (q >> 2) + (q & 3)) * ld + 32 * jj] = convert(acc[ii][jj][q]);
+            } else {
+#pragma unroll
+                for (int ii = 0; ii < II; ++ii)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) {
+                        const int row = kRows * ii + 8 * (q >> 2) + (q & 3);
+                        if (row0 + row < g.m) o[row * ld + 32 * jj] = convert(acc[ii][jj][q]);
+                    }
+            }
+        }
+    };
+    if (g.partial) {
+        store(g.partial + static_cast<int64_t>(slice) * g.m * part_ld(g.n), part_ld(g.n), [](float v) { return v; });
+        return;
+    }
+    float cs[JJ], bias[JJ];
+#pragma unroll
+    for (int jj = 0; jj < JJ; ++jj) {
+        const int64_t col = col_w + 32 * jj < g.n ? col_w + 32 * jj : g.n - 1;
+        cs[jj] = nq::load_f32(g.col_scale, g.col_scale_dtype, col);
+        bias[jj] = g.bias ? nq::load_f32(g.bias, g.bias_dtype, col) : 0.0f;
+    }
+    if (g.mid.planes) {
+        // The rank intermediate as planes: one row group of every wave at a
+        // time goes through LDS, so that a thread has the 32 columns that
+        // share an exponent. Columns past n are zero.
+        float* const park = reinterpret_cast<float*>(lds);
+        each(std::make_integer_sequence<int, II>{}, [&](auto ii_) __attribute__((always_inline)) {
+            constexpr int ii = decltype(ii_)::value;
+            if constexpr (ii > 0) __syncthreads();  // the rows before are read
+#pragma unroll
+            for (int jj = 0; jj < JJ; ++jj) {
+                const bool in = col_w + 32 * jj < g.n;
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    park[(kRows * wm + 8 * (q >> 2) + 4 * h + (q & 3)) * kParkStride + 32 * JJ * wn + 32 * jj + r] =
+                        in ? acc[ii][jj][q] * cs[jj] : 0.0f;
+            }
+            __syncthreads();
+            for (int task = threadIdx.x; task < WR * kRows * (BN / kBK) * 4; task += kBlock) {
+                const int grp = (task >> 4) & 3, rest = task >> 6;
+                const int prow = 16 * (rest % (2 * WR)) + (task & 15), kbl = rest / (2 * WR);
+                const int64_t row = m0 + kRows * (II * (prow >> 5) + ii) + (prow & 31);
+                const int64_t kb = n0 / kBK + kbl;
+                if (row >= g.m || kb >= g.mid_blocks) continue;
+                const float* src = park + prow * kParkStride + kbl * kBK + 4 * grp;
+                v16f half[2];
+#pragma unroll
+                for (int m = 0; m < 8; ++m) {
+                    const v4f v = *reinterpret_cast<const v4f*>(src + 16 * m);
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) half[m >> 2][4 * (m & 3) + b] = v[b];
+                }
+                store_group<P>(g.mid, row, kb, grp, half[0], half[1]);
+            }
+        });
+        return;
+    }
+#pragma unroll
+    for (int ii = 0; ii < II; ++ii)
+#pragma unroll
+        for (int jj = 0; jj < JJ; ++jj)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[ii][jj][q] = acc[ii][jj][q] * cs[jj] + bias[jj];
+    // Salient columns (none for most layers), kSalient at a time in index
+    // order: x of the block's rows goes through LDS.
+    float* const sx = reinterpret_cast<float*>(lds);  // [kSalient][BM]
+    for (int64_t k0 = 0; k0 < g.salient_count; k0 += kSalient) {
+        const int count = static_cast<int>(g.salient_count - k0 < kSalient ? g.salient_count - k0 : kSalient);
+        if (k0 > 0) __syncthreads();
+        for (int i = threadIdx.x; i < count * BM; i += kBlock) {
+            const int64_t row = m0 + i % BM < g.m ? m0 + i % BM : g.m - 1;
+            sx[i] = nq::load_f32(g.x, g.x_dtype, row * g.in + g.salient_indices[k0 + i / BM]);
+        }
+        __syncthreads();
+        for (int k = 0; k < count; ++k) {
+            float w[JJ];
+#pragma unroll
+            for (int jj = 0; jj < JJ; ++jj) {
+                const int64_t col = col_w + 32 * jj < g.n ? col_w + 32 * jj : g.n - 1;
+                w[jj] = nq::load_f32(g.salient_values, g.salient_dtype, col * g.salient_count + k0 + k);
+                if (g.salient_scales) w[jj] *= nq::load_f32(g.salient_scales, g.scale_dtype, k0 + k);
+            }
+#pragma unroll
+            for (int ii = 0; ii < II; ++ii)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const v4f xr = *reinterpret_cast<const v4f*>(sx + k * BM + kRows * (II * wm + ii) + 8 * i + 4 * h);
+#pragma unroll
+                    for (int jj = 0; jj < JJ; ++jj)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[ii][jj][4 * i + j] += w[jj] * xr[j];
+                }
+        }
+    }
+    switch (g.out_dtype) {
+        case NQ_DTYPE_F32:
+            store(static_cast<float*>(g.out), g.n, [](float v) { return v; });
+            break;
+        case NQ_DTYPE_F16:
+            store(static_cast<_Float16*>(g.out), g.n, [](float v) { return static_cast<_Float16>(v); });
+            break;
+        case NQ_DTYPE_BF16:
+            store(static_cast<uint16_t*>(g.out), g.n, [](float v) { return nq::f32_to_bf16_bits(v); });
+            break;
+        default:
+            break;
     }
 }
 
@@ -761,15 +777,169 @@ __device__ __forceinline__ float raw2_value(const Raw2& r, int dtype) {
     return dtype == NQ_DTYPE_F32 ? f32 : (dtype == NQ_DTYPE_BF16 ? bf16 : f16);
 }
 
-// Split-K epilogue, one thread per output element (t, c), grid (the members'
-// column blocks, token rows; t = blockIdx.y + kRowsPerGridZ * blockIdx.z): out[t, c] =
-// (Σ_z partial[z][t][c]) / row_scale[t] * col_scale[c] (+ bias + salient
-// columns for GEMM 2), the slices summed in z order. The column's scale and
-// bias and the first eight partials are loaded before any is used. With
-// out_scale the threads cover out_ld columns and write the fp16 rank
-// intermediate as the direct epilogue does (zeros past column n).
-constexpr int64_t kRowsPerGridZ = 65535;
+// A GEMM of few tokens and few sign rows: a workgroup takes 32 sign rows and
+// its eight waves share the K blocks out (chunks of four, dealt in turn), so
+// that even a small matrix keeps most of the chip busy without a second launch
+// for partial sums. Nothing is shared between the waves until their sums meet
+// in LDS (added in wave order): A fragments go straight from memory (the
+// operand's order is the fragment's) to registers, a step ahead. GEMM 1 takes
+// the 32 rows of one exponent group of the rank intermediate: tile rows
+// 16 m + 4 g + b of its 128-column block, in lane 4 m + b. Bound by latency.
+// Calls with both GEMMs here and on k_sign_gemm: 4096 -> 4096 r1638 at 24
+// tokens 15.9 and 24.6 us, at 61 21.9 and 26.4; at 128 23.6 and 27.8.
+constexpr int kFewWaves = 8;
 
+template <int II, int P>
+__global__ __launch_bounds__(kFewWaves * 64, 2) void k_sign_gemm_few(const GemmBatch batch) {
+    constexpr int Q = 16 * II;                // sums per lane
+    constexpr int kOwn = Q / kFewWaves;       // of which a wave finishes
+    constexpr int kParkStride = 36;
+    __shared__ __attribute__((aligned(16))) float red[kFewWaves * Q * 64];
+    const int member = batch_member(batch, static_cast<int>(blockIdx.x));
+    const GemmArgs& g = batch.p[member];
+    const int ct = static_cast<int>(blockIdx.x) - batch.begin[member];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int h = lane >> 5, r = lane & 31;
+    const int64_t row_block = static_cast<int64_t>(blockIdx.z) * kRowsPerGridZ + blockIdx.y;
+    const int64_t m0 = row_block * (kRows * II);
+    if (m0 >= g.m) return;  // uniform
+    const bool mid = g.mid.planes != nullptr;
+    const int64_t col = mid ? static_cast<int64_t>(ct >> 2) * 128 + 16 * (r >> 2) + 4 * (ct & 3) + (r & 3)
+                            : static_cast<int64_t>(ct) * 32 + r;
+    const int64_t col_c = col < g.n ? col : g.n - 1;  // its words feed sums that are not stored
+    const int nsc = static_cast<int>(g.nb);
+    const int64_t groups = g.a.row_groups, rg0 = row_block * II;
+    const uint32_t* const bt = g.tiles + (col_c >> 4) * nsc * 64;
+    const int wl = 16 * h + static_cast<int>(col_c & 15);
+    const uint8_t* at[II];
+    const uint8_t* et[II];
+#pragma unroll
+    for (int ii = 0; ii < II; ++ii) {
+        const int64_t rg = rg0 + ii < groups ? rg0 + ii : groups - 1;
+        at[ii] = g.a.planes + rg * (2 * P * kPlaneBytes);
+        et[ii] = g.a.exps + rg * 128 + 2 * lane;
+    }
+    constexpr int NA = P > 3 ? 2 : 1;  // as in k_sign_gemm
+    v16f sums[NA][II];
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int ii = 0; ii < II; ++ii) sums[a][ii] = v16f{};
+    uint32_t sign_mask = 0x88888888u, fp4_one = 0x22222222u;
+    constexpr int kE = kPlaneBits;
+    int eb = 127 | (127 - kE) << 8 | (127 - 2 * kE) << 16 | (127 - 3 * kE) << 24, eb4 = 127 - 4 * kE;
+    asm volatile("" : "+v"(sign_mask), "+v"(fp4_one), "+v"(eb), "+v"(eb4));  // keep them in VGPRs
+    struct Step {
+        uint4 lo[II][2 * P];
+        uint2 hi[II][2 * P];
+        int ea[II];
+    };
+    const auto load = [&](int sc, Step& s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ii = 0; ii < II; ++ii) {
+            const uint8_t* p = at[ii] + sc * groups * (2 * P * kPlaneBytes);
+#pragma unroll
+            for (int f = 0; f < 2 * P; ++f) {
+                s.lo[ii][f] = *reinterpret_cast<const uint4*>(p + f * kPlaneBytes + 16 * lane);
+                s.hi[ii][f] = *reinterpret_cast<const uint2*>(p + f * kPlaneBytes + 1024 + 8 * lane);
+            }
+            s.ea[ii] = *reinterpret_cast<const uint16_t*>(et[ii] + sc * groups * 128);
+        }
+    };
+    for (int chunk = wave; 4 * chunk < nsc; chunk += kFewWaves) {
+        const int dw = nsc - 4 * chunk < 4 ? nsc - 4 * chunk : 4;
+        // Four words side by side (a narrow last chunk's load runs into what follows it, not used).
+        const WordRun<4> w0 = *reinterpret_cast<const WordRun<4>*>(bt + chunk * 256 + wl * dw);
+        const WordRun<4> w1 = *reinterpret_cast<const WordRun<4>*>(bt + chunk * 256 + (wl + 32) * dw);
+        Step cur, nxt;
+        load(4 * chunk, cur);
+        each(std::make_integer_sequence<int, 4>{}, [&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            if (i >= dw) return;  // uniform
+            if (i + 1 < 4) load(4 * chunk + (i + 1 < dw ? i + 1 : i), nxt);
+            __builtin_amdgcn_sched_barrier(0);  // the next step's loads stay ahead of this one's MFMAs
+            each(std::make_integer_sequence<int, 2 * P>{}, [&](auto f_) __attribute__((always_inline)) {
+                constexpr int f = decltype(f_)::value, kStep = f / P, kPl = f % P;
+                constexpr int kSum = NA > 1 && kPl > 1 ? 1 : 0;
+                const v8i b = expand_signs(kStep ? w1.w[i] : w0.w[i], sign_mask, fp4_one);
+#pragma unroll
+                for (int ii = 0; ii < II; ++ii) {
+                    const uint4 lo = cur.lo[ii][f];
+                    const uint2 hi = cur.hi[ii][f];
+                    const v8i a = v8i{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z),
+                                      static_cast<int>(lo.w), static_cast<int>(hi.x), static_cast<int>(hi.y), 0, 0};
+                    sums[kSum][ii] = mfma_plane<kStep, kPl>(a, b, sums[kSum][ii], cur.ea[ii], eb, eb4);
+                }
+            });
+            cur = nxt;
+        });
+    }
+#pragma unroll
+    for (int ii = 0; ii < II; ++ii) {
+        if constexpr (NA > 1) sums[0][ii] += sums[1][ii];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) red[(wave * Q + 16 * ii + q) * 64 + lane] = sums[0][ii][q];
+    }
+    __syncthreads();
+    // Wave w finishes sums [w kOwn, + kOwn): rows 32 ii + 8 (q / 4) + 4 h + q % 4.
+    const Raw2 cs_raw = load_raw2(g.col_scale, g.col_scale_dtype, col_c);
+    const Raw2 bias_raw =
+        load_raw2(g.bias ? g.bias : g.col_scale, g.bias ? g.bias_dtype : g.col_scale_dtype, col_c);
+    const float cs = raw2_value(cs_raw, g.col_scale_dtype);
+    float v[kOwn];
+    int row[kOwn];
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+        const int q = wave * kOwn + i;
+        row[i] = kRows * (q >> 4) + 8 * ((q & 15) >> 2) + 4 * h + (q & 3);
+        v[i] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kFewWaves; ++k) v[i] += red[(k * Q + q) * 64 + lane];
+        v[i] *= cs;
+    }
+    if (mid) {
+        __syncthreads();  // every sum is read
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) red[row[i] * kParkStride + r] = col < g.n ? v[i] : 0.0f;
+        __syncthreads();
+        const int t = threadIdx.x;
+        if (t >= kRows * II || m0 + t >= g.m) return;
+        v16f half[2];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const v4f x = *reinterpret_cast<const v4f*>(red + t * kParkStride + 4 * i);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) half[i >> 2][4 * (i & 3) + b] = x[b];
+        }
+        store_group<P>(g.mid, m0 + t, ct >> 2, ct & 3, half[0], half[1]);
+        return;
+    }
+    if (col >= g.n) return;
+    if (g.bias) {
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) v[i] += raw2_value(bias_raw, g.bias_dtype);
+    }
+    for (int64_t k = 0; k < g.salient_count; ++k) {
+        float w = nq::load_f32(g.salient_values, g.salient_dtype, col * g.salient_count + k);
+        if (g.salient_scales) w *= nq::load_f32(g.salient_scales, g.scale_dtype, k);
+        const int64_t idx = g.salient_indices[k];
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) {
+            const int64_t t = m0 + row[i] < g.m ? m0 + row[i] : g.m - 1;
+            v[i] += w * nq::load_f32(g.x, g.x_dtype, t * g.in + idx);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i)
+        if (m0 + row[i] < g.m) nq::store_f32_as(g.out, g.out_dtype, (m0 + row[i]) * g.n + col, v[i]);
+}
+
+// Split-K epilogue of GEMM 2, one thread per output element (t, c), grid (the
+// members' column blocks, token rows; t = blockIdx.y + kRowsPerGridZ *
+// blockIdx.z): out[t, c] = (Σ_z partial[z][t][c]) * col_scale[c] + bias +
+// salient columns, the slices summed in z order. The column's scale and bias
+// and the first eight partials are loaded before any is used.
 __global__ __launch_bounds__(kBlock) void k_reduce_splits(const GemmBatch batch) {
     const int member = batch_member(batch, static_cast<int>(blockIdx.x));
     const GemmArgs& ga = batch.p[member];
@@ -779,21 +949,16 @@ __global__ __launch_bounds__(kBlock) void k_reduce_splits(const GemmBatch batch)
     GemmArgs g;
     g.m = ga.m;
     g.n = ga.n;
-    g.out_ld = ga.out_ld;
-    g.out_scale = ga.out_scale;
     g.out = ga.out;
     g.out_dtype = ga.out_dtype;
     g.partial = ga.partial;
-    g.row_scale = ga.row_scale;
     g.col_scale = ga.col_scale;
     g.col_scale_dtype = ga.col_scale_dtype;
     g.bias = ga.bias;
     g.bias_dtype = ga.bias_dtype;
     g.salient_count = ga.salient_count;
-    g.split = ga.split;
-    asm volatile("" ::"s"(g.m), "s"(g.n), "s"(g.out_ld), "s"(g.out_scale), "s"(g.out), "s"(g.out_dtype),
-                 "s"(g.partial), "s"(g.row_scale), "s"(g.col_scale), "s"(g.col_scale_dtype), "s"(g.bias),
-                 "s"(g.bias_dtype), "s"(g.salient_count), "s"(splits));
+    asm volatile("" ::"s"(g.m), "s"(g.n), "s"(g.out), "s"(g.out_dtype), "s"(g.partial), "s"(g.col_scale),
+                 "s"(g.col_scale_dtype), "s"(g.bias), "s"(g.bias_dtype), "s"(g.salient_count), "s"(splits));
     g.salient_values = ga.salient_values;
     g.salient_dtype = ga.salient_dtype;
     g.salient_scales = ga.salient_scales;
@@ -804,21 +969,9 @@ __global__ __launch_bounds__(kBlock) void k_reduce_splits(const GemmBatch batch)
     g.in = ga.in;
     const int64_t c = static_cast<int64_t>(static_cast<int>(blockIdx.x) - batch.begin[member]) * kBlock + threadIdx.x;
     const int64_t t = static_cast<int64_t>(blockIdx.z) * kRowsPerGridZ + blockIdx.y;
-    const int64_t width = g.out_scale ? g.out_ld : g.n;
-    if (splits <= 1 || c >= width || t >= g.m) return;  // members without a split have no partials
-    // With out_scale: the rank intermediate's position of column c (split
-    // operands: the high part, its remainder 128 further).
-    const int64_t planes = g.split ? 2 : 1;
-    _Float16* const lm = g.out_scale ? static_cast<_Float16*>(g.out) + t * planes * g.out_ld +
-                                           (c >> 7) * (128 * planes) + swizzle4(c & 127)
-                                     : nullptr;
-    if (c >= g.n) {  // only with out_scale: a padding column of the rank intermediate
-        lm[0] = static_cast<_Float16>(0.0f);
-        if (g.split) lm[128] = static_cast<_Float16>(0.0f);
-        return;
-    }
-    const int64_t plane = g.m * g.n;
-    const int64_t pi = t * g.n + c;
+    if (splits <= 1 || c >= g.n || t >= g.m) return;  // members without a split have no partials
+    const int64_t plane = g.m * part_ld(g.n);
+    const int64_t pi = t * part_ld(g.n) + c;
     const Raw2 cs_raw = load_raw2(g.col_scale, g.col_scale_dtype, c);
     const Raw2 bias_raw = load_raw2(g.bias ? g.bias : g.col_scale, g.bias ? g.bias_dtype : g.col_scale_dtype, c);
     float part[8];
@@ -829,21 +982,64 @@ __global__ __launch_bounds__(kBlock) void k_reduce_splits(const GemmBatch batch)
 #pragma unroll
         for (int j = 0; j < 8; ++j) v += part[j];
     }
-    v = v / g.row_scale[t] * raw2_value(cs_raw, g.col_scale_dtype);
+    v *= raw2_value(cs_raw, g.col_scale_dtype);
     if (g.bias) v += raw2_value(bias_raw, g.bias_dtype);
     for (int64_t k = 0; k < g.salient_count; ++k) {
         float w = nq::load_f32(g.salient_values, g.salient_dtype, c * g.salient_count + k);
         if (g.salient_scales) w *= nq::load_f32(g.salient_scales, g.scale_dtype, k);
         v += w * nq::load_f32(g.x, g.x_dtype, t * g.in + g.salient_indices[k]);
     }
-    if (g.out_scale) {
-        const float x = v * g.out_scale[t];
-        const _Float16 hi = static_cast<_Float16>(x);
-        lm[0] = hi;
-        if (g.split) lm[128] = static_cast<_Float16>(x - static_cast<float>(hi));
-    } else {
-        nq::store_f32_as(g.out, g.out_dtype, pi, v);
+    nq::store_f32_as(g.out, g.out_dtype, t * g.n + c, v);
+}
+
+// Split-K epilogue of GEMM 1: planes of (Σ_z partial[z][t][c]) * col_scale[c],
+// zero past the last column. A workgroup takes one 128-column block of 16 rows
+// (16-row groups blockIdx.y + kRowsPerGridZ * blockIdx.z): lane 16 g + r has the
+// 32 columns of row r that share an exponent, wave w sums slices w, w + 4, ...
+// (bound by latency: every load of a slice is issued at once), and the waves
+// meet in LDS in order.
+template <int P>
+__global__ __launch_bounds__(kBlock) void k_reduce_mid(const GemmBatch batch) {
+    __shared__ float sum[3][32][64];
+    const int member = batch_member(batch, static_cast<int>(blockIdx.x));
+    const GemmArgs& g = batch.p[member];
+    const int splits = static_cast<int>(g.splits);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane >> 4;
+    const int64_t kb = static_cast<int>(blockIdx.x) - batch.begin[member];
+    const int64_t row = (static_cast<int64_t>(blockIdx.z) * kRowsPerGridZ + blockIdx.y) * 16 + (lane & 15);
+    const int64_t c0 = kb * kBK + 4 * grp, ld = part_ld(g.n), plane = g.m * ld;
+    const float* src = g.partial + (row < g.m ? row : g.m - 1) * ld + wave * plane;
+    Raw2 cs[32];
+    if (wave == 0) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+            const int64_t c = c0 + 16 * (i >> 2) + (i & 3);
+            cs[i] = load_raw2(g.col_scale, g.col_scale_dtype, c < g.n ? c : g.n - 1);
+        }
     }
+    v16f half[2] = {v16f{}, v16f{}};
+    for (int z = wave; z < splits; z += 4, src += 4 * plane) {
+        v4f v[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] = *reinterpret_cast<const v4f*>(src + (c0 + 16 * m < g.n ? c0 + 16 * m : 0));
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) half[m >> 2][4 * (m & 3) + b] += v[m][b];
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) sum[wave - 1][i][lane] = half[i >> 4][i & 15];
+    }
+    __syncthreads();
+    if (wave > 0 || row >= g.m) return;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        const int64_t c = c0 + 16 * (i >> 2) + (i & 3);
+        const float v = ((half[i >> 4][i & 15] + sum[0][i][lane]) + sum[1][i][lane]) + sum[2][i][lane];
+        half[i >> 4][i & 15] = c < g.n ? v * raw2_value(cs[i], g.col_scale_dtype) : 0.0f;
+    }
+    store_group<P>(g.mid, row, kb, grp, half[0], half[1]);
 }
 
 // Tile counts and 128-column block counts of V [rank, in] and U [out, rank]
@@ -865,178 +1061,202 @@ Geometry geometry(const nq_linear_desc* d) {
 
 int64_t a256(int64_t n) { return (n + 255) & ~int64_t(255); }
 
-// Split of a GEMM with `tiles` (token, sign-row) tiles over K blocks, from a
-// latency model of the K loop (fitted to layer timings on MI355X): a K step
-// costs kStepNs (the next step's tile is in flight during the current one,
-// so a step is about one compute pass, not a memory round trip), while the GPU holds every
-// workgroup at once (kResident: two per CU, bound by LDS); workgroups beyond
-// that run in further rounds; a split adds the reduce launch and the
-// partials' write and read (M x N x 4 bytes per slice, mostly served by the
-// last-level cache). Slices hold at least kMinSliceBlocks K blocks.
-constexpr int64_t kResident = 512;
-constexpr int64_t kResidentSmall = 1024;  // the 64 x 128 block: four per CU
-constexpr double kStepNsSmall = 500.0;    // half the MFMA and A work of a 128-row step
-constexpr int64_t kMinSliceBlocks = 2;
-constexpr double kStepNs = 1000.0;
-constexpr double kReduceNsSmall = 3000.0;  // the reduce launch after 64 x 128 blocks
-constexpr double kReduceNs = 6000.0;       // and after 128-row blocks (measured: 2.5% faster at
-                                           // 256 tokens than 3000, the same above)
-constexpr double kPartialBytesPerNs = 8000.0;
+// Block shapes of k_sign_gemm: tokens x sign rows, and for three and five
+// planes the time of a K step of a workgroup that has its CU to itself and
+// what each of several sharing the CU adds (us, fitted to the sweeps below).
+struct Shape {
+    int64_t rows, cols;
+    double alone[2], shared[2];
+};
+enum ShapeId { kShape32x128, kShape64x128, kShape64x256, kShape128x128, kShape128x256, kShapes, kFew32, kFew64 };
+constexpr Shape kShape[kShapes] = {{32, 128, {0.45, 0.60}, {0.33, 0.44}},
+                                   {64, 128, {0.62, 0.85}, {0.52, 0.80}},
+                                   {64, 256, {0.00, 1.30}, {0.00, 1.15}},   // five planes only
+                                   {128, 128, {1.10, 0.00}, {0.80, 0.00}},  // three planes only
+                                   {128, 256, {1.90, 0.00}, {1.55, 0.00}}};
 
-struct Split {
-    int64_t slices, k_per_split;
+// Block shape (or k_sign_gemm_few's rows) and K slices of one phase's launch.
+struct Plan {
+    int shape;
+    int64_t k_per_split[kPrefillBatch], slices[kPrefillBatch];
 };
 
-// Resident workgroups, K-step cost and reduce cost of the block tile used for `tokens`.
-int64_t resident_for(int64_t tokens) { return tokens <= kBM / 2 ? kResidentSmall : kResident; }
-double step_ns_for(int64_t tokens) { return tokens <= kBM / 2 ? kStepNsSmall : kStepNs; }
-double reduce_ns_for(int64_t tokens) { return tokens <= kBM / 2 ? kReduceNsSmall : kReduceNs; }
+// Plan of a phase: the shape and split with the least time by a model of its K
+// steps, (steps + 2) x the step's time at the CU's average load, plus a
+// reduction where K is split. Narrow shapes win while the grid is small: a
+// step's time is mostly its own chain (barrier, LDS reads, dependent MFMAs).
+// Measured on whole calls (us; every GEMM on one shape, no split: 32 x 128, 64
+// x 128, 128 x 128, 128 x 256; then this plan): 4096 -> 4096 r1638 at 512
+// tokens 34, 40, 55, 80; 34. 4096 -> 2 x 14336 r2549 at 512 126, 106, 108, 118;
+// 90-102. 4096 -> 2 x 12288 r3072 at 2048 452, 374, 346, 322; 318-335. Splits
+// pay only for few tokens of long rows (14336 -> 4096 r2549 at 61: 58 us
+// unsplit, 34 with GEMM 1 in eight slices).
+// A small grid goes to k_sign_gemm_few: 256 workgroups of 32 sign rows and 32
+// tokens (64 above 32) or fewer; beyond, every one of them reading all of A
+// costs more (2 x 12288 sign rows, 768 workgroups, at 24 tokens: 27 us against
+// 24), and so do more than 48 K blocks (10240 columns at 61 tokens: 33.5
+// against 28.8) unless the operand is the smallest (at 24: 23.1 and 26.9).
+constexpr int64_t kFewWgs = 256, kFewBlocks = 48;
+constexpr double kCus = 256.0;
+constexpr int64_t kMinSliceBlocks = 4;
+constexpr double kReduceUs = 5.0;
+constexpr double kPartialBytesPerUs = 4.0e6;
 
-Split split_for(int64_t tiles, int64_t k_blocks, int64_t tokens, int64_t n) {
-    const int64_t resident = resident_for(tokens);
-    const double step_ns = step_ns_for(tokens);
-    Split best{1, k_blocks};
-    double best_ns = -1.0;
-    const int64_t most = k_blocks / kMinSliceBlocks > 1 ? k_blocks / kMinSliceBlocks : 1;
-    for (int64_t want = 1; want <= most; ++want) {
-        Split s;
-        s.k_per_split = (k_blocks + want - 1) / want;
-        s.slices = (k_blocks + s.k_per_split - 1) / s.k_per_split;
-        const int64_t rounds = (tiles * s.slices + resident - 1) / resident;
-        double ns = static_cast<double>(rounds * (s.k_per_split + 1)) * step_ns;
-        if (s.slices > 1)
-            ns += reduce_ns_for(tokens) + 2.0 * static_cast<double>(s.slices * tokens * n * 4) / kPartialBytesPerNs;
-        if (best_ns < 0.0 || ns < best_ns) best = s, best_ns = ns;
+Plan plan_phase(int count, const int64_t* k_blocks, const int64_t* n, const int64_t* cap, int64_t tokens, int planes) {
+    Plan best{};
+    double best_us = -1.0;
+    const int wide = planes == kPlanesSplit ? 1 : 0;
+    int64_t kb_max = 1;
+    for (int i = 0; i < count; ++i) kb_max = k_blocks[i] > kb_max ? k_blocks[i] : kb_max;
+    for (int id = 0; id < kShapes; ++id) {
+        const Shape& sh = kShape[id];
+        if (sh.alone[wide] == 0.0 || (id > 0 && tokens <= kShape[id].rows / 2)) continue;
+        const int64_t mt = (tokens + sh.rows - 1) / sh.rows;
+        for (int64_t kmax = kb_max; kmax >= 1; --kmax) {
+            Plan p{};
+            p.shape = id;
+            int64_t wgs = 0, steps = 0, partial_elems = 0;
+            for (int i = 0; i < count; ++i) {
+                const int64_t most_k = k_blocks[i] / kMinSliceBlocks > 1 ? k_blocks[i] / kMinSliceBlocks : 1;
+                const int64_t most_cap = cap[i] / (tokens * part_ld(n[i])) > 1 ? cap[i] / (tokens * part_ld(n[i])) : 1;
+                int64_t sl = (k_blocks[i] + kmax - 1) / kmax;
+                sl = sl < most_k ? sl : most_k;
+                sl = sl < most_cap ? sl : most_cap;
+                p.k_per_split[i] = ((k_blocks[i] + sl - 1) / sl + 3) / 4 * 4;  // sign words load in runs of four
+                p.slices[i] = (k_blocks[i] + p.k_per_split[i] - 1) / p.k_per_split[i];
+                wgs += mt * ((n[i] + sh.cols - 1) / sh.cols) * p.slices[i];
+                const int64_t own = p.k_per_split[i] < k_blocks[i] ? p.k_per_split[i] : k_blocks[i];
+                steps = own > steps ? own : steps;
+                if (p.slices[i] > 1) partial_elems += p.slices[i] * tokens * n[i];
+            }
+            const double per_cu = static_cast<double>(wgs) / kCus;
+            const double whole = static_cast<double>(static_cast<int64_t>((wgs + 255) / 256));
+            const double busy = (per_cu + whole) / 2 * sh.shared[wide];
+            double us = static_cast<double>(steps + 2) * (per_cu > 1.0 && busy > sh.alone[wide] ? busy : sh.alone[wide]);
+            if (partial_elems > 0) us += kReduceUs + 2.0 * static_cast<double>(partial_elems * 4) / kPartialBytesPerUs;
+            if (best_us < 0.0 || us < best_us) best = p, best_us = us;
+        }
+    }
+    const bool few64 = tokens > 32 && planes == kPlanes;  // five planes of 64 rows would spill
+    int64_t few_wgs = 0;
+    for (int i = 0; i < count; ++i) few_wgs += (n[i] + 31) / 32;
+    few_wgs *= (tokens + (few64 ? 63 : 31)) / (few64 ? 64 : 32);
+    if (few_wgs <= kFewWgs && (kb_max <= kFewBlocks || (tokens <= 32 && planes == kPlanes))) {
+        best = Plan{};
+        best.shape = few64 ? kFew64 : kFew32;
+        for (int i = 0; i < count; ++i) best.k_per_split[i] = k_blocks[i], best.slices[i] = 1;
     }
     return best;
 }
 
-// Splits of the members of one batched GEMM launch: each member's slices
-// come from one bound kmax on K blocks per workgroup, chosen by the same
-// latency model over the whole launch (its workgroups share the GPU), and
-// stay within what the member's partial buffer holds (cap[i] elements) and
-// kMinSliceBlocks. A batch of one takes split_for's choice, which the
-// member's workspace is sized for.
-void batch_splits(int count, const int64_t* tiles, const int64_t* k_blocks, const int64_t* n, const int64_t* cap,
-                  const Split* solo, int64_t tokens, Split* out) {
-    if (count == 1) {
-        out[0] = solo[0];
-        return;
-    }
-    int64_t kb_max = 1;
-    for (int i = 0; i < count; ++i) kb_max = k_blocks[i] > kb_max ? k_blocks[i] : kb_max;
-    double best_ns = -1.0;
-    for (int64_t kmax = kb_max; kmax >= 1; --kmax) {
-        Split cand[kPrefillBatch];
-        int64_t wgs = 0, steps = 0, partial_elems = 0;
-        for (int i = 0; i < count; ++i) {
-            const int64_t most_k = k_blocks[i] / kMinSliceBlocks > 1 ? k_blocks[i] / kMinSliceBlocks : 1;
-            const int64_t most_cap = cap[i] / (tokens * n[i]) > 1 ? cap[i] / (tokens * n[i]) : 1;
-            int64_t sl = (k_blocks[i] + kmax - 1) / kmax;
-            sl = sl < most_k ? sl : most_k;
-            sl = sl < most_cap ? sl : most_cap;
-            cand[i].k_per_split = (k_blocks[i] + sl - 1) / sl;
-            cand[i].slices = (k_blocks[i] + cand[i].k_per_split - 1) / cand[i].k_per_split;
-            wgs += tiles[i] * cand[i].slices;
-            steps = cand[i].k_per_split > steps ? cand[i].k_per_split : steps;
-            if (cand[i].slices > 1) partial_elems += cand[i].slices * tokens * n[i];
-        }
-        const int64_t rounds = (wgs + resident_for(tokens) - 1) / resident_for(tokens);
-        double ns = static_cast<double>(rounds * (steps + 1)) * step_ns_for(tokens);
-        if (partial_elems > 0)
-            ns += reduce_ns_for(tokens) + 2.0 * static_cast<double>(partial_elems * 4) / kPartialBytesPerNs;
-        if (best_ns < 0.0 || ns < best_ns) {
-            best_ns = ns;
-            for (int i = 0; i < count; ++i) out[i] = cand[i];
-        }
+template <int P>
+void launch_gemm(int shape, dim3 grid, hipStream_t stream, const GemmBatch& gb) {
+    switch (shape) {
+        case kShape32x128: hipLaunchKernelGGL((k_sign_gemm<1, 1, 1, P>), grid, dim3(kBlock), 0, stream, gb); break;
+        case kShape64x128: hipLaunchKernelGGL((k_sign_gemm<1, 2, 1, P>), grid, dim3(kBlock), 0, stream, gb); break;
+        case kShape64x256:
+            if constexpr (P == kPlanesSplit) hipLaunchKernelGGL((k_sign_gemm<1, 2, 2, P>), grid, dim3(kBlock), 0, stream, gb);
+            break;
+        case kShape128x128:
+            if constexpr (P == kPlanes) hipLaunchKernelGGL((k_sign_gemm<2, 2, 2, P>), grid, dim3(kBlock), 0, stream, gb);
+            break;
+        case kFew32:
+            hipLaunchKernelGGL((k_sign_gemm_few<1, P>), grid, dim3(kFewWaves * 64), 0, stream, gb);
+            break;
+        case kFew64:
+            if constexpr (P == kPlanes)
+                hipLaunchKernelGGL((k_sign_gemm_few<2, P>), grid, dim3(kFewWaves * 64), 0, stream, gb);
+            break;
+        default:
+            if constexpr (P == kPlanes) hipLaunchKernelGGL((k_sign_gemm<2, 2, 4, P>), grid, dim3(kBlock), 0, stream, gb);
+            break;
     }
 }
 
-// One launch of a phase's GEMMs (p[i].splits, k_per_split and partial set)
-// and, when any member's K is split, one launch of the reductions. Up to 64
-// tokens take the 64 x 128 block tile; otherwise the 128 x 256 block tile is
-// used when it is the cheaper of the two by the round model below (K slices
-// count as blocks of their own), and 128 x 128 when not.
-constexpr double kWideStepCost = 1.65;
-void launch_phase(GemmArgs* p, int count, int64_t tokens, hipStream_t stream) {
-    const int64_t mt = (tokens + kBM - 1) / kBM;
-    const bool small = tokens <= kBM / 2;  // one 64-row block holds every token
-    bool wide = !small;
-    int64_t wide_blocks = 0, narrow_blocks = 0, steps = 0;
-    for (int i = 0; i < count; ++i) {
-        wide_blocks += mt * ((p[i].n + 2 * kBN - 1) / (2 * kBN)) * p[i].splits;
-        narrow_blocks += mt * ((p[i].n + kBN - 1) / kBN) * p[i].splits;
-        steps = p[i].k_per_split > steps ? p[i].k_per_split : steps;
-    }
-    // Rounds of resident workgroups times K steps, a 128 x 256 step costing
-    // kWideStepCost 128 x 128 steps (measured: twice the MFMAs at 1.65x the time).
-    const double narrow_cost = static_cast<double>(((narrow_blocks + kResident - 1) / kResident) * (steps + 1));
-    const double wide_cost =
-        kWideStepCost * static_cast<double>(((wide_blocks + kResident - 1) / kResident) * (steps + 1));
-    wide = wide && wide_cost < narrow_cost;
-    const int64_t bn = wide ? 2 * kBN : kBN;
+// One launch of a phase's GEMMs and, when any member's K is split, one launch
+// of the reductions.
+template <int P>
+void launch_phase(GemmArgs* p, const Plan& plan, int count, int64_t tokens, hipStream_t stream) {
+    const bool few = plan.shape >= kShapes;
+    const int64_t rows = few ? (plan.shape == kFew32 ? 32 : 64) : kShape[plan.shape].rows;
     GemmBatch gb;
     GemmBatch rb;
     int64_t x = 0, rx = 0;
+    const bool mid = p[0].mid.planes != nullptr;
     for (int i = 0; i < kPrefillBatch; ++i) {
         if (i >= count) {
             gb.begin[i] = rb.begin[i] = INT32_MAX;
             gb.p[i] = rb.p[i] = GemmArgs{};
             continue;
         }
-        p[i].col_blocks = (p[i].n + bn - 1) / bn;
+        p[i].k_per_split = plan.k_per_split[i];
+        p[i].splits = plan.slices[i];
+        if (p[i].splits == 1) p[i].partial = nullptr;
+        const int64_t cols = few ? 32 : kShape[plan.shape].cols;
+        p[i].col_blocks = few && mid ? 4 * p[i].mid_blocks : (p[i].n + cols - 1) / cols;
         gb.begin[i] = static_cast<int32_t>(x);
         rb.begin[i] = static_cast<int32_t>(rx);
         gb.p[i] = rb.p[i] = p[i];
         x += p[i].col_blocks * p[i].splits;
-        if (p[i].splits > 1) {
-            const int64_t width = p[i].out_scale ? p[i].out_ld : p[i].n;
-            rx += (width + kBlock - 1) / kBlock;
-        }
+        if (p[i].splits > 1) rx += mid ? p[i].mid_blocks : (p[i].n + kBlock - 1) / kBlock;
     }
-    const dim3 grid(static_cast<unsigned>(x), static_cast<unsigned>(mt));
-    const bool split = p[0].split != 0;  // every member of a batch agrees (launch_prefill_batch)
-    if (small && split)
-        hipLaunchKernelGGL((k_sign_gemm<1, 2, 1, true>), grid, dim3(kBlock), 0, stream, gb);
-    else if (small)
-        hipLaunchKernelGGL((k_sign_gemm<1, 2, 1, false>), grid, dim3(kBlock), 0, stream, gb);
-    else if (wide && split)
-        hipLaunchKernelGGL((k_sign_gemm<1, 4, 2, true>), grid, dim3(kBlock), 0, stream, gb);
-    else if (wide)
-        hipLaunchKernelGGL((k_sign_gemm<1, 4, 2, false>), grid, dim3(kBlock), 0, stream, gb);
-    else if (split)
-        hipLaunchKernelGGL((k_sign_gemm<2, 2, 2, true>), grid, dim3(kBlock), 0, stream, gb);
+    const auto grid_of = [](int64_t cols, int64_t rows) {
+        return dim3(static_cast<unsigned>(cols), static_cast<unsigned>(rows < kRowsPerGridZ ? rows : kRowsPerGridZ),
+                    static_cast<unsigned>((rows + kRowsPerGridZ - 1) / kRowsPerGridZ));
+    };
+    launch_gemm<P>(plan.shape, grid_of(x, (tokens + rows - 1) / rows), stream, gb);
+    if (rx == 0) return;
+    const dim3 grid = grid_of(rx, mid ? (tokens + 15) / 16 : tokens);
+    if (mid)
+        hipLaunchKernelGGL(k_reduce_mid<P>, grid, dim3(kBlock), 0, stream, rb);
     else
-        hipLaunchKernelGGL((k_sign_gemm<2, 2, 2, false>), grid, dim3(kBlock), 0, stream, gb);
-    if (rx > 0) {
-        const dim3 rgrid(static_cast<unsigned>(rx), static_cast<unsigned>(tokens < kRowsPerGridZ ? tokens : kRowsPerGridZ),
-                         static_cast<unsigned>((tokens + kRowsPerGridZ - 1) / kRowsPerGridZ));
-        hipLaunchKernelGGL(k_reduce_splits, rgrid, dim3(kBlock), 0, stream, rb);
-    }
+        hipLaunchKernelGGL(k_reduce_splits, grid, dim3(kBlock), 0, stream, rb);
+}
+
+int planes_of(const nq_linear_desc* d) {
+    return d->prefill_operands == NQ_PREFILL_FP16_SPLIT ? kPlanesSplit : kPlanes;
 }
 
 struct Scratch {
-    int64_t xs16, scale1, lm16, scale2, partial, total;
+    int64_t planes1, exps1, planes2, exps2, partial, total;
     int64_t partial_elems;  // fp32 elements of the partial buffer
-    Split s1, s2;
 };
+
+// Workspace sizes are those of 16-bit operands (two per value when split),
+// their rows' scales and partials for a split of 128 x 128 blocks (64-row up to
+// 64 tokens) by a latency model of K steps of 1 us (0.5), 512 resident
+// workgroups (1024), a reduction of 6 us (3) and 8 TB/s: callers size buffers
+// and nq_linear_static takes or refuses calls by them. The planes come out of
+// the same bytes; what they leave holds the partials.
+int64_t reserved_slices(int64_t tokens, int64_t k_blocks, int64_t n) {
+    const bool small = tokens <= 64;
+    const int64_t tiles = (tokens + 127) / 128 * ((n + 127) / 128);
+    int64_t best = 1;
+    double best_ns = -1.0;
+    const int64_t most = k_blocks / 2 > 1 ? k_blocks / 2 : 1;
+    for (int64_t want = 1; want <= most; ++want) {
+        const int64_t per = (k_blocks + want - 1) / want, slices = (k_blocks + per - 1) / per;
+        const int64_t resident = small ? 1024 : 512;
+        const int64_t rounds = (tiles * slices + resident - 1) / resident;
+        double ns = static_cast<double>(rounds * (per + 1)) * (small ? 500.0 : 1000.0);
+        if (slices > 1) ns += (small ? 3000.0 : 6000.0) + 2.0 * static_cast<double>(slices * tokens * n * 4) / 8000.0;
+        if (best_ns < 0.0 || ns < best_ns) best = slices, best_ns = ns;
+    }
+    return best;
+}
 
 Scratch scratch_layout(const nq_linear_desc* d, int64_t tokens) {
     const Geometry g = geometry(d);
-    const int64_t mt = (tokens + kBM - 1) / kBM;
+    const int64_t groups = (tokens + kRows - 1) / kRows, bytes = 2 * planes_of(d) * kPlaneBytes;
     Scratch s{};
-    s.s1 = split_for(mt * ((d->rank + kBN - 1) / kBN), g.nsc1, tokens, d->rank);
-    s.s2 = split_for(mt * ((d->out_features + kBN - 1) / kBN), g.nsc2, tokens, d->out_features);
-    const int64_t planes = d->prefill_operands == NQ_PREFILL_FP16_SPLIT ? 2 : 1;
-    s.xs16 = 0;
-    s.scale1 = s.xs16 + a256(tokens * g.nsc1 * kBK * 2 * planes);
-    s.lm16 = s.scale1 + a256(tokens * 4);
-    s.scale2 = s.lm16 + a256(tokens * g.nsc2 * kBK * 2 * planes);
-    s.partial = s.scale2 + a256(tokens * 4);
-    const int64_t p1 = s.s1.slices > 1 ? s.s1.slices * tokens * d->rank : 0;
-    const int64_t p2 = s.s2.slices > 1 ? s.s2.slices * tokens * d->out_features : 0;
-    s.partial_elems = p1 > p2 ? p1 : p2;
-    s.total = s.partial + a256(4 * s.partial_elems);
+    s.planes1 = 0;
+    s.exps1 = s.planes1 + a256(g.nsc1 * groups * bytes);
+    s.planes2 = s.exps1 + a256(g.nsc1 * groups * 128);
+    s.exps2 = s.planes2 + a256(g.nsc2 * groups * bytes);
+    s.partial = s.exps2 + a256(g.nsc2 * groups * 128);
+    const int64_t reserved = nq::prefill_reserved_bytes(d, tokens);
+    s.total = s.partial > reserved ? s.partial : reserved;
+    s.partial_elems = (s.total - s.partial) / 4;
     return s;
 }
 
@@ -1044,133 +1264,116 @@ Scratch scratch_layout(const nq_linear_desc* d, int64_t tokens) {
 
 namespace nq {
 
+int64_t prefill_reserved_bytes(const nq_linear_desc* d, int64_t tokens) {
+    if (!d->tiles) return a256(tokens * d->rank * 4);
+    const Geometry g = geometry(d);
+    const int64_t parts = d->prefill_operands == NQ_PREFILL_FP16_SPLIT ? 2 : 1;
+    const int64_t s1 = reserved_slices(tokens, g.nsc1, d->rank), s2 = reserved_slices(tokens, g.nsc2, d->out_features);
+    const int64_t p1 = s1 > 1 ? s1 * tokens * d->rank : 0, p2 = s2 > 1 ? s2 * tokens * d->out_features : 0;
+    return a256(tokens * d->rank * 4) + a256(tokens * g.nsc1 * kBK * 2 * parts) +
+           a256(tokens * g.nsc2 * kBK * 2 * parts) + 2 * a256(tokens * 4) + a256(4 * (p1 > p2 ? p1 : p2));
+}
+
 int64_t prefill_scratch_bytes(const nq_linear_desc* d, int64_t tokens) {
-    if (!d->tiles) return 0;
-    return scratch_layout(d, tokens).total;
+    return d->tiles ? scratch_layout(d, tokens).total : prefill_reserved_bytes(d, tokens);
 }
 
 bool prefill_path_applies(const nq_linear_desc* d, int64_t tokens) {
-    return d->tiles != nullptr && tokens > 16 && tokens <= 65535 * int64_t(kBM);
+    return d->tiles != nullptr && tokens > 16 && tokens <= 65535 * int64_t(128);
 }
 
-int launch_prefill_batch(const nq_linear_desc* const* descs, int count, const void* const* xs, int x_dtype,
-                         int64_t tokens, void* const* ys, int y_dtype, void* const* scratch, hipStream_t stream) {
-    if (count < 1 || count > kPrefillBatch) return NQ_ERR_SHAPE;
-    const int64_t header_words = tiles_header_words();
+}  // namespace nq
+
+namespace {
+
+template <int P>
+int launch_prefill_planes(const nq_linear_desc* const* descs, int count, const void* const* xs, int x_dtype,
+                          int64_t tokens, void* const* ys, int y_dtype, void* const* scratch, hipStream_t stream) {
+    const int64_t header_words = nq::tiles_header_words();
     auto aligned = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
     Geometry geo[kPrefillBatch];
     Scratch sl[kPrefillBatch];
+    Operand mid[kPrefillBatch];
     PrepBatch pb{};
     bool all_vec = true;
-    int64_t pad_max = 0;
-    const int split = descs[0]->prefill_operands == NQ_PREFILL_FP16_SPLIT ? 1 : 0;
+    int64_t nkb_max = 0;
     for (int i = 0; i < count; ++i) {
         const nq_linear_desc* d = descs[i];
         geo[i] = geometry(d);
         if (d->tiles_bytes < (header_words + geo[i].v_words + geo[i].u_words) * 4) return NQ_ERR_ARGUMENT;
         if (d->prefill_operands != descs[0]->prefill_operands) return NQ_ERR_ARGUMENT;
-        // The GEMMs read the fp16 staging buffers with 16-byte vector loads.
+        // The planes and partials are written and read by 16-byte accesses.
         if (!aligned(scratch[i], 16)) return NQ_ERR_ALIGNMENT;
         sl[i] = scratch_layout(d, tokens);
-        char* ws = static_cast<char*>(scratch[i]);
+        uint8_t* ws = static_cast<uint8_t*>(scratch[i]);
+        const int64_t groups = (tokens + kRows - 1) / kRows;
         PrepArgs& pa = pb.p[i];
         pa.act = xs[i];
-        pa.ld = d->in_features;
+        pa.act_dtype = x_dtype;
         pa.colscale = d->scale_pre;
         pa.colscale_dtype = d->scale_dtype;
-        // Vector row loads: 8 elements per load, 16-byte aligned rows.
-        pa.vec = (d->in_features % 8 == 0 && aligned(xs[i], 16) && aligned(d->scale_pre, 16)) ? 1 : 0;
+        pa.tokens = tokens;
         pa.cols = d->in_features;
-        pa.cols_pad = geo[i].nsc1 * kBK;
-        pa.out16 = reinterpret_cast<_Float16*>(ws + sl[i].xs16);
-        pa.split = split;
-        pa.scale_out = reinterpret_cast<float*>(ws + sl[i].scale1);
-        pa.max_mid_bits = static_cast<const uint32_t*>(d->tiles) + tiles_max_mid_word();
-        pa.bound_scale_out = reinterpret_cast<float*>(ws + sl[i].scale2);
-        all_vec = all_vec && pa.vec && d->scale_dtype == descs[0]->scale_dtype;
-        pad_max = pa.cols_pad > pad_max ? pa.cols_pad : pad_max;
+        pa.nkb = geo[i].nsc1;
+        pa.out = Operand{ws + sl[i].planes1, ws + sl[i].exps1, groups};
+        mid[i] = Operand{ws + sl[i].planes2, ws + sl[i].exps2, groups};
+        all_vec = all_vec && d->in_features % 4 == 0 && aligned(xs[i], 16) && aligned(d->scale_pre, 16) &&
+                  d->scale_dtype == descs[0]->scale_dtype;
+        nkb_max = pa.nkb > nkb_max ? pa.nkb : nkb_max;
     }
 
-    // Row passes: one launch, grid (tokens, members).
-    const dim3 rows(static_cast<unsigned>(tokens), static_cast<unsigned>(count));
+    // Row passes: one launch.
+    const dim3 rows(static_cast<unsigned>((tokens + 15) / 16), static_cast<unsigned>((nkb_max + 3) / 4),
+                    static_cast<unsigned>(count));
+    const int sdt = descs[0]->scale_dtype;
     bool prepped = false;
-    if (all_vec && pad_max <= int64_t(kPrepChunksMax) * 8 * kBlock) {
-        const bool short_rows = pad_max <= 2 * 8 * kBlock;
-        const int sdt = descs[0]->scale_dtype;
-#define NQ_PREP(ADT, SDT)                                                                                      \
-    if (x_dtype == ADT && sdt == SDT) {                                                                        \
-        if (short_rows)                                                                                        \
-            hipLaunchKernelGGL((k_prep_rows_vec<ADT, SDT, 2>), rows, dim3(kBlock), 0, stream, pb);              \
-        else                                                                                                   \
-            hipLaunchKernelGGL((k_prep_rows_vec<ADT, SDT, kPrepChunksMax>), rows, dim3(kBlock), 0, stream, pb); \
-        prepped = true;                                                                                        \
+#define NQ_PREP(ADT, SDT)                                                                                  \
+    if (all_vec && x_dtype == ADT && sdt == SDT) {                                                         \
+        hipLaunchKernelGGL((k_prep_rows<ADT, SDT, P, true>), rows, dim3(kBlock), 0, stream, pb);            \
+        prepped = true;                                                                                    \
     }
 #define NQ_PREP_S(ADT) NQ_PREP(ADT, NQ_DTYPE_F16) NQ_PREP(ADT, NQ_DTYPE_BF16) NQ_PREP(ADT, NQ_DTYPE_F32)
-        NQ_PREP_S(NQ_DTYPE_BF16) NQ_PREP_S(NQ_DTYPE_F16) NQ_PREP_S(NQ_DTYPE_F32)
+    NQ_PREP_S(NQ_DTYPE_BF16) NQ_PREP_S(NQ_DTYPE_F16) NQ_PREP_S(NQ_DTYPE_F32)
 #undef NQ_PREP_S
 #undef NQ_PREP
-    }
-    if (!prepped) hipLaunchKernelGGL(k_prep_rows, rows, dim3(kBlock), 0, stream, pb, x_dtype);
+    if (!prepped) hipLaunchKernelGGL((k_prep_rows<0, 0, P, false>), rows, dim3(kBlock), 0, stream, pb);
 
-    const int64_t mt = (tokens + kBM - 1) / kBM;
-    int64_t tiles[kPrefillBatch], kb[kPrefillBatch], n[kPrefillBatch], cap[kPrefillBatch];
-    Split solo[kPrefillBatch], sp[kPrefillBatch];
+    int64_t kb[kPrefillBatch], n[kPrefillBatch], cap[kPrefillBatch];
     GemmArgs g[kPrefillBatch];
 
-    // GEMM 1: lm16 = fp16 rank intermediate, scaled per row by scale2.
-    for (int i = 0; i < count; ++i) {
-        tiles[i] = mt * ((descs[i]->rank + kBN - 1) / kBN);
-        kb[i] = geo[i].nsc1;
-        n[i] = descs[i]->rank;
-        cap[i] = sl[i].partial_elems;
-        solo[i] = sl[i].s1;
-    }
-    batch_splits(count, tiles, kb, n, cap, solo, tokens, sp);
+    // GEMM 1: the rank intermediate.
     for (int i = 0; i < count; ++i) {
         const nq_linear_desc* d = descs[i];
-        char* ws = static_cast<char*>(scratch[i]);
+        kb[i] = geo[i].nsc1;
+        n[i] = d->rank;
+        cap[i] = sl[i].partial_elems;
         GemmArgs& a = g[i];
         a = GemmArgs{};
-        a.a = pb.p[i].out16;
+        a.a = pb.p[i].out;
         a.m = tokens;
-        a.kpad = geo[i].nsc1 * kBK;
         a.tiles = static_cast<const uint32_t*>(d->tiles) + header_words;
         a.n = d->rank;
         a.nb = geo[i].nsc1;
-        a.row_scale = pb.p[i].scale_out;
         a.col_scale = d->scale_mid;
         a.col_scale_dtype = d->scale_dtype;
-        a.out = ws + sl[i].lm16;
-        a.out_dtype = NQ_DTYPE_F16;
-        a.out_scale = pb.p[i].bound_scale_out;
-        a.out_ld = geo[i].nsc2 * kBK;  // GEMM 1's column blocks cover exactly this width
-        a.split = split;
-        a.k_per_split = sp[i].k_per_split;
-        a.splits = sp[i].slices;
-        a.partial = sp[i].slices > 1 ? reinterpret_cast<float*>(ws + sl[i].partial) : nullptr;
+        a.mid = mid[i];
+        a.mid_blocks = geo[i].nsc2;
+        a.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(scratch[i]) + sl[i].partial);
     }
-    launch_phase(g, count, tokens, stream);
+    launch_phase<P>(g, plan_phase(count, kb, n, cap, tokens, P), count, tokens, stream);
 
-    // GEMM 2: y = s_out * (lm16 · U±1ᵀ) / scale2 + salient columns + bias.
-    for (int i = 0; i < count; ++i) {
-        tiles[i] = mt * ((descs[i]->out_features + kBN - 1) / kBN);
-        kb[i] = geo[i].nsc2;
-        n[i] = descs[i]->out_features;
-        solo[i] = sl[i].s2;
-    }
-    batch_splits(count, tiles, kb, n, cap, solo, tokens, sp);
+    // GEMM 2: y = s_out * (lm · U±1ᵀ) + salient columns + bias.
     for (int i = 0; i < count; ++i) {
         const nq_linear_desc* d = descs[i];
-        char* ws = static_cast<char*>(scratch[i]);
+        kb[i] = geo[i].nsc2;
+        n[i] = d->out_features;
         GemmArgs& a = g[i];
         a = GemmArgs{};
-        a.a = reinterpret_cast<const _Float16*>(ws + sl[i].lm16);
+        a.a = mid[i];
         a.m = tokens;
-        a.kpad = geo[i].nsc2 * kBK;
         a.tiles = static_cast<const uint32_t*>(d->tiles) + header_words + geo[i].v_words;
         a.n = d->out_features;
         a.nb = geo[i].nsc2;
-        a.row_scale = pb.p[i].bound_scale_out;
         a.col_scale = d->scale_post;
         a.col_scale_dtype = d->scale_dtype;
         a.x = xs[i];
@@ -1186,13 +1389,22 @@ int launch_prefill_batch(const nq_linear_desc* const* descs, int count, const vo
         a.bias_dtype = d->bias_dtype;
         a.out = ys[i];
         a.out_dtype = y_dtype;
-        a.split = split;
-        a.k_per_split = sp[i].k_per_split;
-        a.splits = sp[i].slices;
-        a.partial = sp[i].slices > 1 ? reinterpret_cast<float*>(ws + sl[i].partial) : nullptr;
+        a.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(scratch[i]) + sl[i].partial);
     }
-    launch_phase(g, count, tokens, stream);
-    return launch_status();
+    launch_phase<P>(g, plan_phase(count, kb, n, cap, tokens, P), count, tokens, stream);
+    return nq::launch_status();
+}
+
+}  // namespace
+
+namespace nq {
+
+int launch_prefill_batch(const nq_linear_desc* const* descs, int count, const void* const* xs, int x_dtype,
+                         int64_t tokens, void* const* ys, int y_dtype, void* const* scratch, hipStream_t stream) {
+    if (count < 1 || count > kPrefillBatch) return NQ_ERR_SHAPE;
+    if (descs[0]->prefill_operands == NQ_PREFILL_FP16_SPLIT)
+        return launch_prefill_planes<kPlanesSplit>(descs, count, xs, x_dtype, tokens, ys, y_dtype, scratch, stream);
+    return launch_prefill_planes<kPlanes>(descs, count, xs, x_dtype, tokens, ys, y_dtype, scratch, stream);
 }
 
 int launch_prefill(const nq_linear_desc* d, const void* x, int x_dtype, int64_t tokens, void* y, int y_dtype,

@@ -9,11 +9,14 @@
 // ordering) race on it and must not be issued.
 #include <mutex>
 
-#include "nq_common.h"
+#include "nq_prefill.h"
 
 namespace {
 
-static __device__ __align__(256) uint8_t scratch[NQ_STATIC_SCRATCH_BYTES];
+// Prefill calls are taken or refused by their reserved bytes, which their
+// planes of a few tokens (whole groups of 32 rows) can exceed.
+constexpr int64_t kArrayBytes = int64_t(NQ_STATIC_SCRATCH_BYTES) * nq::kPrefillOverReserve;
+static __device__ __align__(256) uint8_t scratch[kArrayBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_lock;
@@ -45,7 +48,7 @@ int scratch_address(void** out) {
 
 extern "C" int nq_linear_static(const nq_linear_desc* desc, const void* x, int32_t x_dtype, int64_t tokens,
                                 void* y, int32_t y_dtype, void* stream) {
-    const int64_t need = nq_linear_workspace_bytes(desc, tokens);
+    const int64_t need = nq::linear_reserved_bytes(desc, tokens);
     if (need < 0) {
         // The same validation nq_linear runs, for its status code.
         return nq_linear(desc, x, x_dtype, tokens, y, y_dtype, nullptr, 0, stream);
@@ -54,5 +57,5 @@ extern "C" int nq_linear_static(const nq_linear_desc* desc, const void* x, int32
     void* ws = nullptr;
     const int st = scratch_address(&ws);
     if (st != NQ_OK) return st;
-    return nq_linear(desc, x, x_dtype, tokens, y, y_dtype, ws, NQ_STATIC_SCRATCH_BYTES, stream);
+    return nq_linear(desc, x, x_dtype, tokens, y, y_dtype, ws, kArrayBytes, stream);
 }

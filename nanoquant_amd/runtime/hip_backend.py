@@ -150,11 +150,11 @@ class HipPackedBackend:
         kernels); without it every call takes the canonical-word fp32 path.
         ``decode_launch``: ``"split"`` runs the two decode stages as two
         kernels, ``"fused"`` as one kernel with an in-kernel grid handoff.
-        ``prefill_operands`` (above 16 tokens): ``"fp16"`` rounds the prefill
-        GEMMs' activations and rank intermediate to fp16 (about 3e-4 rel-L2
-        per linear); ``"split"`` carries each as an fp16 value plus an fp16
-        remainder (about 1e-6), at twice the MFMA work, for callers whose
-        errors compound through many layers."""
+        ``prefill_operands`` (above 16 tokens): ``"fp16"`` carries the
+        prefill GEMMs' activations and rank intermediate in three 6-bit planes
+        (about 6e-5 rel-L2 per linear, within what fp16 operands have);
+        ``"split"`` in five (about 1e-7), for callers whose errors compound
+        through many layers."""
 
         if decode_launch not in _DECODE_LAUNCH:
             raise ValueError(f"decode_launch must be one of {sorted(_DECODE_LAUNCH)}")

@@ -345,6 +345,71 @@ def test_prefill_ragged_geometries(tokens, geometry):
     _check_shape(backend, state, tokens, seed=tokens)
 
 
+def _exact_linear(state, x):
+    """The layer's output in 64 bits, from its words and scales."""
+
+    def signs(words, cols):
+        bits = (words[:, :, None] >> torch.arange(32, dtype=torch.int32)) & 1
+        return 1.0 - 2.0 * bits.reshape(words.shape[0], -1)[:, :cols].double()
+
+    spec, x = state.spec, x.double()
+    mid = (x * state.scale_pre.double()) @ signs(state.right_words, spec.in_features).t() * state.scale_mid.double()
+    y = mid @ signs(state.left_words, spec.rank).t() * state.scale_post.double()
+    return y if state.bias is None else y + state.bias.double()
+
+
+@pytest.mark.parametrize("operands,bar", [("fp16", 1e-4), ("split", 5e-7)])
+@pytest.mark.parametrize(
+    "tokens,geometry",
+    [
+        # few sign rows, 32 and 64 tokens a block: edges of row groups, K chunks and exponent groups
+        (17, (35, 17, 33)), (32, (128, 128, 128)), (33, (516, 65, 130)), (64, (640, 257, 96)), (65, (1152, 900, 513)),
+        # one wave group without a chunk; more chunks than waves
+        (20, (100, 40, 4100)), (31, (4100, 96, 200)),
+        # split K over ragged columns (rank % 4 = 1), and its direct neighbour
+        (40, (8192, 130, 301)), (61, (6200, 4096, 1021)), (24, (6200, 9000, 1021)),
+        # 32-, 64- and 128-row blocks in LDS, rows past the last token
+        (127, (900, 9100, 700)), (257, (1300, 6000, 1030)), (513, (2052, 3000, 1500)), (1025, (700, 5000, 3000)),
+    ],
+)
+def test_prefill_planes_edges(tokens, geometry, operands, bar):
+    """Every form of the prefill GEMMs against 64 bits. Three planes leave at
+    most 2^-14 of a 32-column group's largest value, 4.4e-5 rel-L2 on normal
+    rows and sqrt(2) of it over both GEMMs; five planes keep fp32's 24 bits
+    (3e-8), and fp32 sums of up to 8192 terms add to that. A second call on the
+    same input gives the same bits."""
+
+    in_f, out_f, rank = geometry
+    backend = HipPackedBackend(prefill_operands=operands)
+    _say("prefill planes", tokens, geometry, operands)
+    shape = syn.LinearShape("blocks.0.mlp.gate_proj", in_f, out_f, rank)
+    state = syn.synthetic_packed_layer(shape, seed=tokens + sum(geometry), bias=True)
+    x = syn.synthetic_activations(tokens, in_f, seed=tokens).float()
+    x *= 1.0 + torch.rand(x.shape, generator=torch.Generator().manual_seed(1)) / 3  # all 24 bits in use
+    layer = backend.prepare(state, "cuda")
+    y = backend.linear(x.cuda(), layer)
+    expected = _exact_linear(state, x)
+    err = float((y.cpu().double() - expected).norm() / expected.norm())
+    print(f"  rel_l2={err:.2e}", flush=True)
+    assert err <= bar
+    assert torch.equal(backend.linear(x.cuda(), layer), y)
+
+
+def test_prefill_planes_with_an_outlier_channel():
+    """One channel a thousand times the others: its group's other values keep
+    2^-14 of it, at most sqrt(31) 2^-14 = 3.4e-4 of the channel's own share of
+    the output (fp16 operands round that share itself by 2^-11)."""
+
+    shape = syn.LinearShape("blocks.0.mlp.gate_proj", 1024, 600, 700)
+    state = syn.synthetic_packed_layer(shape, seed=5)
+    x = syn.synthetic_activations(48, 1024, seed=6).float()
+    x[:, 77] = 1000.0 * torch.sign(x[:, 77])
+    backend = HipPackedBackend()
+    y = backend.linear(x.cuda(), backend.prepare(state, "cuda"))
+    expected = _exact_linear(state, x)
+    assert float((y.cpu().double() - expected).norm() / expected.norm()) <= 3.4e-4
+
+
 @pytest.mark.parametrize("geometry", [(1024, 64, 8000, 2), (512, 7990, 300, 0)])
 def test_prefill_wide_blocks(geometry):
     """GEMMs that take the 128 x 256 block tile at M = 2048 (512 such blocks:
