@@ -2,6 +2,7 @@
 // logic. The kernels and the tile layout are documented in
 // nq_decode_kernels.h.
 #include "nq_decode_kernels.h"
+#include "nq_decode_planes.h"
 
 namespace nqdec {
 namespace {
@@ -170,16 +171,13 @@ void pick_waves(int64_t nc, int tpb, int tb, int& nw, int& kc) {
 }
 
 // The same for the several-token stages of the split launch: at most eight
-// waves, two per chunk slot with four token blocks (blocks_per_wave); with one
-// token block two chunks per wave per pass when the slots would not cover the
-// chunks (a wave holding two blocks has no registers for a second chunk).
+// waves; with one token block two chunks per wave per pass when the waves
+// would not cover the chunks (a wave holding two blocks has no registers for a
+// second chunk).
 void pick_waves_multi(int64_t nc, int tb, int& nw, int& kc) {
-    const int ng = tb > 2 ? 2 : 1;
-    const int64_t max_slots = 8 / ng;
-    kc = nc > max_slots && tb == 1 ? 2 : 1;
-    int64_t slots = (nc + kc - 1) / kc;
-    if (slots > max_slots) slots = max_slots;
-    nw = static_cast<int>(slots) * ng;
+    kc = nc > 8 && tb == 1 ? 2 : 1;
+    const int64_t waves = (nc + kc - 1) / kc;
+    nw = static_cast<int>(waves < 8 ? waves : 8);
 }
 
 // Dynamic LDS of a stage: per-wave operand areas (stage 1), the partial sums
@@ -225,12 +223,20 @@ int pick_tiles(int stage, int64_t tiles, int nw, int kc, int tb, bool fused) {
 constexpr int64_t kStage0Tokens = 5;
 bool stage0_path(int64_t tokens) { return tokens >= kStage0Tokens; }
 
+// Tokens from which both launches take the fp6 planes (nq_decode_planes.hip):
+// with three or four blocks of four tokens the int8 digits are 64 bytes a
+// column against 48 for all sixteen rows, and a plane's MFMA covers them at
+// once. Measured at 5 and 16 tokens (us a call, digits against planes): 4096 ->
+// 4096 r1638 15.3 / 15.4 and 29.0 / 15.8, 4096 -> 2 x 12288 r3072 20.6 / 19.8
+// and 29.7 / 20.9; at 8, 10240 -> 2560 r1536 17.5 / 22.0.
+constexpr int64_t kPlanesTokens = 9;
+bool planes_path(int64_t tokens) { return tokens >= kPlanesTokens; }
+
 // Tiles per workgroup of the several-token stages: a wave's A operands (8 KB
 // per block of four tokens per chunk) are shared by its TW tiles, against
 // fewer waves. One token block (stage 2 after the in-kernel staging): four
-// tiles from 4096 waves, two from 2048. Two or four blocks (stage 0 path):
-// two tiles in both stages (measured best against one and four, per stage,
-// at 8 and 16 tokens).
+// tiles from 4096 waves, two from 2048. Two blocks (stage 0 path): two tiles in
+// both stages (measured best against one and four, per stage, at 8 tokens).
 int pick_tiles_multi(int64_t tiles, int nw, int tb) {
     if (tb > 1) return 2;
     const int64_t waves = tiles * nw;
@@ -339,8 +345,8 @@ int plan_shapes(HostBatch& batch, int64_t tokens, int ak, bool fused, Shapes& sh
     }
     LaunchShape s1{}, s2{};
     s1.tpb = s2.tpb = tokens == 1 ? 1 : 4;
-    // Blocks of four tokens: 1, 2 or 4 in the split launch, 1 or 4 fused.
-    s1.tb = s2.tb = tokens <= 4 ? 1 : (tokens <= 8 && !fused && stage0_path(tokens) ? 2 : 4);
+    // Blocks of four tokens: 1 or 2 in the split launch, 1 or 4 fused.
+    s1.tb = s2.tb = tokens <= 4 ? 1 : (fused ? 4 : 2);
     s1.ak = s2.ak = ak;
     if (fused) {
         // The fused kernel keeps both stages' registers live: blocks of four
@@ -515,6 +521,8 @@ int launch_decode_batch(const nq_linear_desc* const* descs, int count, const voi
             }
         }
     }
+    if (planes_path(tokens))
+        return launch_decode_planes(descs, count, xs, x_dtype, tokens, ys, y_dtype, scratch, stream);
     return launch_batch(batch, tokens, ak, descs[0]->decode_launch == NQ_DECODE_FUSED, stream, pair);
 }
 

@@ -72,7 +72,8 @@
 //     boundary is the grid-wide barrier. From five tokens a kernel 0 first
 //     stages x * s_in once per (chunk, token block) and kernel 1 loads those
 //     operands instead of staging them in every workgroup (k_decode_stage0,
-//     k_decode_stage1m below).
+//     k_decode_stage1m below). From nine tokens both launches take the fp6
+//     planes (nq_decode_planes.hip).
 //   fused: one kernel whose first grid rows are the stage-1 workgroups and
 //     the rest the stage-2 workgroups. Stage-1 workgroups store the operands
 //     at agent scope and then signal; stage-2 workgroups issue their U loads,
@@ -1669,26 +1670,14 @@ __device__ __forceinline__ void stage0_wave(const Lin& a, int c, int tb, int tbl
     }
 }
 
-// Token blocks per wave and wave groups per chunk of the several-token
-// kernels: a wave holds the A operands of at most two token blocks (64
-// VGPRs per chunk), so with four blocks two waves share each chunk, wave w
-// taking blocks 2 (w % 2) and 2 (w % 2) + 1 of chunk slot w / 2.
-template <int TB>
-constexpr int blocks_per_wave() { return TB > 2 ? 2 : TB; }
-template <int TB>
-constexpr int wave_groups() { return TB / blocks_per_wave<TB>(); }
-
 // One stage-1 workgroup of the several-token path: tiles [t0, t0 + TW) of
 // linear `a`, operands from xq; TB blocks of four tokens in the layout.
 template <int TB, int TW, int KC>
 __device__ __forceinline__ void stage1m_wg(const Lin& a, int wg_in, char* __restrict__ lds) {
     constexpr int TPB = 4;
-    constexpr int TBW = blocks_per_wave<TB>(), NG = wave_groups<TB>();
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int grp = wave % NG, slot = wave / NG;
     const int nw = a.nw1;
-    const int nslots = nw / NG;
     const int nthreads = nw * 64;
     const int tokens = a.tokens;
     const int nblk = (tokens + TPB - 1) / TPB;
@@ -1709,13 +1698,11 @@ __device__ __forceinline__ void stage1m_wg(const Lin& a, int wg_in, char* __rest
     RawElem rs0;
     float maxsm = 0.0f, xmv = 0.0f;
 
-    // This wave's token blocks are grp * TBW + i, i < gblk.
-    const int gblk0 = nblk - grp * TBW;
-    const int gblk = gblk0 < 0 ? 0 : (gblk0 > TBW ? TBW : gblk0);
+    const int gblk = nblk > TB ? TB : nblk;
     const auto pass = [&](const int base, const bool first) __attribute__((always_inline)) {
-        const PassChunks<KC> pc = pass_chunks<KC>(base, slot, nslots, nc);
-        S2Regs<TBW, TW> r[KC];
-        int e[KC][TBW];
+        const PassChunks<KC> pc = pass_chunks<KC>(base, wave, nw, nc);
+        S2Regs<TB, TW> r[KC];
+        int e[KC][TB];
 #pragma unroll
         for (int j = 0; j < KC; ++j) load_words(r[j].w, a.v_tiles, nt, nb, t0, pc.c[j], lane);
         // Every block of the wave's group is loaded (xq holds TB blocks per
@@ -1723,8 +1710,8 @@ __device__ __forceinline__ void stage1m_wg(const Lin& a, int wg_in, char* __rest
 #pragma unroll
         for (int j = 0; j < KC; ++j)
 #pragma unroll
-            for (int i = 0; i < TBW; ++i) {
-                const int tb = grp * TBW + i;
+            for (int i = 0; i < TB; ++i) {
+                const int tb = i;
 #pragma unroll
                 for (int m = 0; m < 8; ++m)
                     r[j].a[i][m] = *reinterpret_cast<const v4i*>(
@@ -1743,24 +1730,24 @@ __device__ __forceinline__ void stage1m_wg(const Lin& a, int wg_in, char* __rest
             if (!pc.live[j]) continue;  // uniform
             const int c = pc.c[j];
             const int dw = chunk_words32(nb, c);
-            v4i S[TBW];
-            float sc[TBW];
+            v4i S[TB];
+            float sc[TB];
 #pragma unroll
-            for (int i = 0; i < TBW; ++i) {
+            for (int i = 0; i < TB; ++i) {
                 S[i] = ones_mfma(r[j].a[i]);
                 sc[i] = exp2i(-e[j][i] - 7);
             }
 #pragma unroll
             for (int tt = 0; tt < TW; ++tt) {
-                float part[TBW];
-                tile_partials<4, TBW>(r[j].a, S, r[j].w[tt], dw, sc, part);
+                float part[TB];
+                tile_partials<4, TB>(r[j].a, S, r[j].w[tt], dw, sc, part);
 #pragma unroll
-                for (int i = 0; i < TBW; ++i)
-                    if (i < gblk) red[((c * TW + tt) * TB + grp * TBW + i) * 64 + lane] = part[i];
+                for (int i = 0; i < TB; ++i)
+                    if (i < gblk) red[((c * TW + tt) * TB + i) * 64 + lane] = part[i];
             }
         }
     };
-    const int step = nslots * KC;
+    const int step = nw * KC;
     pass(0, true);
     for (int base = step; base < nc; base += step) pass(base, false);
     if (static_cast<int>(threadIdx.x) < nxm) cmx[threadIdx.x] = xmv;
@@ -1833,21 +1820,13 @@ __device__ __forceinline__ float bits_value(uint32_t b, int dtype) {
 template <int TPB, int TB, int TW, int KC, bool FUSED, bool PAIR = false>
 __device__ __forceinline__ void stage2_wg(const Lin& a, int wg_in, char* __restrict__ lds,
                                           const Lin* pair = nullptr) {
-    // Split launch with four token blocks: two waves per chunk slot
-    // (blocks_per_wave); one token or the fused launch: one wave per slot.
-    constexpr int NG = (TPB == 4 && !FUSED) ? wave_groups<TB>() : 1;
-    constexpr int TBW = TB / NG;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int grp = wave % NG, slot = wave / NG;
     const int nw = a.nw2;
-    const int nslots = nw / NG;
     const int nthreads = nw * 64;  // the workgroup size (blockDim.x is a vector load of a hidden argument)
     const int tokens = a.tokens;
     const int nblk = (tokens + TPB - 1) / TPB;
-    // This wave's token blocks are grp * TBW + i, i < gblk.
-    const int gblk0 = nblk - grp * TBW;
-    const int gblk = gblk0 < 0 ? 0 : (gblk0 > TBW ? TBW : gblk0);
+    const int gblk = nblk > TB ? TB : nblk;
     const int nwg = static_cast<int>(a.nwg2);
     const bool dead = wg_in >= nwg;  // computes the last workgroup's tiles, stores nothing
     const int wg = dead ? nwg - 1 : wg_in;
@@ -1887,12 +1866,12 @@ __device__ __forceinline__ void stage2_wg(const Lin& a, int wg_in, char* __restr
     // workgroup issues both members' loads before either waits.
     struct PassRegs {
         PassChunks<KC> pc;
-        S2Regs<TBW, TW> r[KC];
-        int e[TBW];
+        S2Regs<TB, TW> r[KC];
+        int e[TB];
     };
     const auto load_pass = [&](const Lin& m, PassRegs& ps, const int base, const bool first)
                                __attribute__((always_inline)) {
-        ps.pc = pass_chunks<KC>(base, slot, nslots, nc);
+        ps.pc = pass_chunks<KC>(base, wave, nw, nc);
 #pragma unroll
         for (int j = 0; j < KC; ++j) load_words(ps.r[j].w, m.u_tiles, nt, nb, t0, ps.pc.c[j], lane);
         // The U words do not depend on stage 1; the fused launch waits for its
@@ -1909,14 +1888,14 @@ __device__ __forceinline__ void stage2_wg(const Lin& a, int wg_in, char* __restr
 #pragma unroll
             for (int j = 0; j < KC; ++j)
 #pragma unroll
-                for (int i = 0; i < TBW; ++i)
+                for (int i = 0; i < TB; ++i)
 #pragma unroll
                     for (int mm = 0; mm < 8; ++mm)
                         ps.r[j].a[i][mm] = *reinterpret_cast<const v4i*>(
-                            m.lmq + lmq_offset<TPB, TB>(ps.pc.c[j], grp * TBW + i, mm, lane & 15, lane >> 4));
+                            m.lmq + lmq_offset<TPB, TB>(ps.pc.c[j], i, mm, lane & 15, lane >> 4));
 #pragma unroll
-            for (int i = 0; i < TBW; ++i) {
-                const int t = (grp * TBW + i) * TPB + (lane >> 4);
+            for (int i = 0; i < TB; ++i) {
+                const int t = i * TPB + (lane >> 4);
                 ps.e[i] = m.lme[t < tokens ? t : tokens - 1];
             }
         }
@@ -1956,25 +1935,25 @@ __device__ __forceinline__ void stage2_wg(const Lin& a, int wg_in, char* __restr
                 for (int tt = 0; tt < TW; ++tt)
                     redm[(c * TW + tt) * 64 + lane] = tile_partial<4>(ps.r[j].a[0], S, ps.r[j].w[tt], dw, sc);
             } else {
-                v4i S[TBW];
-                float sc[TBW];
+                v4i S[TB];
+                float sc[TB];
 #pragma unroll
-                for (int i = 0; i < TBW; ++i) {
+                for (int i = 0; i < TB; ++i) {
                     S[i] = ones_mfma(ps.r[j].a[i]);
                     sc[i] = ps.e[i] == kPoisonExp ? __builtin_nanf("") : exp2i(-ps.e[i] - 7);
                 }
 #pragma unroll
                 for (int tt = 0; tt < TW; ++tt) {
-                    float part[TBW];
-                    tile_partials<4, TBW>(ps.r[j].a, S, ps.r[j].w[tt], dw, sc, part);
+                    float part[TB];
+                    tile_partials<4, TB>(ps.r[j].a, S, ps.r[j].w[tt], dw, sc, part);
 #pragma unroll
-                    for (int i = 0; i < TBW; ++i)
-                        if (i < gblk) redm[((c * TW + tt) * TB + grp * TBW + i) * 64 + lane] = part[i];
+                    for (int i = 0; i < TB; ++i)
+                        if (i < gblk) redm[((c * TW + tt) * TB + i) * 64 + lane] = part[i];
                 }
             }
         }
     };
-    const int step = nslots * KC;
+    const int step = nw * KC;
     {
         PassRegs pa;
         load_pass(a, pa, 0, true);

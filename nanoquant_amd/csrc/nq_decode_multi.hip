@@ -1,4 +1,4 @@
-// Launchers of the several-token decode path (split launch, 2-16 tokens):
+// Launchers of the several-token decode path (split launch, 5-8 tokens):
 // k_decode_stage0 and k_decode_stage1m, documented in nq_decode_kernels.h.
 #include "nq_decode_kernels.h"
 
@@ -46,7 +46,6 @@ int enqueue_stage1m(const Batch& batch, const LaunchShape& s, hipStream_t stream
     if (s.tb == 1) return s.kc == 2 ? by_tiles<1, 2>(batch, s, stream) : by_tiles<1, 1>(batch, s, stream);
     if (s.kc != 1) return NQ_ERR_LAUNCH;  // two token blocks per wave: one chunk per pass
     if (s.tb == 2) return by_tiles<2, 1>(batch, s, stream);
-    if (s.tb == 4) return by_tiles<4, 1>(batch, s, stream);
     return NQ_ERR_LAUNCH;
 }
 

@@ -7,36 +7,7 @@
 //   GEMM 2:       y[t, o] = s_out[o] * (lm · U±1ᵀ)[t, o]
 //                           + Σ_k x[t, idx_k] W_sal[o, k] (* scale_k) + bias[o]
 //
-// Activation operands. A group of 32 columns of a row shares a power of two
-// 2^e (its largest value lies in [2, 4) of it); a value is the sum of P fp6
-// (e2m3) numbers, each the rounding of what the ones before left over, plane p
-// in units of 2^(e - 5p). A plane takes a value below 4 to a remainder of at
-// most 1/8, which the next plane, 32 times finer, sees below 4 again, so every
-// plane adds five bits: P = 3 holds 16 bits below the group's largest value
-// (half a unit is 2^-14 of 4: 4e-5 rel-L2 on normal rows, where single fp16
-// operands have 2e-4 to 3e-4), P = 5 all 24 bits of an fp32 value of the
-// group's largest binade (split operands: NQ_PREFILL_FP16_SPLIT). The group's
-// exponent is the MFMA's A scale and the plane's 2^-5p its B scale, so no
-// pass over the row is needed for a scale of its own, the rank intermediate is
-// formed from its own values (no bound), and the sums come out unscaled. A
-// group that holds a NaN or an infinity has the NaN scale: every output of the
-// token is NaN, as the reference's fp32 forward yields (a non-finite
-// activation reaches every rank value with both signs; reference.py:208-217).
-//
-// Why fp6 planes. The signs are exact in fp4 (+-1), the products exact, and
-// the matrix cores take fp6 x fp4 at four times the fp16 rate (register-only
-// loops on this chip: 4.1 - 6.7 PFLOP/s against 1.28 - 1.85, held down by
-// power either way), so three planes cost 3/4 of one fp16 pass and five planes
-// 5/8 of the two of split fp16 operands. Expanding signs costs one shift and
-// one and-or for eight of them instead of three instructions for four.
-//
-// Sign operand, straight from the decode tile layout (16-row tiles; in
-// 128-column block kb = 4c + d a lane's word d of chunk c holds, at bit 8b + m,
-// column 128kb + 16m + 4g + b for lane group g). A 32 x 32 x 64 MFMA takes, in
-// lane 32h + r, 32 k slots of B column r: exactly one word, that of lane group
-// g = 2 step + h for 64-column step `step`. Slot 8s + j is the nibble j of
-// dword s, sign bit 4j + s of the word: column 16 (4 (j & 1) + s) + 4g + (j >> 1).
-// The columns of one word are the 32-column group that shares a scale.
+// The operands' form and why: nq_planes.h.
 //
 // Activation operand in memory, in the order the MFMA and LDS want it: per
 // 128-column block kb and group of 32 rows, for each 64-column step and plane
@@ -57,116 +28,14 @@
 // order (deterministic) and applies the epilogue. A batched call runs up to
 // eight GEMMs of one phase in one launch, their (column block, slice) ranges
 // concatenated along grid x.
-#include <utility>
-
+#include "nq_planes.h"
 #include "nq_prefill.h"
 
 namespace {
 
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef uint32_t v6u __attribute__((ext_vector_type(6)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v32f __attribute__((ext_vector_type(32)));
-
-constexpr int kBlock = 256;
-constexpr int kBK = 128;                 // columns per K step
-constexpr int kTileRows = 16;
-constexpr int kRows = 32;                // rows of an operand group
-constexpr int kPlaneBytes = 1536;        // 32 rows x 64 columns of 6 bits
-constexpr int kPlaneBits = 5;            // what a plane adds
-constexpr int kPrefillBatch = 8;         // members of one batched call
-constexpr int kPlanes = 3, kPlanesSplit = 5;
-constexpr int64_t kRowsPerGridZ = 65535;  // grid y's limit; rows beyond it go to grid z
-// s_waitcnt vmcnt(n) expcnt(7) lgkmcnt(15): wait until this wave has at most n
-// vector memory operations in flight (gfx9 encoding), as a builtin the
-// compiler's own wait tracking takes into account.
-constexpr int wait_vmcnt(int n) { return (n & 15) | 0x0F70 | (n >> 4) << 14; }
-constexpr int kWaitVmcnt0 = wait_vmcnt(0);
-
-__device__ __forceinline__ float exp2i(int e) { return __uint_as_float(static_cast<uint32_t>(e + 127) << 23); }
-
-// An activation matrix as fp6 planes: rows in groups of 32 (row_groups of
-// them; the rows past the last token hold anything), nkb 128-column blocks.
-struct Operand {
-    uint8_t* planes;     // [nkb][row_groups][2][P][1536]
-    uint8_t* exps;       // [nkb][row_groups][64][2]
-    int64_t row_groups;
-};
-
-// Columns 4g + b + 16m of 128-column block kb of a row, a = m in [0, 4) (four
-// b each) and c = m in [4, 8), as P planes.
-template <int P>
-__device__ __forceinline__ void store_group(const Operand& op, int64_t row, int64_t kb, int g, v16f a, v16f c) {
-    uint32_t top = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const uint32_t x = __float_as_uint(a[i]) & 0x7fffffffu, y = __float_as_uint(c[i]) & 0x7fffffffu;
-        top = top > x ? top : x;
-        top = top > y ? top : y;
-    }
-    const bool finite = top < 0x7f800000u;
-    int e = static_cast<int>(top >> 23) - 128;  // 2^e: half the largest value's binade
-    e = e < -100 ? -100 : (finite ? e : 0);
-    const int64_t at = kb * op.row_groups + (row >> 5);
-    const int lane = 32 * (g & 1) + static_cast<int>(row & 31);
-    uint8_t* const dst = op.planes + (at * 2 + (g >> 1)) * (P * kPlaneBytes);
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        const float unit = exp2i(e - kPlaneBits * p);
-        v6u w = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, c, unit);
-        // The conversion's operands outlive it, or the compiler lets its result
-        // overlap them, and what is written first is read again (seen in the
-        // last plane: 5.7e-6 rel-L2 with five).
-        asm volatile("" : "+v"(w) : "v"(a), "v"(c), "v"(unit));
-        *reinterpret_cast<uint4*>(dst + p * kPlaneBytes + 16 * lane) = make_uint4(w[0], w[1], w[2], w[3]);
-        *reinterpret_cast<uint2*>(dst + p * kPlaneBytes + 1024 + 8 * lane) = make_uint2(w[4], w[5]);
-        if (p + 1 < P) {
-            v32f got = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(w, unit);
-            asm volatile("" : "+v"(got) : "v"(w), "v"(unit));
-#pragma unroll
-            for (int i = 0; i < 16; ++i) a[i] -= got[2 * i], c[i] -= got[2 * i + 1];  // exact
-        }
-    }
-    op.exps[(at * 64 + lane) * 2 + (g >> 1)] = static_cast<uint8_t>(finite ? e + 127 : 255);
-}
-
-// Four elements of a buffer as fp32: one load (the host checked alignment).
-template <int DT>
-__device__ __forceinline__ v4f load4_as(const void* __restrict__ p, int64_t i) {
-    if constexpr (DT == NQ_DTYPE_F32) return *reinterpret_cast<const v4f*>(static_cast<const float*>(p) + i);
-    const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p) + i);
-    v4f v;
-    if constexpr (DT == NQ_DTYPE_BF16) {
-        v[0] = __uint_as_float(w.x << 16), v[1] = __uint_as_float(w.x & 0xffff0000u);
-        v[2] = __uint_as_float(w.y << 16), v[3] = __uint_as_float(w.y & 0xffff0000u);
-    } else {
-        v[0] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w.x)));
-        v[1] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w.x >> 16)));
-        v[2] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w.y)));
-        v[3] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w.y >> 16)));
-    }
-    return v;
-}
-
-// Row pass of one member of a batched call.
-struct PrepArgs {
-    const void* act;                 // [tokens, cols] activations
-    const void* colscale;            // [cols] s_in
-    int act_dtype, colscale_dtype;
-    int64_t tokens, cols, nkb;
-    Operand out;
-};
-
-struct PrepBatch {
-    PrepArgs p[kPrefillBatch];
-};
-
 // planes of act * colscale, zero past the last column. Grid: 16-row groups,
 // four 128-column blocks (one per wave), members; lane 16 g + r takes row r and
-// columns 16 m + 4 g + [0, 4). Bound by memory and launch: VEC reads four
-// elements per load (cols % 4 == 0, aligned), typed, all issued before the
-// first use; the generic form takes any type, alignment and width.
+// columns 16 m + 4 g + [0, 4). Bound by memory and launch.
 // Written and read once, 2048 x 14336 bf16 moves 126 MB in 23.5 us (5.4 TB/s;
 // fp16 operands with a scale per row: 19.4 us for 117 MB); 61 x 4096 4.6 us.
 template <int ADT, int SDT, int P, bool VEC>
@@ -175,47 +44,12 @@ __global__ __launch_bounds__(kBlock) void k_prep_rows(const PrepBatch batch) {
     const int lane = threadIdx.x & 63, g = lane >> 4;
     const int64_t row = static_cast<int64_t>(blockIdx.x) * 16 + (lane & 15);
     const int64_t kb = static_cast<int64_t>(blockIdx.y) * 4 + (threadIdx.x >> 6);
-    const int64_t cols = pa.cols;
     if (kb >= pa.nkb || row >= pa.tokens) return;
-    const int64_t c0 = kb * kBK + 4 * g, at = row * cols + c0;
     v16f half[2];
-    if constexpr (VEC) {
-        v4f x[8], s[8];
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            const int64_t back = c0 + 16 * m < cols ? 16 * m : -c0;  // past the row: its first columns, dropped below
-            x[m] = load4_as<ADT>(pa.act, at + back);
-            s[m] = load4_as<SDT>(pa.colscale, c0 + back);
-        }
-#pragma unroll
-        for (int m = 0; m < 8; ++m)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) half[m >> 2][4 * (m & 3) + b] = c0 + 16 * m < cols ? x[m][b] * s[m][b] : 0.0f;
-    } else {
-#pragma unroll
-        for (int m = 0; m < 8; ++m)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int64_t c = 16 * m + b;
-                half[m >> 2][4 * (m & 3) + b] = c0 + c < cols
-                                                    ? nq::load_f32(pa.act, pa.act_dtype, at + c) *
-                                                          nq::load_f32(pa.colscale, pa.colscale_dtype, c0 + c)
-                                                    : 0.0f;
-            }
-    }
+    GroupLoad<ADT, SDT, VEC> raw;
+    raw.load(pa, row, kb, g);
+    raw.values(pa, row, kb, g, half);
     store_group<P>(pa.out, row, kb, g, half[0], half[1]);
-}
-
-// Signs of one word as the B operand (32 fp4 values of +-1): nibble j of dword
-// s takes sign bit 4j + s.
-__device__ __forceinline__ v8i expand_signs(uint32_t w, uint32_t mask, uint32_t one) {
-    // The masks come in registers: a VOP3 instruction cannot take two literals.
-    v8i b = {};
-    b[0] = static_cast<int>(((w << 3) & mask) | one);
-    b[1] = static_cast<int>(((w << 2) & mask) | one);
-    b[2] = static_cast<int>(((w << 1) & mask) | one);
-    b[3] = static_cast<int>((w & mask) | one);
-    return b;
 }
 
 // One plane's product of a 64-column step: A fp6 (format 2) with its row
@@ -226,78 +60,10 @@ __device__ __forceinline__ v16f mfma_plane(const v8i& a, const v8i& b, const v16
     else return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 2, 4, STEP, ea, 0, eb4);
 }
 
-// A wave-uniform value, in scalar registers.
-__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
-    return static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32))) << 32 |
-           static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
-}
-
-template <typename F, int... I>
-__device__ __forceinline__ void each(std::integer_sequence<int, I...>, const F& f) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-
 // The LDS byte address of a shared pointer, for M0.
 __device__ __forceinline__ uint32_t lds_address(char* p) {
     typedef __attribute__((address_space(3))) char lds_char_t;
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_char_t*)p));
-}
-
-template <int W>
-struct __attribute__((packed, aligned(4))) WordRun {
-    uint32_t w[W];
-};
-
-struct GemmArgs {
-    Operand a;                // [m] rows of nb 128-column blocks
-    int64_t m;                // tokens
-    const uint32_t* tiles;    // sign tiles [rt][nb * 64] (chunked, see above)
-    int64_t n;                // sign rows (rank or out)
-    int64_t nb;               // 128-column blocks
-    const void* col_scale;    // [n] s_mid or s_out
-    int col_scale_dtype;
-    // GEMM 1: the rank intermediate's operand (planes set); GEMM 2: y and what joins it
-    Operand mid;
-    int64_t mid_blocks;       // 128-column blocks of `mid`
-    const void* x;
-    int x_dtype;
-    int64_t in;
-    int64_t salient_count;
-    const int32_t* salient_indices;
-    const void* salient_values;
-    int salient_dtype;
-    const void* salient_scales;
-    int scale_dtype;
-    const void* bias;
-    int bias_dtype;
-    void* out;                // [M, n]
-    int out_dtype;
-    int64_t k_per_split;      // K blocks per K slice
-    int64_t splits;           // K slices (1: no split)
-    int64_t col_blocks;       // column blocks at the launch's block width
-    float* partial;           // [splits][M][part_ld(n)] raw accumulators, or null (direct epilogue)
-};
-
-// Floats per row of the partials: rows begin at multiples of 16 bytes.
-__host__ __device__ constexpr int64_t part_ld(int64_t n) { return (n + 3) & ~int64_t(3); }
-
-// Up to kPrefillBatch GEMMs of one phase (the members of a batched call share
-// the token count) in one launch. Grid x concatenates the members' ranges:
-// member i owns [begin[i], begin[i + 1]) (k_sign_gemm: col_blocks * splits
-// workgroups, slice-major; the reductions: their column blocks, none for a
-// member without a split); begin[i] = INT32_MAX past the last member.
-struct GemmBatch {
-    int32_t begin[kPrefillBatch];
-    GemmArgs p[kPrefillBatch];
-};
-
-// The member whose range holds grid-x index x: the last one beginning at or
-// before it (a member with an empty range shares its begin with the next).
-__device__ __forceinline__ int batch_member(const GemmBatch& b, int x) {
-    int m = 0;
-#pragma unroll
-    for (int i = 1; i < kPrefillBatch; ++i) m = x >= b.begin[i] ? i : m;
-    return m;
 }
 
 // Block shapes, as (WR wave rows, II 32-row A fragments and JJ 32-column B
@@ -755,26 +521,6 @@ __global__ __launch_bounds__(kBlock, 2) void k_sign_gemm(const GemmBatch batch) 
         default:
             break;
     }
-}
-
-// Element i of an F32 / F16 / BF16 buffer from two unconditional 16-bit
-// loads (the halves of an fp32, or the same half twice), decoded by a
-// uniform select: no branch surrounds the loads, so they issue together.
-struct Raw2 {
-    uint32_t lo, hi;
-};
-
-__device__ __forceinline__ Raw2 load_raw2(const void* __restrict__ p, int dtype, int64_t i) {
-    const uint16_t* h = static_cast<const uint16_t*>(p);
-    const bool wide = dtype == NQ_DTYPE_F32;
-    return Raw2{h[wide ? 2 * i : i], h[wide ? 2 * i + 1 : i]};
-}
-
-__device__ __forceinline__ float raw2_value(const Raw2& r, int dtype) {
-    const float f32 = __uint_as_float((r.hi << 16) | (r.lo & 0xffffu));
-    const float bf16 = __uint_as_float(r.lo << 16);
-    const float f16 = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(r.lo)));
-    return dtype == NQ_DTYPE_F32 ? f32 : (dtype == NQ_DTYPE_BF16 ? bf16 : f16);
 }
 
 // A GEMM of few tokens and few sign rows: a workgroup takes 32 sign rows and

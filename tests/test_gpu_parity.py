@@ -395,6 +395,33 @@ def test_prefill_planes_edges(tokens, geometry, operands, bar):
     assert torch.equal(backend.linear(x.cuda(), layer), y)
 
 
+@pytest.mark.parametrize("launch", ["split", "fused"])
+@pytest.mark.parametrize("tokens", [9, 13, 16])
+@pytest.mark.parametrize("geometry,x_dtype,scale_dtype", [
+    ((35, 17, 33), torch.float32, torch.float16),        # generic loads, one narrow chunk
+    ((516, 131, 129), torch.bfloat16, torch.float16),    # narrow last chunk, two exponent groups past the rank
+    ((4100, 2000, 520), torch.float16, torch.float16),   # more chunks than waves, 32 sign rows a workgroup
+    ((1152, 9000, 768), torch.float32, torch.bfloat16),  # 64
+    ((700, 16500, 300), torch.bfloat16, torch.float32),  # 128
+])
+def test_decode_planes_edges(geometry, x_dtype, scale_dtype, tokens, launch):
+    """9 to 16 tokens against 64 bits: four planes leave at most 2^-19 of a
+    32-column group's largest value, 1.4e-6 rel-L2 on normal rows and sqrt(2) of
+    it over both GEMMs, and fp32 sums add to that."""
+
+    in_f, out_f, rank = geometry
+    backend = HipPackedBackend(decode_launch=launch)
+    _say("decode planes", geometry, tokens, launch)
+    shape = syn.LinearShape("blocks.0.mlp.gate_proj", in_f, out_f, rank)
+    state = syn.synthetic_packed_layer(shape, seed=tokens + sum(geometry), bias=True, scale_dtype=scale_dtype)
+    x = syn.synthetic_activations(tokens, in_f, seed=tokens).to(x_dtype)
+    y = backend.linear(x.cuda(), backend.prepare(state, "cuda"))
+    expected = _exact_linear(state, x)
+    err = float((y.cpu().double() - expected).norm() / expected.norm())
+    print(f"  rel_l2={err:.2e}", flush=True)
+    assert err <= 5e-6
+
+
 def test_prefill_planes_with_an_outlier_channel():
     """One channel a thousand times the others: its group's other values keep
     2^-14 of it, at most sqrt(31) 2^-14 = 3.4e-4 of the channel's own share of
