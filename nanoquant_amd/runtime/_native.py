@@ -190,7 +190,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         "nq_read_stream": (c_int, [vp, c_i64, vp, c_i64, vp]),
         "nq_linear_batch": (
             c_int,
-            [ctypes.POINTER(desc_p), ctypes.c_int32, ctypes.POINTER(vp), ctypes.c_int32, c_i64,
+            # vp: an array of descriptor pointers or of their addresses.
+            [vp, ctypes.c_int32, ctypes.POINTER(vp), ctypes.c_int32, c_i64,
              ctypes.POINTER(vp), ctypes.c_int32, ctypes.POINTER(vp), ctypes.POINTER(c_i64), vp],
         ),
         "nq_linear_batch_fused": (
@@ -268,6 +269,10 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def current_stream_handle(device: torch.device) -> int:
+    # The raw handle: a Stream object built for every launch costs several times as much. What has
+    # no device index (a CPU tensor's device, which is refused there) takes the public call.
+    if device.type == "cuda" and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

@@ -35,6 +35,7 @@ from nanoquant_amd.runtime.row_sidecar import RowSidecarLayerState
 HIP_PACKED_BACKEND_NAME = "rocm-packed-hip"
 HIP_PACKED_BACKEND_VERSION = "1"
 _FLOAT_DTYPES = ("float16", "bfloat16", "float32")
+_DEVICE_FLOATS = (torch.float32, torch.bfloat16, torch.float16)
 _REQUIRED_ARCH = "gfx950"
 
 
@@ -132,6 +133,10 @@ def _describe(
         desc.row_values = ptr(p.row_values)
         desc.row_scales = ptr(p.row_scales)
 
+
+# Argument arrays of a batch of n members.
+_POINTERS = [ctypes.c_void_p * n for n in range(9)]
+_SIZES = [ctypes.c_int64 * n for n in range(9)]
 
 _DECODE_LAUNCH = {"split": _native.NQ_DECODE_SPLIT, "fused": _native.NQ_DECODE_FUSED}
 _PREFILL_OPERANDS = {"fp16": _native.NQ_PREFILL_FP16, "split": _native.NQ_PREFILL_FP16_SPLIT}
@@ -311,46 +316,51 @@ class HipPackedBackend:
         (src/nanoquant/runtime/cuda_backend.py:65-144): members may have distinct
         inputs and any rank; inputs may be the same tensor."""
 
-        if len(values) != len(layers) or not 1 <= len(layers) <= 8:
+        n = len(layers)
+        if len(values) != n or not 1 <= n <= 8:
             raise ValueError("HIP packed batch needs 1-8 layers with one input each")
-        if len({id(layer) for layer in layers}) != len(layers):
+        if len(set(map(id, layers))) != n:
             raise ValueError("HIP packed batch members must be distinct prepared layers")
         payloads = [self._payload(layer) for layer in layers]
-        if any(p.tiles is None for p in payloads):
-            raise ValueError("HIP packed batch requires layers prepared with tiled decode")
-        tokens = {v.numel() // layer.spec.in_features for v, layer in zip(values, layers)}
-        dtypes = {v.dtype for v in values}
-        if len(tokens) != 1 or len(dtypes) != 1:
-            raise ValueError("HIP packed batch members must share token count and input dtype")
-        (count,) = tokens
-        for value, layer, payload in zip(values, layers, payloads):
-            _check_value(value, layer.spec, payload.device)
-        if output_dtype not in (torch.float32, torch.bfloat16, torch.float16):
+        for payload in payloads:
+            if payload.tiles is None:
+                raise ValueError("HIP packed batch requires layers prepared with tiled decode")
+        specs = [layer.spec for layer in layers]
+        dtype = values[0].dtype
+        count = values[0].numel() // specs[0].in_features
+        for value, spec in zip(values, specs):
+            if value.dtype != dtype or value.numel() // spec.in_features != count:
+                raise ValueError("HIP packed batch members must share token count and input dtype")
+        for value, spec, payload in zip(values, specs, payloads):
+            _check_value(value, spec, payload.device)
+        if output_dtype not in _DEVICE_FLOATS:
             raise ValueError(f"HIP packed output dtype is unsupported: {output_dtype}")
         device = payloads[0].device
         if outs is None:
-            outs = [
-                torch.empty((*v.shape[:-1], layer.spec.out_features), dtype=output_dtype, device=device)
-                for v, layer in zip(values, layers)
-            ]
-        for out, value, layer in zip(outs, values, layers):
-            shape = (*value.shape[:-1], layer.spec.out_features)
-            if tuple(out.shape) != shape or out.dtype != output_dtype or not out.is_contiguous():
-                raise ValueError("HIP packed output tensor shape, dtype or layout differs")
+            outs = [torch.empty((*v.shape[:-1], spec.out_features), dtype=output_dtype, device=device)
+                    for v, spec in zip(values, specs)]
+        else:
+            for out, value, spec in zip(outs, values, specs):
+                shape = (*value.shape[:-1], spec.out_features)
+                if tuple(out.shape) != shape or out.dtype != output_dtype or not out.is_contiguous():
+                    raise ValueError("HIP packed output tensor shape, dtype or layout differs")
         lib = _native.load()
-        n = len(layers)
-        sizes = [int(lib.nq_linear_workspace_bytes(ctypes.byref(p.desc), count)) for p in payloads]
+        sizes = [lib.nq_linear_workspace_bytes(ctypes.byref(p.desc), count) for p in payloads]
         if min(sizes) < 0:
             raise ValueError("HIP packed layer descriptor was rejected")
-        workspaces = [torch.empty(max(b, 1), dtype=torch.uint8, device=device) for b in sizes]
-        desc_ptrs = (ctypes.POINTER(_native.LinearDesc) * n)(*[ctypes.pointer(p.desc) for p in payloads])
-        x_ptrs = (ctypes.c_void_p * n)(*[v.data_ptr() for v in values])
-        y_ptrs = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
-        w_ptrs = (ctypes.c_void_p * n)(*[w.data_ptr() for w in workspaces])
-        w_sizes = (ctypes.c_int64 * n)(*sizes)
+        # One allocation holds every member's workspace, 256-byte aligned.
+        offsets = [0]
+        for size in sizes:
+            offsets.append(offsets[-1] + (size + 255 & -256))
+        workspace = torch.empty(max(offsets[-1], 1), dtype=torch.uint8, device=device)
+        base = workspace.data_ptr()
+        pointers, code = _POINTERS[n], _native.dtype_code
         status = lib.nq_linear_batch(
-            desc_ptrs, n, x_ptrs, _native.dtype_code(values[0].dtype), count, y_ptrs,
-            _native.dtype_code(output_dtype), w_ptrs, w_sizes, _native.current_stream_handle(device),
+            pointers(*[ctypes.addressof(p.desc) for p in payloads]), n,
+            pointers(*[v.data_ptr() for v in values]), code(dtype), count,
+            pointers(*[o.data_ptr() for o in outs]), code(output_dtype),
+            pointers(*[base + offset for offset in offsets[:n]]), _SIZES[n](*sizes),
+            _native.current_stream_handle(device),
         )
         _native.check("nq_linear_batch", status)
         return list(outs)
@@ -562,30 +572,24 @@ class HipPackedBackend:
         payload = self._payload(layer)
         spec = layer.spec
         _check_value(value, spec, payload.device)
-        if output_dtype not in (torch.float32, torch.bfloat16, torch.float16):
+        if output_dtype not in _DEVICE_FLOATS:
             raise ValueError(f"HIP packed output dtype is unsupported: {output_dtype}")
         tokens = value.numel() // spec.in_features
         shape = (*value.shape[:-1], spec.out_features)
+        device = value.device
         if out is None:
-            out = torch.empty(shape, dtype=output_dtype, device=value.device)
+            out = torch.empty(shape, dtype=output_dtype, device=device)
         elif tuple(out.shape) != shape or out.dtype != output_dtype or not out.is_contiguous():
             raise ValueError("HIP packed output tensor shape, dtype or layout differs")
         lib = _native.load()
-        desc = payload.desc
-        ws_bytes = int(lib.nq_linear_workspace_bytes(ctypes.byref(desc), tokens))
+        desc = ctypes.byref(payload.desc)
+        ws_bytes = lib.nq_linear_workspace_bytes(desc, tokens)
         if ws_bytes < 0:
             raise ValueError("HIP packed layer descriptor was rejected")
-        workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=value.device)
+        workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
         status = lib.nq_linear(
-            ctypes.byref(desc),
-            value.data_ptr(),
-            _native.dtype_code(value.dtype),
-            tokens,
-            out.data_ptr(),
-            _native.dtype_code(output_dtype),
-            workspace.data_ptr(),
-            ws_bytes,
-            _native.current_stream_handle(value.device),
+            desc, value.data_ptr(), _native.dtype_code(value.dtype), tokens, out.data_ptr(),
+            _native.dtype_code(output_dtype), workspace.data_ptr(), ws_bytes, _native.current_stream_handle(device),
         )
         _native.check("nq_linear", status)
         return out
@@ -650,7 +654,8 @@ def grouped_hip_projection(value: torch.Tensor, group: HipProjectionGroup) -> tu
 def _check_value(value: torch.Tensor, spec: QuantizedLinearSpec, device: torch.device) -> None:
     if value.device != device:
         raise ValueError("HIP packed input and prepared layer must use the same device")
-    if canonical_torch_dtype(value.dtype) not in _FLOAT_DTYPES:
+    if value.dtype not in _DEVICE_FLOATS:
+        canonical_torch_dtype(value.dtype)  # names a dtype that no runtime tensor has
         raise ValueError(f"HIP packed input dtype is unsupported: {value.dtype}")
     if value.ndim == 0 or value.shape[-1] != spec.in_features:
         raise ValueError("HIP packed input feature dimension differs from the layer")
