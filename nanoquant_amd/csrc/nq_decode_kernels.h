@@ -271,7 +271,7 @@ static_assert(sizeof(LinArgs) == 256 && offsetof(LinArgs, u_tiles) == 64 && offs
               "one use per 64-byte line");
 
 // Stage-2 operand bytes of a [out, rank] U for `tokens` tokens (1: one block of
-// one token; 2-4: one block of four; 5-16: four blocks of four). A multiple of 256.
+// one token; 2-4: one block of four; above: as four blocks of four). A multiple of 256.
 __host__ __device__ inline int64_t lmq_bytes_for(const MatGeo& g2, int64_t tokens) {
     return g2.nc * (tokens == 1 ? 2048 : (tokens <= 4 ? 8192 : 32768));
 }
@@ -2158,7 +2158,7 @@ __global__ __launch_bounds__(THREADS) void k_decode_fused(const Batch batch) {
 
 // Launch bound of a configuration (see k_decode_stage1): blocks of up to four
 // tokens take up to 16 waves of one chunk or 12 of two; several token blocks
-// take at most 8 waves (their operand registers for two or four blocks would
+// take at most 8 waves (their operand registers for two blocks would
 // spill under a bound of 16 waves).
 constexpr int threads_for(int tpb, int kc, int tb = 1) { return tb > 1 ? 512 : (kc == 1 ? 1024 : 768); }
 

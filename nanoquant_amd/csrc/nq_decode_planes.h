@@ -6,7 +6,8 @@
 
 namespace nq {
 
-// Scratch bytes of one linear.
+// Scratch bytes one linear needs: less than decode_scratch_bytes (48.5 bytes a
+// column of x and of the rank against 64), which callers size buffers by.
 int64_t decode_planes_bytes(const nq_linear_desc* d);
 
 // Planes of x * s_in, GEMM 1, GEMM 2 for 1..8 linears sharing the token count

@@ -234,6 +234,7 @@ int launch_decode_planes(const nq_linear_desc* const* descs, int count, const vo
     int64_t nkb_max = 0;
     for (int i = 0; i < count; ++i) {
         const nq_linear_desc* d = descs[i];
+        if (decode_planes_bytes(d) > decode_scratch_bytes(d, tokens)) return NQ_ERR_WORKSPACE;
         const int64_t nb1 = (d->in_features + kBK - 1) / kBK, nb2 = (d->rank + kBK - 1) / kBK;
         const int64_t v_words = (d->rank + kTileRows - 1) / kTileRows * nb1 * 64;
         uint8_t* const ws = static_cast<uint8_t*>(scratch[i]);

@@ -123,6 +123,38 @@ def test_qk_norm_rope_cache(head_dim, q_heads, kv_heads, cache_dtype):
     assert (kc[:, untouched].float() == 7.0).all() and (vc[:, untouched].float() == 7.0).all()
 
 
+@pytest.mark.parametrize("q_heads,kv_heads", [(1, 1), (2, 1), (3, 1), (4, 1), (6, 1), (14, 2)])
+def test_qk_norm_rope_cache_partial_head_groups(q_heads, kv_heads):
+    """Head counts on both sides of a multiple of four, the heads of a workgroup, with q, k and
+    the table's end inside one: every head is written once and nothing past the last one (the
+    buffers are followed by a guard). Arithmetic as above, so its tolerance."""
+
+    g = _g(17)
+    tokens, max_pos, start, d = 3, 8, 6, 64  # the third token lies outside the cache
+    q = torch.randn(tokens, q_heads * d, generator=g)
+    k = torch.randn(tokens, kv_heads * d, generator=g)
+    v = torch.randn(tokens, kv_heads * d, generator=g)
+    cos, sin = ods.rope_tables(d, 1e6, max_pos)
+    backing = torch.full((kv_heads + 4, max_pos, d), 7.0, device=DEV)
+    vback = torch.full_like(backing, 7.0)
+    out = torch.full((tokens * q_heads * d + 4 * d,), 7.0, device=DEV)
+    ops.launch_qk_norm_rope_cache(
+        q.to(DEV), k.to(DEV), v.to(DEV), q_heads=q_heads, kv_heads=kv_heads, head_dim=d, q_norm=None, k_norm=None,
+        eps=1e-6, cos=cos.to(DEV), sin=sin.to(DEV), position=torch.tensor([start], dtype=torch.int32, device=DEV),
+        k_cache=backing[:kv_heads], v_cache=vback[:kv_heads], q_out=out[: tokens * q_heads * d],
+    )
+    inside = max_pos - start
+    c, s = cos[start:], sin[start:]
+    eq = ods.apply_rope(q.view(tokens, q_heads, d)[:inside], c, s)
+    ek = ods.apply_rope(k.view(tokens, kv_heads, d)[:inside], c, s)
+    got = out.cpu()
+    assert relative_l2(got[: inside * q_heads * d].view(inside, q_heads, d), eq) < 1e-6
+    assert (got[inside * q_heads * d:] == 7.0).all()
+    assert relative_l2(backing[:kv_heads, start:].cpu().transpose(0, 1), ek) < 1e-6
+    assert torch.equal(vback[:kv_heads, start:].cpu().transpose(0, 1), v.view(tokens, kv_heads, d)[:inside])
+    assert (backing[kv_heads:] == 7.0).all() and (vback[kv_heads:] == 7.0).all()
+
+
 def reference_attention(q, kc, vc, start, scaling):
     """fp32 causal GQA over cache rows [0, start + t] (q [T, Hq, D], caches [Hkv, L, D])."""
 
