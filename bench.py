@@ -1111,7 +1111,7 @@ def main(argv=None) -> int:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "bf16-in/fp32-acc (1-bit signs, int8-digit MFMA decode, fp16 MFMA prefill)",
+        "dtype": "bf16-in/fp32-acc (1-bit signs, int8-digit MFMA decode, fp6-plane MFMA prefill)",
         "data": ("synthetic: Bernoulli(0.5) signs, fp16 lognormal(0,0.25) scales, bf16 N(0,1) activations, "
                  "random-init bf16 N(0,0.02) embeddings/lm_head"),
         "config": {"workload": workload, "value_is": unit_note, "global_batch": 1, "layers": args.layers,
