@@ -236,9 +236,13 @@ bool planes_path(int64_t tokens) { return tokens >= kPlanesTokens; }
 // per block of four tokens per chunk) are shared by its TW tiles, against
 // fewer waves. One token block (stage 2 after the in-kernel staging): four
 // tiles from 4096 waves, two from 2048. Two blocks (stage 0 path): two tiles in
-// both stages (measured best against one and four, per stage, at 8 tokens).
+// both stages (measured best against one and four, per stage, at 8 tokens),
+// one where two would leave more than half of the CUs idle (192 tiles).
+// Against two tiles (us a call at 8 tokens in a graph): stage 1 of 48 tiles
+// 13.7 -> 13.0, of 103 15.5 -> 15.3, of 231 15.7 -> 17.1; stage 2 of 160 tiles
+// with 96 in stage 1 17.3 -> 16.6.
 int pick_tiles_multi(int64_t tiles, int nw, int tb) {
-    if (tb > 1) return 2;
+    if (tb > 1) return tiles <= 192 ? 1 : 2;
     const int64_t waves = tiles * nw;
     return waves >= 4 * 1024 ? 4 : (waves >= 2 * 1024 ? 2 : 1);
 }

@@ -422,6 +422,24 @@ def test_decode_planes_edges(geometry, x_dtype, scale_dtype, tokens, launch):
     assert err <= 5e-6
 
 
+@pytest.mark.parametrize("tokens", [5, 8])
+@pytest.mark.parametrize("out_f,rank", [(3072, 3072), (3088, 3072), (3072, 3073), (17, 33)])
+def test_two_token_blocks_one_or_two_tiles(out_f, rank, tokens):
+    """5 to 8 tokens at up to 192 tiles of a stage (one a workgroup) and above (two): chunk sums
+    add up in chunk order, so the split launch equals the fused one bit for bit; against 64 bits
+    the operands' 2^-23 of a bound about sqrt(K) above the values leaves 2e-5, 1e-4 with the sums."""
+
+    in_f = 1100
+    _say("two token blocks", out_f, rank, tokens)
+    state = syn.synthetic_packed_layer(syn.LinearShape("blocks.0.mlp.gate_proj", in_f, out_f, rank), seed=out_f + rank)
+    x = syn.synthetic_activations(tokens, in_f, seed=tokens)
+    split, fused = HipPackedBackend(), HipPackedBackend(decode_launch="fused")
+    y = split.linear(x.cuda(), split.prepare(state, "cuda"))
+    assert torch.equal(y, fused.linear(x.cuda(), fused.prepare(state, "cuda")))
+    expected = _exact_linear(state, x)
+    assert float((y.cpu().double() - expected).norm() / expected.norm()) <= 1e-4
+
+
 def test_prefill_planes_with_an_outlier_channel():
     """One channel a thousand times the others: its group's other values keep
     2^-14 of it, at most sqrt(31) 2^-14 = 3.4e-4 of the channel's own share of
