@@ -1214,8 +1214,9 @@ __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const Flas
 #pragma unroll
                 for (int j = 0; j < 4; ++j) o[d0 + i][j] = fmaf(o[d0 + i][j], keep, y[i][j]);
         }
-        if (edge && wild[half]) {
-            // The values that store_tile left out, for the tokens that see their rows.
+        if (wild[half]) {
+            // The values that store_tile left out, for the tokens that see their rows: in every
+            // tile with rows past `first`, also one whose rows all of this unit's tokens see.
             const int r_end = last < row0 + R - 1 ? last : row0 + R - 1;
             for (int r = row0 > first ? row0 : first + 1; r <= r_end; ++r) {
                 const int rr = r - row0;

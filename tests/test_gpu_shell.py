@@ -274,6 +274,47 @@ def test_prompt_attention_non_finite_value_is_causal(q_heads, kv_heads, head_dim
     assert not torch.isfinite(out[hit]).any()
 
 
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize(
+    "q_heads,kv_heads,head_dim,tokens,start,max_pos",
+    [
+        # a workgroup's units in one token tile, in two, in three and in four: its later units see
+        # whole tiles of rows that its first one does not
+        (8, 2, 128, 70, 20, 96),
+        (16, 8, 128, 70, 20, 96),
+        (6, 2, 128, 130, 47, 200),
+        (4, 4, 64, 70, 0, 96),
+        (4, 4, 64, 70, 20, 96),
+        (2, 2, 256, 64, 0, 64),
+        (8, 4, 256, 64, 15, 80),
+        # the cache shared out between workgroups; enough workgroups for one wave half each
+        (4, 4, 64, 70, 880, 1000),
+        (64, 64, 64, 513, 20, 533),
+    ],
+)
+def test_prompt_attention_non_finite_value_at_any_row(q_heads, kv_heads, head_dim, tokens, start, max_pos, value):
+    """As above for rows that every token sees, that some do, in the first, a middle and the last
+    tile: the tokens at or after the row are not finite in that dimension, all else keeps its bits."""
+
+    g = _g(18)
+    kc = torch.randn(kv_heads, max_pos, head_dim, generator=g).to(torch.bfloat16).to(DEV)
+    vc = torch.randn(kv_heads, max_pos, head_dim, generator=g).to(torch.bfloat16).to(DEV)
+    q = 2 * torch.randn(tokens, q_heads, head_dim, generator=g).to(DEV)
+    call = dict(position=torch.tensor([start], dtype=torch.int32, device=DEV), scaling=head_dim**-0.5,
+                out_dtype=torch.float32)
+    base = ops.launch_attention(q, kc, vc, **call).view(tokens, q_heads, head_dim)
+    group, dim = q_heads // kv_heads, head_dim - 27
+    for row in sorted({0, start, start + 1, start + 5, start + 17, start + tokens // 2, start + tokens - 1}):
+        _say("value row", q_heads, kv_heads, head_dim, start, row)
+        bad = vc.clone()
+        bad[1, row, dim] = value
+        out = ops.launch_attention(q, kc, bad, **call).view(tokens, q_heads, head_dim)
+        hit = torch.zeros_like(base, dtype=torch.bool)
+        hit[max(row - start, 0):, group:2 * group, dim] = True
+        assert torch.equal(out[~hit], base[~hit])
+        assert not torch.isfinite(out[hit]).any()
+
+
 def test_prompt_attention_tokens_outside_the_cache_are_zero():
     g = _g(16)
     kc = torch.randn(2, 40, 128, generator=g).to(torch.bfloat16).to(DEV)
