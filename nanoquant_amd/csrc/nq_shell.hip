@@ -587,13 +587,14 @@ __global__ __launch_bounds__(D * GROUPS) void k_attention_merge(
         float mnew = mrun;
 #pragma unroll
         for (int i = 0; i < ROUND; ++i) mnew = b0 + i < nb ? fmaxf(mnew, mb[i]) : mnew;
-        const float keep = nq::merge_exp(mrun - mnew);  // 0 in the first round
+        const float base = mnew == -INFINITY ? 0.0f : mnew;  // every block so far weighs 0 (-inf - -inf is NaN)
+        const float keep = nq::merge_exp(mrun - base);  // 0 in the first round
         lsum *= keep;
         acc *= keep;
 #pragma unroll
         for (int i = 0; i < ROUND; ++i) {
             if (b0 + i < nb) {  // a select: slots past the position may hold anything
-                const float f = nq::merge_exp(mb[i] - mnew);
+                const float f = nq::merge_exp(mb[i] - base);
                 lsum = fmaf(lb[i], f, lsum);
                 acc = fmaf(ab[i], f, acc);
             }
@@ -609,6 +610,7 @@ __global__ __launch_bounds__(D * GROUPS) void k_attention_merge(
         const int groups = nb < (GROUPS - 1) * ROUND + 1 ? (nb + ROUND - 1) / ROUND : GROUPS;  // that hold a block
         float mnew = mrun;
         for (int i = 1; i < groups; ++i) mnew = fmaxf(mnew, g_m[i]);
+        mnew = mnew == -INFINITY ? 0.0f : mnew;
         const float keep = nq::merge_exp(mrun - mnew);
         lsum *= keep;
         acc *= keep;
@@ -977,6 +979,46 @@ struct FlashArgs {
     float* part_acc;
 };
 
+// One query against cache rows [begin, end) in fp32, by one wave, 64 rows at a
+// time: the running max of the scaled scores, the sum of the weights and the
+// weighted values of dimensions (D / 64) lane + [0, D / 64). `q` is uniform.
+template <int D, int CT>
+__device__ void fp32_attention_row(const float* __restrict__ q, const char* __restrict__ k_head,
+                                   const char* __restrict__ v_head, int begin, int end, float scaling, int lane,
+                                   float& m, float& l, float (&acc)[D / kWave]) {
+    constexpr int E = D / kWave, U = 8;
+    m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int j = 0; j < E; ++j) acc[j] = 0.0f;
+    for (int r0 = begin; r0 < end; r0 += kWave) {
+        const int rows = end - r0 < kWave ? end - r0 : kWave;
+        const int64_t r = r0 + (lane < rows ? lane : rows - 1);
+        const float score = lane < rows ? k_row_dot<D, CT>(k_head + r * (2 * D), q) * scaling : -INFINITY;
+        const float mx = fmaxf(m, wave_max(score));
+        const float base = mx == -INFINITY ? 0.0f : mx;  // no score above -inf yet: their weights are 0
+        const float keep = m == -INFINITY ? 0.0f : expf(m - base);
+        const float w = lane < rows ? expf(score - base) : 0.0f;
+        m = mx;
+        l = l * keep + wave_sum(w);
+#pragma unroll
+        for (int j = 0; j < E; ++j) acc[j] *= keep;
+        for (int i0 = 0; i0 < rows; i0 += U) {
+            float vv[U][E];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t i = r0 + (i0 + u < rows ? i0 + u : rows - 1);
+                load_v<E, CT>(v_head + (i * D + lane * E) * 2, vv[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + u < rows) {
+#pragma unroll
+                    for (int j = 0; j < E; ++j) acc[j] = fmaf(row_lane(w, i0 + u), vv[u][j], acc[j]);
+                }
+        }
+    }
+}
+
 template <int D, int CT, int HALVES>
 __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const FlashArgs g) {
     constexpr int R = flash_rows<D>();
@@ -1268,42 +1310,97 @@ __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const Flas
         mc = mcn;
     }
     l = column_sum(l);
-    if (!unit_ok || t >= g.tokens) return;
-    if (g.splits > 1) {
-        if (pt < static_cast<int64_t>(split) * g.tiles_per_split * R || pt >= g.max_positions || p0 < 0) return;
-        const int64_t pi = attn_part_index(t, h, split, g.q_heads, g.splits);
-#pragma unroll
-        for (int dt = 0; dt < ND; ++dt) *reinterpret_cast<v4f_t*>(g.part_acc + pi * D + 16 * dt + 4 * kg) = o[dt];
-        if (kg == 0) {
-            g.part_ml[2 * pi] = m == -INFINITY ? m : mc * 0.69314718055994531f;
-            g.part_ml[2 * pi + 1] = l;
-        }
-        return;
-    }
+    const int64_t split_row0 = static_cast<int64_t>(split) * g.tiles_per_split * R;
+    const bool ours = unit_ok && t < g.tokens;
     const bool in_range = p0 >= 0 && pt < g.max_positions;  // tokens outside the cache: zero
-    const int64_t out0 = (t * g.q_heads + h) * D + 4 * kg;
+    const bool live = ours && in_range && pt >= split_row0;
+    if (g.splits > 1) {
+        if (live) {
+            const int64_t pi = attn_part_index(t, h, split, g.q_heads, g.splits);
 #pragma unroll
-    for (int dt = 0; dt < ND; ++dt) {
-        v4f_t y;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) y[i] = in_range ? o[dt][i] / l : 0.0f;
-        const int64_t oi = out0 + 16 * dt;
-        if (g.odt == NQ_DTYPE_F32) {
-            float* const dst = static_cast<float*>(g.out) + oi;
-            if (g.vec_out) *reinterpret_cast<v4f_t*>(dst) = y;
-            else dst[0] = y[0], dst[1] = y[1], dst[2] = y[2], dst[3] = y[3];
-        } else {
-            uint16_t* const dst = static_cast<uint16_t*>(g.out) + oi;
-            uint2 w;
-            w.x = pack2(g.odt, y[0], y[1]);
-            w.y = pack2(g.odt, y[2], y[3]);
-            if (g.vec_out) {
-                *reinterpret_cast<uint2*>(dst) = w;
-            } else {
-                dst[0] = static_cast<uint16_t>(w.x), dst[1] = static_cast<uint16_t>(w.x >> 16);
-                dst[2] = static_cast<uint16_t>(w.y), dst[3] = static_cast<uint16_t>(w.y >> 16);
+            for (int dt = 0; dt < ND; ++dt) *reinterpret_cast<v4f_t*>(g.part_acc + pi * D + 16 * dt + 4 * kg) = o[dt];
+            if (kg == 0) {
+                g.part_ml[2 * pi] = m == -INFINITY ? m : mc * 0.69314718055994531f;
+                g.part_ml[2 * pi + 1] = l;
             }
         }
+    } else if (ours) {
+        const int64_t out0 = (t * g.q_heads + h) * D + 4 * kg;
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) {
+            v4f_t y;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = in_range ? o[dt][i] / l : 0.0f;
+            const int64_t oi = out0 + 16 * dt;
+            if (g.odt == NQ_DTYPE_F32) {
+                float* const dst = static_cast<float*>(g.out) + oi;
+                if (g.vec_out) *reinterpret_cast<v4f_t*>(dst) = y;
+                else dst[0] = y[0], dst[1] = y[1], dst[2] = y[2], dst[3] = y[3];
+            } else {
+                uint16_t* const dst = static_cast<uint16_t*>(g.out) + oi;
+                uint2 w;
+                w.x = pack2(g.odt, y[0], y[1]);
+                w.y = pack2(g.odt, y[2], y[3]);
+                if (g.vec_out) {
+                    *reinterpret_cast<uint2*>(dst) = w;
+                } else {
+                    dst[0] = static_cast<uint16_t>(w.x), dst[1] = static_cast<uint16_t>(w.x >> 16);
+                    dst[2] = static_cast<uint16_t>(w.y), dst[3] = static_cast<uint16_t>(w.y >> 16);
+                }
+            }
+        }
+    }
+
+    // An infinity in the cache meets parts of a query or of a weight that have
+    // the other sign or are zero, so it ends as NaN where fp32 arithmetic has
+    // a weight of zero (a score of -inf) or an infinite output. Elements that
+    // came out infinite or NaN are computed once more in fp32; all others keep
+    // what they have. Nothing of this is in the loop above (testing every
+    // value of V there costs 48 VALU instructions a tile and wave).
+    float z = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z = fmaf(o[dt][i], 0.0f, z);
+    const uint64_t odd = __ballot(live && z != z);
+    if (odd == 0) return;  // uniform per wave
+    uint32_t odd_lo = 0, odd_hi = 0;  // this lane's elements: bit 4 dt + i
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t bit = o[dt][i] * 0.0f != 0.0f ? 1u << ((4 * dt + i) & 31) : 0u;
+            if (dt < 8) odd_lo |= bit;
+            else odd_hi |= bit;
+        }
+    __threadfence();  // the stores above are done before others go to the same places
+    constexpr int E = D / kWave;
+    const int split_end = split_row0 + g.tiles_per_split * R < g.max_positions
+                              ? static_cast<int>(split_row0) + g.tiles_per_split * R : static_cast<int>(g.max_positions);
+    for (uint32_t rest = static_cast<uint32_t>((odd | odd >> 16 | odd >> 32 | odd >> 48) & 0xffff); rest; rest &= rest - 1) {
+        const int nn = __builtin_ctz(rest);
+        const int64_t tt = t0 + nn;
+        const float* const qr = g.q + (tt * g.q_heads + h) * D;
+        float qz = 0.0f;
+#pragma unroll
+        for (int j = 0; j < E; ++j) qz = fmaf(qr[lane + kWave * j], 0.0f, qz);
+        if (__ballot(qz != qz)) continue;  // no finite score: NaN throughout, as it is
+        const int end = p0 + tt + 1 < split_end ? static_cast<int>(p0 + tt) + 1 : split_end;
+        float m1, l1, acc[E];
+        fp32_attention_row<D, CT>(qr, k_head, v_head, static_cast<int>(split_row0), end, g.scaling, lane, m1, l1, acc);
+        const float l0 = __shfl(l, nn, kWave);
+        const bool whole = l0 * 0.0f != 0.0f;  // the sum is NaN, so every element is
+        const int64_t pi = attn_part_index(tt, h, split, g.q_heads, g.splits);
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const int d = lane * E + j, src = 16 * ((d >> 2) & 3) + nn, at = 4 * (d >> 4) + (d & 3);
+            const uint32_t lo_bits = __shfl(odd_lo, src, kWave), hi_bits = __shfl(odd_hi, src, kWave);
+            if (!((at < 32 ? lo_bits : hi_bits) >> (at & 31) & 1)) continue;
+            // Beside a sum and a max that stand, the element in their units.
+            if (g.splits > 1) g.part_acc[pi * D + d] = whole ? acc[j] : acc[j] / l1 * l0;
+            else nq::store_f32_as(g.out, g.odt, (tt * g.q_heads + h) * D + d, acc[j] / l1);
+        }
+        if (g.splits > 1 && whole && lane == 0) g.part_ml[2 * pi] = m1, g.part_ml[2 * pi + 1] = l1;
     }
 }
 

@@ -315,6 +315,65 @@ def test_prompt_attention_non_finite_value_at_any_row(q_heads, kv_heads, head_di
         assert not torch.isfinite(out[hit]).any()
 
 
+def _attention_by_token(q, kc, vc, start, scaling):
+    """reference_attention token by token, so that no row past a token touches it."""
+
+    t, hq, d = q.shape
+    group = hq // kc.shape[0]
+    out = torch.empty_like(q)
+    for i in range(t):
+        keys, values = kc[:, : start + i + 1].float(), vc[:, : start + i + 1].float()
+        qi = q[i].view(-1, group, d)
+        weights = torch.softmax((qi[:, :, None, :] * keys[:, None]).sum(-1) * scaling, dim=-1)
+        out[i] = (weights[..., None] * values[:, None]).sum(2).reshape(hq, d)
+    return out.reshape(t, -1)
+
+
+@pytest.mark.parametrize("cache_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "q_heads,kv_heads,head_dim,tokens,start,max_pos",
+    [
+        (4, 4, 64, 37, 20, 96),
+        (8, 2, 128, 40, 30, 70),
+        (8, 4, 256, 18, 15, 80),
+        (4, 2, 64, 20, 1400, 1500),  # the cache in several parts and a merge
+        (2, 2, 128, 18, 40, 1500),   # most parts past the position
+    ],
+)
+def test_prompt_attention_infinite_cache_rows(q_heads, kv_heads, head_dim, tokens, start, max_pos, cache_dtype):
+    """Infinite keys and values do what fp32 arithmetic does with them: a score of -inf weighs
+    nothing (also where a whole part of the cache has no other), one of +inf makes the token NaN,
+    an infinite value an infinity of its sign; the rest is finite, within the tolerance above."""
+
+    g = _g(19)
+    kc = torch.randn(kv_heads, max_pos, head_dim, generator=g).to(cache_dtype)
+    vc = torch.randn(kv_heads, max_pos, head_dim, generator=g).to(cache_dtype)
+    q = 0.5 * torch.randn(tokens, q_heads, head_dim, generator=g)
+    q[..., 5] = q[..., 5].abs() + 0.1  # the sign of key element 5 is that of the infinite score
+    inf = float("inf")
+    cases = {
+        "-inf scores": lambda k, v: k[:, start // 3 : start + 3, 5].fill_(-inf),
+        "-inf scores of the first rows": lambda k, v: k[:, :start, 5].fill_(-inf),
+        "-inf scores of the last rows": lambda k, v: k[0, start + 2 :, 5].fill_(-inf),
+        "+inf score": lambda k, v: k[0, start + 7, 5].fill_(inf),
+        "values": lambda k, v: (v[0, 2, 9].fill_(inf), v[-1, start + 1, head_dim - 1].fill_(-inf)),
+        "both": lambda k, v: (k[:, start // 2, 5].fill_(-inf), v[:, 1, 3].fill_(inf)),
+    }
+    position = torch.tensor([start], dtype=torch.int32, device=DEV)
+    for name, spoil in cases.items():
+        _say("infinite rows", name, q_heads, kv_heads, head_dim, cache_dtype)
+        kb, vb = kc.clone(), vc.clone()
+        spoil(kb, vb)
+        out = ops.launch_attention(q.to(DEV), kb.to(DEV), vb.to(DEV), position=position, scaling=head_dim**-0.5,
+                                   out_dtype=torch.float32).cpu()
+        expected = _attention_by_token(q, kb, vb, start, head_dim**-0.5)
+        finite = torch.isfinite(expected)
+        assert torch.equal(torch.isnan(out), torch.isnan(expected))
+        assert torch.equal(out[torch.isinf(expected)], expected[torch.isinf(expected)])
+        assert torch.isfinite(out[finite]).all() and finite.any()
+        assert relative_l2(out[finite], expected[finite]) < 1e-5
+
+
 def test_prompt_attention_tokens_outside_the_cache_are_zero():
     g = _g(16)
     kc = torch.randn(2, 40, 128, generator=g).to(torch.bfloat16).to(DEV)
