@@ -1080,22 +1080,45 @@ __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const Flas
     const char* const v_head = g.v_cache + head0 * (2 * D);
 
     // Query operand: token n, dimensions 32 st + 8 kg + [0, 8), in three parts.
+    // fp16 parts hold 24 bits only between 2^-11 and 65504, so the token's
+    // query is first brought to [2^14, 2^15) by a power of two, which goes into
+    // the factor of its scores.
     Frag qa[3][NS];
+    float c = g.scaling * 1.4426950408889634f;  // weights are 2^(c s - c max)
     {
         const float* qp = g.q + ((t < g.tokens ? t : g.tokens - 1) * g.q_heads + h) * D + 8 * kg;
+        float x[NS][8];
 #pragma unroll
         for (int st = 0; st < NS; ++st) {
             const float4 a = *reinterpret_cast<const float4*>(qp + 32 * st);
             const float4 b = *reinterpret_cast<const float4*>(qp + 32 * st + 4);
-            const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            x[st][0] = a.x, x[st][1] = a.y, x[st][2] = a.z, x[st][3] = a.w;
+            x[st][4] = b.x, x[st][5] = b.y, x[st][6] = b.z, x[st][7] = b.w;
+        }
+        if constexpr (CT == NQ_DTYPE_F16) {
+            float top = 0.0f;
+#pragma unroll
+            for (int st = 0; st < NS; ++st)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(x[st][e]));
+            const int shift = 141 - static_cast<int>(__float_as_uint(column_max(top)) >> 23);
+            const int k = shift < 100 ? shift : 100;  // a query below 2^-86 stays smaller than that
+            const float up = __uint_as_float(static_cast<uint32_t>(127 + k) << 23);
+            c *= __uint_as_float(static_cast<uint32_t>(127 - k) << 23);
+#pragma unroll
+            for (int st = 0; st < NS; ++st)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[st][e] *= up;
+        }
+#pragma unroll
+        for (int st = 0; st < NS; ++st)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 uint32_t hh[3];
-                split3_pair<CT>(x[2 * e], x[2 * e + 1], hh);
+                split3_pair<CT>(x[st][2 * e], x[st][2 * e + 1], hh);
 #pragma unroll
                 for (int p = 0; p < 3; ++p) qa[p][st].u[e] = hh[p];
             }
-        }
     }
 
     // This thread's V patch: rows 4 vq + [0, 4), dimensions 8 vc + [0, 8); the
@@ -1160,7 +1183,6 @@ __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const Flas
     };
 
     if (threadIdx.x < HALVES) wild[threadIdx.x] = 0;
-    const float c = g.scaling * 1.4426950408889634f;  // weights are 2^(c s - c max)
     v4f_t o[ND];
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt) o[dt] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};

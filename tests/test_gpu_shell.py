@@ -374,6 +374,24 @@ def test_prompt_attention_infinite_cache_rows(q_heads, kv_heads, head_dim, token
         assert relative_l2(out[finite], expected[finite]) < 1e-5
 
 
+@pytest.mark.parametrize("magnitude", [1e-12, 1e-6, 0.01, 1e5, 1e30])
+@pytest.mark.parametrize("cache_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,tokens,start", [(4, 4, 64, 20, 9), (8, 2, 128, 33, 5), (2, 1, 256, 18, 700)])
+def test_prompt_attention_query_magnitudes(q_heads, kv_heads, head_dim, tokens, start, cache_dtype, magnitude):
+    """The query is fp32: one of any magnitude keeps its 24 bits beside a 16-bit cache (an fp16
+    part ends at 65504 and at steps of 2^-24). Scores are as large as in the tests above."""
+
+    g = _g(20)
+    rows = start + tokens
+    kc = torch.randn(kv_heads, rows, head_dim, generator=g).to(cache_dtype)
+    vc = torch.randn(kv_heads, rows, head_dim, generator=g).to(cache_dtype)
+    q = 2 * magnitude * torch.randn(tokens, q_heads, head_dim, generator=g)
+    scaling = head_dim**-0.5 / magnitude
+    out = ops.launch_attention(q.to(DEV), kc.to(DEV), vc.to(DEV), scaling=scaling, out_dtype=torch.float32,
+                               position=torch.tensor([start], dtype=torch.int32, device=DEV))
+    assert relative_l2(out.cpu(), reference_attention(q, kc, vc, start, scaling)) < 1e-5
+
+
 def test_prompt_attention_tokens_outside_the_cache_are_zero():
     g = _g(16)
     kc = torch.randn(2, 40, 128, generator=g).to(torch.bfloat16).to(DEV)
