@@ -1228,25 +1228,33 @@ __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const Flas
 #pragma unroll
                 for (int j = 0; j < 4; ++j) s[ct][j] = 16 * ct + 4 * kg + j <= seen ? s[ct][j] : -INFINITY;
         }
-        float mx = m;
+        // The weights are relative to the running max; with an fp16 cache to
+        // the tile's own, where it is 2^15, and the tile joins by the factor
+        // `join`: fp16 parts hold 24 bits of what is above 2^-26 of that (2^-11
+        // of the row's largest weight otherwise), and 2^-40 of it below.
+        constexpr bool kOwnMax = CT == NQ_DTYPE_F16;
+        constexpr float kTop = kOwnMax ? 15.0f : 0.0f;
+        float mx = kOwnMax ? -INFINITY : m;
 #pragma unroll
         for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
             for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[ct][j]);
         mx = column_max(mx);
-        const float mc_new = mx == -INFINITY ? 0.0f : mx * c;
+        const float mc_tile = mx == -INFINITY ? 0.0f : fmaf(mx, c, -kTop);
+        const float mc_new = kOwnMax && m > mx ? mc : mc_tile;
         const float keep = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mc - mc_new);
-        m = mx;
+        const float join = kOwnMax && mx != -INFINITY ? __builtin_amdgcn_exp2f(mc_tile - mc_new) : 1.0f;
+        m = kOwnMax ? fmaxf(m, mx) : mx;
         mc = mc_new;
         float lt = 0.0f;
 #pragma unroll
         for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                s[ct][j] = __builtin_amdgcn_exp2f(fmaf(s[ct][j], c, -mc));
+                s[ct][j] = __builtin_amdgcn_exp2f(fmaf(s[ct][j], c, -mc_tile));
                 lt += s[ct][j];
             }
-        l = fmaf(l, keep, lt);
+        l = fmaf(l, keep, kOwnMax ? lt * join : lt);
         Frag pa[3][R / 32];
 #pragma unroll
         for (int ks = 0; ks < R / 32; ++ks)
@@ -1276,7 +1284,8 @@ __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const Flas
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) o[d0 + i][j] = fmaf(o[d0 + i][j], keep, y[i][j]);
+                for (int j = 0; j < 4; ++j)
+                    o[d0 + i][j] = fmaf(o[d0 + i][j], keep, kOwnMax ? y[i][j] * join : y[i][j]);
         }
         if (wild[half]) {
             // The values that store_tile left out, for the tokens that see their rows: in every
@@ -1289,7 +1298,7 @@ __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const Flas
                 for (int ct = 0; ct < NC; ++ct)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) w = rr >> 4 == ct && (rr & 3) == j ? s[ct][j] : w;
-                w = __shfl(w, 16 * ((rr >> 2) & 3) + n, kWave);
+                w = __shfl(w, 16 * ((rr >> 2) & 3) + n, kWave) * join;
                 const uint16_t* vr = reinterpret_cast<const uint16_t*>(v_head) + static_cast<uint32_t>(r) * D + 4 * kg;
 #pragma unroll
                 for (int dt = 0; dt < ND; ++dt)

@@ -392,6 +392,29 @@ def test_prompt_attention_query_magnitudes(q_heads, kv_heads, head_dim, tokens, 
     assert relative_l2(out.cpu(), reference_attention(q, kc, vc, start, scaling)) < 1e-5
 
 
+@pytest.mark.parametrize("cache_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,tokens,start", [(4, 4, 64, 20, 60), (8, 2, 128, 33, 40), (2, 1, 256, 18, 700), (4, 2, 128, 17, 1100)])
+def test_prompt_attention_beside_a_heavy_row(q_heads, kv_heads, head_dim, tokens, start, cache_dtype):
+    """Row 0 takes nearly all of the weight (the others about e^-12 of it) and has no value, so the
+    output is what the light rows leave: their weights keep 24 bits, as the scores do (an fp16
+    part ends at steps of 2^-24). Tolerance as above: scores of 12 are rounded by 1e-6."""
+
+    g = _g(21)
+    rows = start + tokens
+    q = torch.randn(tokens, q_heads, head_dim, generator=g)
+    q[..., 0] = 4.0
+    kc = torch.randn(kv_heads, rows, head_dim, generator=g).to(cache_dtype)
+    kc[:, 0] = 0
+    kc[:, 0, 0] = 3 * head_dim**0.5  # a score of 12, the others about +-1
+    vc = torch.randn(kv_heads, rows, head_dim, generator=g).to(cache_dtype)
+    vc[:, 0] = 0
+    out = ops.launch_attention(q.to(DEV), kc.to(DEV), vc.to(DEV), scaling=head_dim**-0.5, out_dtype=torch.float32,
+                               position=torch.tensor([start], dtype=torch.int32, device=DEV))
+    expected = reference_attention(q, kc, vc, start, head_dim**-0.5)
+    assert expected.abs().max() < 0.02
+    assert relative_l2(out.cpu(), expected) < 1e-5
+
+
 def test_prompt_attention_tokens_outside_the_cache_are_zero():
     g = _g(16)
     kc = torch.randn(2, 40, 128, generator=g).to(torch.bfloat16).to(DEV)
