@@ -6,7 +6,7 @@
 
 namespace nq {
 
-// Scratch bytes one linear needs: less than decode_scratch_bytes (48.5 bytes a
+// Scratch bytes one linear needs: less than decode_scratch_bytes (60.5 bytes a
 // column of x and of the rank against 64), which callers size buffers by.
 int64_t decode_planes_bytes(const nq_linear_desc* d);
 

@@ -1,15 +1,25 @@
 // Decode calls of 9 to 16 tokens: the two GEMMs on fp6 activation planes and
 // fp4 signs (nq_planes.h) with v_mfma_scale_f32_16x16x128_f8f6f4.
 //
-// Four planes: 20 bits, 1.4e-6 rel-L2 on normal rows (the int8 digits of the
-// 1 to 4-token kernels end at 6e-6 to 2e-5, their exponent coming from a bound
-// on the rank intermediate). The operand of 16 rows and a 128-column block is,
-// per plane, 64 lanes' first 16 bytes and then their last 8 (lane 16 g + row
-// holds lane group g's 32 columns); exponents [kb / 4][lane][kb % 4].
+// Five planes, 25 bits below the largest of 32 columns: the int8 digits of the
+// calls of up to eight tokens hold 24 bits of the largest of 512, so no row
+// keeps fewer here, with outlier channels either (4 planes, 20 bits, did:
+// 4096 columns, one of them a thousand times the others, 2.1e-6 rel-L2 in
+// digits, 3.0e-6 in four planes, 1.4e-7 in five; 64 columns 2.0e-7, 1.8e-6,
+// 7e-8; normal rows of 4096 1.6e-5, 1.5e-6, 1.0e-7, the digits' rank
+// intermediate taking its exponent from a bound). The operand of 16 rows and a
+// 128-column block is, per plane, 64 lanes' first 16 bytes and then their last
+// 8 (lane 16 g + row holds lane group g's 32 columns); exponents
+// [kb / 4][lane][kb % 4].
 //
 // k_planes_gemm16: a workgroup takes 32 NG sign rows and its eight waves share
 // the K blocks out in chunks of four (a lane's sign words of a chunk are one
-// 16-byte load, and all of a chunk's loads are issued at once). A wave reads an
+// 16-byte load). With 32 sign rows all of a chunk's loads are issued before its
+// first MFMA, by a scheduling barrier: left alone the compiler interleaves them
+// to save registers, and a chunk takes several round trips (16 tokens, us: 4096
+// -> 4096 r1638 16.9 and 14.4 with it, 10240 -> 2560 r1536 24.7 and 18.6). With
+// 64 the registers that takes halve the workgroups of a CU, which costs more
+// (4096 -> 2 x 12288 r3072 21.5 with it, 19.9 without). A wave reads an
 // operand fragment once for all of its 2 NG tiles, straight from memory:
 // nothing is shared between waves until their sums meet in LDS, added in wave
 // order. GEMM 1's tiles are cut across the sign tiles so that two of them hold
@@ -17,17 +27,16 @@
 // 128-row block, m < 4 and m >= 4), which the workgroup then converts.
 // Bound by latency (three launches, a chunk or two per wave) and, for long
 // rows, by every workgroup reading the whole operand. Against the int8 stages
-// at 16 tokens (us a call): 4096 -> 4096 r1638 15.8 and 29.0, 4096 -> 2 x 12288
-// r3072 20.9 and 29.7, 10240 -> 2560 r1536 22.5 and 23.0, 14336 -> 4096 r2549
-// 26.6 and 29.1; the first's kernels take 4.0, 8.1 and 5.3. GEMM 1 forming its
-// operand from x itself, without k_planes_prep16, was slower (15.6 us against
-// 4.0 + 8.1): every workgroup repeats the conversion.
+// at 16 tokens (us a call): 4096 -> 4096 r1638 14.4 and 28.5, 4096 -> 2 x 12288
+// r3072 19.9 and 27.6, 10240 -> 2560 r1536 18.6 and 22.2, 14336 -> 4096 r2549
+// 22.7 and 28.1. GEMM 1 forming its operand from x itself, without
+// k_planes_prep16, was slower: every workgroup repeats the conversion.
 #include "nq_decode_planes.h"
 #include "nq_planes.h"
 
 namespace {
 
-constexpr int kP = 4;          // planes
+constexpr int kP = 5;          // planes
 constexpr int kWaves = 8;
 constexpr int kM = 16;         // token rows
 
@@ -47,9 +56,11 @@ __global__ __launch_bounds__(kBlock) void k_planes_prep16(const PrepBatch batch)
                      half[0], half[1]);
 }
 
+// Plane PL's product of K block I of a chunk: B scales 2^(-5 PL) are the bytes of `eb` and `eb4`.
 template <int PL, int I>
-__device__ __forceinline__ v4f mfma16_plane(const v8i& a, const v8i& b, const v4f& c, int ea, int eb) {
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 4, I, ea, PL, eb);
+__device__ __forceinline__ v4f mfma16_plane(const v8i& a, const v8i& b, const v4f& c, int ea, int eb, int eb4) {
+    if constexpr (PL < 4) return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 4, I, ea, PL, eb);
+    else return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 4, I, ea, 0, eb4);
 }
 
 template <int NG>
@@ -80,13 +91,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_planes_gemm16(const GemmBatc
         tile_at[t] = static_cast<uint32_t>(c >> 4) * nsc * 64;
         wl[t] = 16 * kg + (c & 15);
     }
-    v4f acc[T];
+    // Planes 2 to 4 sum up apart from the two coarse ones, as in k_sign_gemm
+    // (the matrix core truncates what it adds to an accumulator).
+    v4f acc[2][T];
 #pragma unroll
-    for (int t = 0; t < T; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int t = 0; t < T; ++t) acc[0][t] = acc[1][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     uint32_t sign_mask = 0x88888888u, fp4_one = 0x22222222u;
     constexpr int kE = kPlaneBits;
-    int eb = 127 | (127 - kE) << 8 | (127 - 2 * kE) << 16 | (127 - 3 * kE) << 24;  // B scales 2^(-5p)
-    asm volatile("" : "+v"(sign_mask), "+v"(fp4_one), "+v"(eb));  // keep them in VGPRs
+    int eb = 127 | (127 - kE) << 8 | (127 - 2 * kE) << 16 | (127 - 3 * kE) << 24, eb4 = 127 - 4 * kE;
+    asm volatile("" : "+v"(sign_mask), "+v"(fp4_one), "+v"(eb), "+v"(eb4));  // keep them in VGPRs
     for (int chunk = wave; 4 * chunk < nsc; chunk += kWaves) {
         const int dw = nsc - 4 * chunk < 4 ? nsc - 4 * chunk : 4;
         // A narrow last chunk's words lie closer; the load runs into what follows them, not used.
@@ -106,6 +119,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_planes_gemm16(const GemmBatc
             }
         }
         const int ea = *reinterpret_cast<const int*>(g.a.exps + chunk * 256 + 4 * lane);
+        if constexpr (NG == 1) __builtin_amdgcn_sched_barrier(0);
         each(std::make_integer_sequence<int, 4>{}, [&](auto i_) __attribute__((always_inline)) {
             constexpr int i = decltype(i_)::value;
             if (i >= dw) return;  // uniform
@@ -119,17 +133,18 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_planes_gemm16(const GemmBatc
                 const v8i a = v8i{static_cast<int>(l.x), static_cast<int>(l.y), static_cast<int>(l.z),
                                   static_cast<int>(l.w), static_cast<int>(u.x), static_cast<int>(u.y), 0, 0};
 #pragma unroll
-                for (int t = 0; t < T; ++t) acc[t] = mfma16_plane<f, i>(a, b[t], acc[t], ea, eb);
+                for (int t = 0; t < T; ++t)
+                    acc[f > 1][t] = mfma16_plane<f, i>(a, b[t], acc[f > 1][t], ea, eb, eb4);
             });
         });
     }
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) red[(wave * Q + 4 * t + j) * 64 + lane] = acc[t][j];
+        for (int j = 0; j < 4; ++j) red[(wave * Q + 4 * t + j) * 64 + lane] = acc[0][t][j] + acc[1][t][j];
     __syncthreads();
     // Wave w finishes sums [w NG, + NG): token 4 kg + j of tile t, q = 4 t + j.
-    const int t_own = wave * NG / 4;  // NG <= 4: one tile
+    const int t_own = wave * NG / 4;  // NG <= 2: one tile
     const int64_t col = column(t_own), col_c = col < g.n ? col : g.n - 1;
     const Raw2 cs_raw = load_raw2(g.col_scale, g.col_scale_dtype, col_c);
     const Raw2 bias_raw =
@@ -186,13 +201,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void k_planes_gemm16(const GemmBatc
 }
 
 // One GEMM phase of a batch. 32 sign rows a workgroup keep most CUs busy; a wide
-// phase takes 128 or 64, which read the operand a quarter or half as often (2 x
-// 12288 sign rows at 16 tokens, the call: 20.9 us with 128, 21.1 with 64, 23.7
-// with 32; 4096: 22.9, 18.0, 15.8).
+// phase takes 64, which read the operand half as often (2 x 12288 sign rows at
+// 16 tokens, the call: 19.9 us with 64, 23.7 with 32, 22.4 with 128).
 void launch_phase16(GemmArgs* p, int count, hipStream_t stream) {
     int64_t groups = 0;
     for (int i = 0; i < count; ++i) groups += (p[i].n + 31) / 32;
-    const int ng = groups >= 512 ? 4 : (groups >= 256 ? 2 : 1);
+    const int ng = groups >= 256 ? 2 : 1;
     GemmBatch gb;
     int64_t x = 0;
     for (int i = 0; i < kPrefillBatch; ++i) {
@@ -202,9 +216,7 @@ void launch_phase16(GemmArgs* p, int count, hipStream_t stream) {
         if (i < count) x += p[i].mid.planes ? (4 * p[i].mid_blocks + ng - 1) / ng : (p[i].n + 32 * ng - 1) / (32 * ng);
     }
     const dim3 grid(static_cast<unsigned>(x)), block(kWaves * 64);
-    if (ng == 4)
-        hipLaunchKernelGGL(k_planes_gemm16<4>, grid, block, 0, stream, gb);
-    else if (ng == 2)
+    if (ng == 2)
         hipLaunchKernelGGL(k_planes_gemm16<2>, grid, block, 0, stream, gb);
     else
         hipLaunchKernelGGL(k_planes_gemm16<1>, grid, block, 0, stream, gb);
