@@ -84,10 +84,18 @@ __device__ __forceinline__ int make_planes(v16f a, v16f c, v6u (&w)[P]) {
     }
     const bool finite = top < 0x7f800000u;
     int e = static_cast<int>(top >> 23) - 128;  // 2^e: half the largest value's binade
-    e = e < -100 ? -100 : (finite ? e : 0);
+    e = e < -127 ? -127 : (finite ? e : 0);     // the scale's smallest exponent
+    // A small group is cut from its values times 2^64 (exact), so that the last
+    // plane's unit is a normal number too.
+    const bool small = e < -64;
+    if (small) {
+        const float up = exp2i(64);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) a[i] *= up, c[i] *= up;
+    }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-        const float unit = exp2i(e - kPlaneBits * p);
+        const float unit = exp2i((small ? e + 64 : e) - kPlaneBits * p);
         w[p] = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, c, unit);
         // The conversion's operands outlive it, or the compiler lets its result
         // overlap them, and what is written first is read again (seen in the

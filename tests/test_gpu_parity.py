@@ -467,6 +467,23 @@ def test_two_token_blocks_one_or_two_tiles(out_f, rank, tokens):
     assert float((y.cpu().double() - expected).norm() / expected.norm()) <= 1e-4
 
 
+@pytest.mark.parametrize("exponent", [-60, -90, -104, -112])
+@pytest.mark.parametrize("tokens,operands,bar", [(9, "fp16", 5e-7), (16, "fp16", 5e-7), (24, "fp16", 1e-4), (24, "split", 5e-7), (300, "fp16", 1e-4), (300, "split", 5e-7)])
+def test_planes_of_small_rows(tokens, operands, bar, exponent):
+    """Rows of any magnitude keep their bits: the group's exponent goes down to 2^-127. The bars are
+    those of ordinary rows above; results stay normal fp32 numbers."""
+
+    _say("small rows", tokens, operands, exponent)
+    state = syn.synthetic_packed_layer(syn.LinearShape("blocks.0.mlp.gate_proj", 516, 260, 200), seed=tokens)
+    x = syn.synthetic_activations(tokens, 516, seed=tokens).float() * 2.0**exponent
+    backend = HipPackedBackend(prefill_operands=operands)
+    y = backend.linear(x.cuda(), backend.prepare(state, "cuda"))
+    expected = _exact_linear(state, x)
+    err = float((y.cpu().double() - expected).norm() / expected.norm())
+    print(f"  rel_l2={err:.2e} largest={float(expected.abs().max()):.1e}", flush=True)
+    assert err <= bar
+
+
 def test_prefill_planes_with_an_outlier_channel():
     """One channel a thousand times the others: its group's other values keep
     2^-14 of it, at most sqrt(31) 2^-14 = 3.4e-4 of the channel's own share of
