@@ -170,15 +170,10 @@ void pick_waves(int64_t nc, int tpb, int tb, int& nw, int& kc) {
     }
 }
 
-// The same for the several-token stages of the split launch: at most eight
-// waves; with one token block two chunks per wave per pass when the waves
-// would not cover the chunks (a wave holding two blocks has no registers for a
-// second chunk).
-void pick_waves_multi(int64_t nc, int tb, int& nw, int& kc) {
-    kc = nc > 8 && tb == 1 ? 2 : 1;
-    const int64_t waves = (nc + kc - 1) / kc;
-    nw = static_cast<int>(waves < 8 ? waves : 8);
-}
+// The same for the stages of the split launch at 5 to 8 tokens: at most eight
+// waves of one chunk (a wave holding two token blocks has no registers for a
+// second one).
+int waves_multi(int64_t nc) { return static_cast<int>(nc < 8 ? nc : 8); }
 
 // Dynamic LDS of a stage: per-wave operand areas (stage 1), the partial sums
 // [nc][tw][tb][64], the chunk maxima [nc][tpb * tb] (stage 1) and, for one
@@ -236,12 +231,13 @@ bool planes_path(int64_t tokens) { return tokens >= kPlanesTokens; }
 // Tiles per workgroup of the several-token stages: a wave's A operands (8 KB
 // per block of four tokens per chunk) are shared by its TW tiles, against
 // fewer waves. One token block (stage 2 after the in-kernel staging): four
-// tiles from 4096 waves, two from 2048. Two blocks (stage 0 path): two tiles in
-// both stages (measured best against one and four, per stage, at 8 tokens),
-// one where two would leave more than half of the CUs idle (192 tiles).
-// Against two tiles (us a call at 8 tokens in a graph): stage 1 of 48 tiles
-// 13.7 -> 13.0, of 103 15.5 -> 15.3, of 231 15.7 -> 17.1; stage 2 of 160 tiles
-// with 96 in stage 1 17.3 -> 16.6.
+// tiles from 4096 waves, two from 2048. Two blocks (stage 0 path): two tiles
+// from 193 on, one below, which leaves fewer CUs idle. The line lies where a
+// batch, whose grid is its members x the largest one's tiles, changes sides
+// (one and two tiles, us a call at 8 tokens in a graph): stage 1 of 185 tiles
+// in three members 16.0 and 16.2, of 192 in two 13.0 and 13.2, of 231 in three
+// 17.1 and 15.7. A linear alone would gain from one tile up to 256 (stage 1 of
+// 256 13.0 and 13.3, stage 2 11.5 and 12.3) and loses from 288 on (16.2 and 14.6).
 int pick_tiles_multi(int64_t tiles, int nw, int tb) {
     if (tb > 1) return tiles <= 192 ? 1 : 2;
     const int64_t waves = tiles * nw;
@@ -371,8 +367,9 @@ int plan_shapes(HostBatch& batch, int64_t tokens, int ak, bool fused, Shapes& sh
             s2.tw = tokens == 1 ? pick_tiles(2, tiles2, s2.nw, s2.kc, s2.tb, false)
                                 : pick_tiles_multi(tiles2, s2.nw, s2.tb);
         } else {
-            pick_waves_multi(nc1, s1.tb, s1.nw, s1.kc);
-            pick_waves_multi(nc2, s2.tb, s2.nw, s2.kc);
+            s1.nw = waves_multi(nc1);
+            s2.nw = waves_multi(nc2);
+            s1.kc = s2.kc = 1;
             s1.tw = pick_tiles_multi(tiles1, s1.nw, s1.tb);
             s2.tw = pick_tiles_multi(tiles2, s2.nw, s2.tb);
             // Partial sums within 64 KB of LDS.

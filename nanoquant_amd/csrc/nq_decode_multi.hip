@@ -11,22 +11,13 @@ int go0(const Batch& batch, const LaunchShape& s, hipStream_t stream) {
     return nq::launch_status();
 }
 
-template <int TB, int TW, int KC>
+// Two token blocks in a wave's registers: one chunk per wave and pass.
+template <int TW>
 int go1(const Batch& batch, const LaunchShape& s, hipStream_t stream) {
     constexpr int kThreads = 512;
     if (64 * s.nw > kThreads) return NQ_ERR_LAUNCH;
-    hipLaunchKernelGGL((k_decode_stage1m<TB, TW, KC, kThreads>), s.grid, dim3(64 * s.nw), s.lds, stream, batch);
+    hipLaunchKernelGGL((k_decode_stage1m<2, TW, 1, kThreads>), s.grid, dim3(64 * s.nw), s.lds, stream, batch);
     return nq::launch_status();
-}
-
-template <int TB, int KC>
-int by_tiles(const Batch& batch, const LaunchShape& s, hipStream_t stream) {
-    switch (s.tw) {
-        case 1: return go1<TB, 1, KC>(batch, s, stream);
-        case 2: return go1<TB, 2, KC>(batch, s, stream);
-        case 4: return go1<TB, 4, KC>(batch, s, stream);
-        default: return NQ_ERR_LAUNCH;
-    }
 }
 
 }  // namespace
@@ -42,10 +33,9 @@ int enqueue_stage0(const Batch& batch, const LaunchShape& s, hipStream_t stream)
 }
 
 int enqueue_stage1m(const Batch& batch, const LaunchShape& s, hipStream_t stream) {
-    if (s.tpb != 4) return NQ_ERR_LAUNCH;
-    if (s.tb == 1) return s.kc == 2 ? by_tiles<1, 2>(batch, s, stream) : by_tiles<1, 1>(batch, s, stream);
-    if (s.kc != 1) return NQ_ERR_LAUNCH;  // two token blocks per wave: one chunk per pass
-    if (s.tb == 2) return by_tiles<2, 1>(batch, s, stream);
+    if (s.tpb != 4 || s.tb != 2 || s.kc != 1) return NQ_ERR_LAUNCH;
+    if (s.tw == 1) return go1<1>(batch, s, stream);
+    if (s.tw == 2) return go1<2>(batch, s, stream);
     return NQ_ERR_LAUNCH;
 }
 

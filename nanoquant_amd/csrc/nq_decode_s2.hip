@@ -23,10 +23,10 @@ int by_tiles(const Batch& batch, const LaunchShape& s, hipStream_t stream) {
 
 // Two token blocks (five to eight tokens): one chunk per wave per pass.
 int by_tiles_blocks(const Batch& batch, const LaunchShape& s, hipStream_t stream) {
-    if (s.kc != 1) return NQ_ERR_LAUNCH;
-    if (s.tw == 4) return go<4, 2, 4, 1>(batch, s, stream);
+    if (s.tb != 2 || s.kc != 1) return NQ_ERR_LAUNCH;
+    if (s.tw == 1) return go<4, 2, 1, 1>(batch, s, stream);
     if (s.tw == 2) return go<4, 2, 2, 1>(batch, s, stream);
-    return go<4, 2, 1, 1>(batch, s, stream);
+    return NQ_ERR_LAUNCH;
 }
 
 template <int TW, int KC>

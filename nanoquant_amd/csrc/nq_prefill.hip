@@ -837,11 +837,12 @@ struct Plan {
 // 90-102. 4096 -> 2 x 12288 r3072 at 2048 452, 374, 346, 322; 318-335. Splits
 // pay only for few tokens of long rows (14336 -> 4096 r2549 at 61: 58 us
 // unsplit, 34 with GEMM 1 in eight slices).
-// A small grid goes to k_sign_gemm_few: 256 workgroups of 32 sign rows and 32
-// tokens (64 above 32) or fewer; beyond, every one of them reading all of A
-// costs more (2 x 12288 sign rows, 768 workgroups, at 24 tokens: 27 us against
-// 24), and so do more than 48 K blocks (10240 columns at 61 tokens: 33.5
-// against 28.8) unless the operand is the smallest (at 24: 23.1 and 26.9).
+// A small grid goes to k_sign_gemm_few, without a search: 256 workgroups of 32
+// sign rows and 32 tokens (64 above 32, which read the signs and A half as
+// often) or fewer; beyond, every one of them reading all of A costs more (2 x
+// 12288 sign rows, 768 workgroups, at 24 tokens: 27 us against 24), and so do
+// more than 48 K blocks (10240 columns at 61 tokens: 33.5 against 28.8) unless
+// the operand is the smallest (at 24: 23.1 and 26.9).
 constexpr int64_t kFewWgs = 256, kFewBlocks = 48;
 constexpr double kCus = 256.0;
 constexpr int64_t kMinSliceBlocks = 4;
@@ -854,6 +855,15 @@ Plan plan_phase(int count, const int64_t* k_blocks, const int64_t* n, const int6
     const int wide = planes == kPlanesSplit ? 1 : 0;
     int64_t kb_max = 1;
     for (int i = 0; i < count; ++i) kb_max = k_blocks[i] > kb_max ? k_blocks[i] : kb_max;
+    const bool few64 = tokens > 32 && planes == kPlanes;  // five planes of 64 rows would spill
+    int64_t few_wgs = 0;
+    for (int i = 0; i < count; ++i) few_wgs += (n[i] + 31) / 32;
+    few_wgs *= (tokens + (few64 ? 63 : 31)) / (few64 ? 64 : 32);
+    if (few_wgs <= kFewWgs && (kb_max <= kFewBlocks || (tokens <= 32 && planes == kPlanes))) {
+        best.shape = few64 ? kFew64 : kFew32;
+        for (int i = 0; i < count; ++i) best.k_per_split[i] = k_blocks[i], best.slices[i] = 1;
+        return best;
+    }
     for (int id = 0; id < kShapes; ++id) {
         const Shape& sh = kShape[id];
         if (sh.alone[wide] == 0.0 || (id > 0 && tokens <= kShape[id].rows / 2)) continue;
@@ -883,46 +893,40 @@ Plan plan_phase(int count, const int64_t* k_blocks, const int64_t* n, const int6
             if (best_us < 0.0 || us < best_us) best = p, best_us = us;
         }
     }
-    const bool few64 = tokens > 32 && planes == kPlanes;  // five planes of 64 rows would spill
-    int64_t few_wgs = 0;
-    for (int i = 0; i < count; ++i) few_wgs += (n[i] + 31) / 32;
-    few_wgs *= (tokens + (few64 ? 63 : 31)) / (few64 ? 64 : 32);
-    if (few_wgs <= kFewWgs && (kb_max <= kFewBlocks || (tokens <= 32 && planes == kPlanes))) {
-        best = Plan{};
-        best.shape = few64 ? kFew64 : kFew32;
-        for (int i = 0; i < count; ++i) best.k_per_split[i] = k_blocks[i], best.slices[i] = 1;
-    }
     return best;
 }
 
+// NQ_ERR_LAUNCH for a shape that the operands have no kernel for (kShape's zeros keep plans off them).
 template <int P>
-void launch_gemm(int shape, dim3 grid, hipStream_t stream, const GemmBatch& gb) {
+int launch_gemm(int shape, dim3 grid, hipStream_t stream, const GemmBatch& gb) {
     switch (shape) {
-        case kShape32x128: hipLaunchKernelGGL((k_sign_gemm<1, 1, 1, P>), grid, dim3(kBlock), 0, stream, gb); break;
-        case kShape64x128: hipLaunchKernelGGL((k_sign_gemm<1, 2, 1, P>), grid, dim3(kBlock), 0, stream, gb); break;
-        case kShape64x256:
-            if constexpr (P == kPlanesSplit) hipLaunchKernelGGL((k_sign_gemm<1, 2, 2, P>), grid, dim3(kBlock), 0, stream, gb);
-            break;
-        case kShape128x128:
-            if constexpr (P == kPlanes) hipLaunchKernelGGL((k_sign_gemm<2, 2, 2, P>), grid, dim3(kBlock), 0, stream, gb);
-            break;
+        case kShape32x128: hipLaunchKernelGGL((k_sign_gemm<1, 1, 1, P>), grid, dim3(kBlock), 0, stream, gb); return NQ_OK;
+        case kShape64x128: hipLaunchKernelGGL((k_sign_gemm<1, 2, 1, P>), grid, dim3(kBlock), 0, stream, gb); return NQ_OK;
         case kFew32:
             hipLaunchKernelGGL((k_sign_gemm_few<1, P>), grid, dim3(kFewWaves * 64), 0, stream, gb);
-            break;
-        case kFew64:
-            if constexpr (P == kPlanes)
-                hipLaunchKernelGGL((k_sign_gemm_few<2, P>), grid, dim3(kFewWaves * 64), 0, stream, gb);
-            break;
-        default:
-            if constexpr (P == kPlanes) hipLaunchKernelGGL((k_sign_gemm<2, 2, 4, P>), grid, dim3(kBlock), 0, stream, gb);
-            break;
+            return NQ_OK;
+        default: break;
     }
+    if constexpr (P == kPlanesSplit) {
+        if (shape != kShape64x256) return NQ_ERR_LAUNCH;
+        hipLaunchKernelGGL((k_sign_gemm<1, 2, 2, P>), grid, dim3(kBlock), 0, stream, gb);
+    } else {
+        if (shape == kShape128x128)
+            hipLaunchKernelGGL((k_sign_gemm<2, 2, 2, P>), grid, dim3(kBlock), 0, stream, gb);
+        else if (shape == kShape128x256)
+            hipLaunchKernelGGL((k_sign_gemm<2, 2, 4, P>), grid, dim3(kBlock), 0, stream, gb);
+        else if (shape == kFew64)
+            hipLaunchKernelGGL((k_sign_gemm_few<2, P>), grid, dim3(kFewWaves * 64), 0, stream, gb);
+        else
+            return NQ_ERR_LAUNCH;
+    }
+    return NQ_OK;
 }
 
 // One launch of a phase's GEMMs and, when any member's K is split, one launch
 // of the reductions.
 template <int P>
-void launch_phase(GemmArgs* p, const Plan& plan, int count, int64_t tokens, hipStream_t stream) {
+int launch_phase(GemmArgs* p, const Plan& plan, int count, int64_t tokens, hipStream_t stream) {
     const bool few = plan.shape >= kShapes;
     const int64_t rows = few ? (plan.shape == kFew32 ? 32 : 64) : kShape[plan.shape].rows;
     GemmBatch gb;
@@ -950,13 +954,14 @@ void launch_phase(GemmArgs* p, const Plan& plan, int count, int64_t tokens, hipS
         return dim3(static_cast<unsigned>(cols), static_cast<unsigned>(rows < kRowsPerGridZ ? rows : kRowsPerGridZ),
                     static_cast<unsigned>((rows + kRowsPerGridZ - 1) / kRowsPerGridZ));
     };
-    launch_gemm<P>(plan.shape, grid_of(x, (tokens + rows - 1) / rows), stream, gb);
-    if (rx == 0) return;
+    const int st = launch_gemm<P>(plan.shape, grid_of(x, (tokens + rows - 1) / rows), stream, gb);
+    if (st != NQ_OK || rx == 0) return st;
     const dim3 grid = grid_of(rx, mid ? (tokens + 15) / 16 : tokens);
     if (mid)
         hipLaunchKernelGGL(k_reduce_mid<P>, grid, dim3(kBlock), 0, stream, rb);
     else
         hipLaunchKernelGGL(k_reduce_splits, grid, dim3(kBlock), 0, stream, rb);
+    return NQ_OK;
 }
 
 int planes_of(const nq_linear_desc* d) {
@@ -1106,7 +1111,8 @@ int launch_prefill_planes(const nq_linear_desc* const* descs, int count, const v
         a.mid_blocks = geo[i].nsc2;
         a.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(scratch[i]) + sl[i].partial);
     }
-    launch_phase<P>(g, plan_phase(count, kb, n, cap, tokens, P), count, tokens, stream);
+    const int st = launch_phase<P>(g, plan_phase(count, kb, n, cap, tokens, P), count, tokens, stream);
+    if (st != NQ_OK) return st;
 
     // GEMM 2: y = s_out * (lm · U±1ᵀ) + salient columns + bias.
     for (int i = 0; i < count; ++i) {
@@ -1137,8 +1143,8 @@ int launch_prefill_planes(const nq_linear_desc* const* descs, int count, const v
         a.out_dtype = y_dtype;
         a.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(scratch[i]) + sl[i].partial);
     }
-    launch_phase<P>(g, plan_phase(count, kb, n, cap, tokens, P), count, tokens, stream);
-    return nq::launch_status();
+    const int st2 = launch_phase<P>(g, plan_phase(count, kb, n, cap, tokens, P), count, tokens, stream);
+    return st2 != NQ_OK ? st2 : nq::launch_status();
 }
 
 }  // namespace
