@@ -1816,23 +1816,30 @@ int64_t proj_workgroups(int64_t vocab, int64_t hidden) {
 int attention_blocks(int64_t max_positions) { return static_cast<int>((max_positions + kSeqBlock - 1) / kSeqBlock); }
 
 // How a prompt attention of `groups` workgroups (four units each) over up to
-// `tiles` cache tiles is laid out.
+// `tiles` cache tiles of `rows` rows is laid out.
 struct FlashPlan {
     int halves;
     int64_t splits, tiles_per_split;
 };
 
 // Fewer than 128 workgroups leave most of the chip idle: their cache goes to
-// several (two tiles each or more, up to 16 and to 512 workgroups in all) when
-// it is long enough to pay for the merge: 17 tokens after 1000 (16 workgroups)
-// 13 us split, 30 us not; 128 after 3000 (64) 39 and 75 us; 256 after 1000
-// (128) 35 us either way; 64 after none (32, 640-row cache) 10 and 9 us. Below
-// 512, eight waves share a workgroup's cache between them (17 after 1000: 30
-// us against 35 in four; 1024 tokens, 512 workgroups: 44 either way).
-FlashPlan flash_plan(int64_t groups, int64_t tiles) {
+// several (64 rows each or more, as the workspace holds; up to 16 and to 512
+// workgroups in all) where it pays for the merge: from two tiles on up to 32
+// workgroups, from eight beyond. Not split and split, bf16, 32 / 8 heads of
+// 128 where not said: 17 tokens after 100 with 16 / 4 heads (8 workgroups) 10.8
+// and 9.5 us, after 300 (16) 15.8 and 10.5; 64 after 250 (32) 16.2 and 12.8;
+// 33 after 300 with 16 / 8 16.4 and 10.6; 100 after none (56, 300-row cache)
+// 10.7 and 11.4; 128 after 3000 (64) 75 and 39; 256 after 1000 (128) 35 either
+// way. Two tiles each or more lost where a split could have one (17 after 1000
+// 13.4 and 12.2). Below 512 workgroups that are not split, eight waves share a
+// workgroup's cache between them (17 after 1000: 30 us against 35 in four; 1024
+// tokens, 512 workgroups: 44 either way).
+FlashPlan flash_plan(int64_t groups, int64_t tiles, int64_t rows) {
     FlashPlan p;
-    int64_t want = groups < 128 && tiles >= 8 ? 512 / groups : 1;
-    want = want < tiles / 2 ? want : tiles / 2;
+    const bool split = groups <= 32 ? tiles >= 2 : groups < 128 && tiles >= 8;
+    const int64_t most = tiles * rows / kSeqBlock;
+    int64_t want = split ? 512 / groups : 1;
+    want = want < most ? want : most;
     want = want < 16 ? want : 16;
     want = want > 1 ? want : 1;
     p.tiles_per_split = (tiles + want - 1) / want;
@@ -1854,7 +1861,7 @@ int launch_prompt_attention(const float* q, const void* kc, const void* vc, int6
     const int64_t groups = quads * kv_heads;
     if (groups > 0x7fffffff) return NQ_ERR_SHAPE;
     const int64_t tiles = (max_positions + R - 1) / R;
-    const FlashPlan plan = flash_plan(groups, tiles);
+    const FlashPlan plan = flash_plan(groups, tiles, R);
     FlashArgs a;
     a.q = q;
     a.k_cache = static_cast<const char*>(kc);

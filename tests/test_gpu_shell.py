@@ -228,6 +228,13 @@ def test_attention(tokens, start, q_heads, kv_heads, head_dim, cache_dtype):
         (20, 0, 32, 8, 128, 4096),
         (17, 1000, 16, 4, 128, 1200),
         (18, 2100, 8, 2, 256, 2200),
+        # two, three and five tiles (of 32 rows: two and three blocks of 64), a part each; one short of two
+        (17, 60, 16, 4, 128, 77),
+        (17, 120, 16, 4, 128, 140),
+        (33, 250, 16, 8, 128, 300),
+        (30, 70, 8, 4, 256, 100),
+        (18, 130, 8, 4, 256, 150),
+        (17, 40, 16, 4, 128, 63),
         # enough tokens for one half per workgroup
         (1040, 37, 32, 8, 128, 1077),
         (1030, 5, 16, 16, 64, 1050),
