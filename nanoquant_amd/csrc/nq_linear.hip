@@ -402,7 +402,6 @@ int validate(const nq_linear_desc* d) {
 // the prefill path's scratch from lm on.
 struct WorkspaceLayout {
     int64_t lm_offset, patch_offset, decode_offset, total;
-    int64_t reserved;  // what nq_linear_static holds against its limit
 };
 
 WorkspaceLayout workspace_layout(const nq_linear_desc* d, int64_t tokens) {
@@ -410,12 +409,8 @@ WorkspaceLayout workspace_layout(const nq_linear_desc* d, int64_t tokens) {
     w.patch_offset = 0;
     w.lm_offset = align256(tokens * d->patch_rank * 4);
     w.decode_offset = w.lm_offset + align256(tokens * d->rank * 4);
-    if (nq::decode_path_applies(d, tokens)) {
-        w.total = w.reserved = w.decode_offset + nq::decode_scratch_bytes(d, tokens);
-    } else {
-        w.total = w.lm_offset + nq::prefill_scratch_bytes(d, tokens);
-        w.reserved = w.lm_offset + nq::prefill_reserved_bytes(d, tokens);
-    }
+    w.total = nq::decode_path_applies(d, tokens) ? w.decode_offset + nq::decode_scratch_bytes(d, tokens)
+                                                 : w.lm_offset + nq::prefill_scratch_bytes(d, tokens);
     return w;
 }
 
@@ -477,7 +472,8 @@ extern "C" int64_t nq_linear_workspace_bytes(const nq_linear_desc* desc, int64_t
 
 int64_t nq::linear_reserved_bytes(const nq_linear_desc* desc, int64_t tokens) {
     if (validate(desc) != NQ_OK || tokens <= 0) return -1;
-    return workspace_layout(desc, tokens).reserved;
+    if (nq::decode_path_applies(desc, tokens)) return workspace_layout(desc, tokens).total;
+    return align256(tokens * desc->patch_rank * 4) + nq::prefill_reserved_bytes(desc, tokens);
 }
 
 extern "C" int nq_linear(const nq_linear_desc* d, const void* x, int32_t x_dtype, int64_t tokens,

@@ -977,8 +977,9 @@ struct Scratch {
 // their rows' scales and partials for a split of 128 x 128 blocks (64-row up to
 // 64 tokens) by a latency model of K steps of 1 us (0.5), 512 resident
 // workgroups (1024), a reduction of 6 us (3) and 8 TB/s: callers size buffers
-// and nq_linear_static takes or refuses calls by them. The planes come out of
-// the same bytes; what they leave holds the partials.
+// and nq_linear_static takes or refuses calls by them. Where the planes take
+// more than the 16-bit operands, the sizes grow so that the partials keep
+// theirs; where they take less, what they leave holds more partials.
 int64_t reserved_slices(int64_t tokens, int64_t k_blocks, int64_t n) {
     const bool small = tokens <= 64;
     const int64_t tiles = (tokens + 127) / 128 * ((n + 127) / 128);
@@ -996,6 +997,21 @@ int64_t reserved_slices(int64_t tokens, int64_t k_blocks, int64_t n) {
     return best;
 }
 
+int64_t reserved_partial_bytes(const nq_linear_desc* d, int64_t tokens) {
+    const Geometry g = geometry(d);
+    const int64_t s1 = reserved_slices(tokens, g.nsc1, d->rank), s2 = reserved_slices(tokens, g.nsc2, d->out_features);
+    const int64_t p1 = s1 > 1 ? s1 * tokens * d->rank : 0, p2 = s2 > 1 ? s2 * tokens * d->out_features : 0;
+    return a256(4 * (p1 > p2 ? p1 : p2));
+}
+
+// Everything else that is reserved: the fp32 rank intermediate, 16-bit operands, row scales.
+int64_t reserved_operand_bytes(const nq_linear_desc* d, int64_t tokens) {
+    const Geometry g = geometry(d);
+    const int64_t parts = d->prefill_operands == NQ_PREFILL_FP16_SPLIT ? 2 : 1;
+    return a256(tokens * d->rank * 4) + a256(tokens * g.nsc1 * kBK * 2 * parts) +
+           a256(tokens * g.nsc2 * kBK * 2 * parts) + 2 * a256(tokens * 4);
+}
+
 Scratch scratch_layout(const nq_linear_desc* d, int64_t tokens) {
     const Geometry g = geometry(d);
     const int64_t groups = (tokens + kRows - 1) / kRows, bytes = 2 * planes_of(d) * kPlaneBytes;
@@ -1005,8 +1021,11 @@ Scratch scratch_layout(const nq_linear_desc* d, int64_t tokens) {
     s.planes2 = s.exps1 + a256(g.nsc1 * groups * 128);
     s.exps2 = s.planes2 + a256(g.nsc2 * groups * bytes);
     s.partial = s.exps2 + a256(g.nsc2 * groups * 128);
-    const int64_t reserved = nq::prefill_reserved_bytes(d, tokens);
-    s.total = s.partial > reserved ? s.partial : reserved;
+    // Room for the reserved partials beside the planes, which take more than
+    // 16-bit operands where few tokens fill whole groups of 32 rows (without
+    // it 9000 -> 300 r240 at 33 tokens had no room to split K: 36 us, 20 with).
+    const int64_t operands = reserved_operand_bytes(d, tokens);
+    s.total = (s.partial > operands ? s.partial : operands) + reserved_partial_bytes(d, tokens);
     s.partial_elems = (s.total - s.partial) / 4;
     return s;
 }
@@ -1017,12 +1036,7 @@ namespace nq {
 
 int64_t prefill_reserved_bytes(const nq_linear_desc* d, int64_t tokens) {
     if (!d->tiles) return a256(tokens * d->rank * 4);
-    const Geometry g = geometry(d);
-    const int64_t parts = d->prefill_operands == NQ_PREFILL_FP16_SPLIT ? 2 : 1;
-    const int64_t s1 = reserved_slices(tokens, g.nsc1, d->rank), s2 = reserved_slices(tokens, g.nsc2, d->out_features);
-    const int64_t p1 = s1 > 1 ? s1 * tokens * d->rank : 0, p2 = s2 > 1 ? s2 * tokens * d->out_features : 0;
-    return a256(tokens * d->rank * 4) + a256(tokens * g.nsc1 * kBK * 2 * parts) +
-           a256(tokens * g.nsc2 * kBK * 2 * parts) + 2 * a256(tokens * 4) + a256(4 * (p1 > p2 ? p1 : p2));
+    return reserved_operand_bytes(d, tokens) + reserved_partial_bytes(d, tokens);
 }
 
 int64_t prefill_scratch_bytes(const nq_linear_desc* d, int64_t tokens) {

@@ -7,6 +7,9 @@ import ctypes
 import re
 from pathlib import Path
 
+import pytest
+import torch
+
 from nanoquant_amd.runtime import _native
 
 HEADERS = sorted((Path(__file__).resolve().parent.parent / "include").glob("*.h"))
@@ -39,6 +42,26 @@ def test_host_only_entry_points():
     assert lib.nq_linear_workspace_bytes(ctypes.byref(desc), 1) == -1
     assert lib.nq_linear(ctypes.byref(desc), None, 0, 1, None, 0, None, 0, None) == _native.NQ_ERR_SHAPE
     assert lib.nq_unpack_signs(None, 1, 1, 1, 0, None, None) == _native.NQ_ERR_ARGUMENT
+
+
+@pytest.mark.parametrize("operands,planes", [(_native.NQ_PREFILL_FP16, 3), (_native.NQ_PREFILL_FP16_SPLIT, 5)])
+@pytest.mark.parametrize("tokens", [17, 33, 40, 64, 65, 100])
+@pytest.mark.parametrize("in_f,out_f,rank", [(9000, 300, 240), (14336, 300, 512), (8200, 512, 500)])
+def test_workspace_leaves_room_to_split_long_rows(in_f, out_f, rank, tokens, operands, planes):
+    """A few tokens of long rows and few sign rows need K split: beside the operands' planes (whole
+    groups of 32 rows, 1536 bytes a 64-column step and plane) the workspace holds at least eight
+    slices of GEMM 1's fp32 sums."""
+
+    lib = _native.load()
+    desc = _native.LinearDesc()
+    desc.in_features, desc.out_features, desc.rank = in_f, out_f, rank
+    desc.scale_dtype = _native.dtype_code(torch.float16)
+    desc.prefill_operands = operands
+    for name in ("right_words", "left_words", "scale_pre", "scale_mid", "scale_post", "tiles"):
+        setattr(desc, name, 256)  # an address: the size depends on its presence alone
+    size = int(lib.nq_linear_workspace_bytes(ctypes.byref(desc), tokens))
+    blocks, groups = -(-in_f // 128) + -(-rank // 128), -(-tokens // 32)
+    assert size >= blocks * groups * (2 * planes * 1536 + 128) + 8 * tokens * rank * 4
 
 
 def test_tile_layout_restatement_is_a_bit_permutation():
