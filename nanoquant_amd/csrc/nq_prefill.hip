@@ -532,7 +532,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_sign_gemm(const GemmBatch batch) 
 // the 32 rows of one exponent group of the rank intermediate: tile rows
 // 16 m + 4 g + b of its 128-column block, in lane 4 m + b. Bound by latency.
 // Calls with both GEMMs here and on k_sign_gemm: 4096 -> 4096 r1638 at 24
-// tokens 15.9 and 24.6 us, at 61 21.9 and 26.4; at 128 23.6 and 27.8.
+// tokens 15.9 and 24.6 us, at 61 16.9 and 26.4; at 128 23.6 and 27.8.
 constexpr int kFewWaves = 8;
 
 template <int II, int P>
@@ -837,13 +837,17 @@ struct Plan {
 // 90-102. 4096 -> 2 x 12288 r3072 at 2048 452, 374, 346, 322; 318-335. Splits
 // pay only for few tokens of long rows (14336 -> 4096 r2549 at 61: 58 us
 // unsplit, 34 with GEMM 1 in eight slices).
-// A small grid goes to k_sign_gemm_few, without a search: 256 workgroups of 32
-// sign rows and 32 tokens (64 above 32, which read the signs and A half as
-// often) or fewer; beyond, every one of them reading all of A costs more (2 x
-// 12288 sign rows, 768 workgroups, at 24 tokens: 27 us against 24), and so do
-// more than 48 K blocks (10240 columns at 61 tokens: 33.5 against 28.8) unless
-// the operand is the smallest (at 24: 23.1 and 26.9).
-constexpr int64_t kFewWgs = 256, kFewBlocks = 48;
+// A small grid goes to k_sign_gemm_few, without a search: at most 256
+// workgroups (one a CU) of 32 sign rows and 32 tokens, or else 64 tokens, which
+// read the signs half as often (32 against 64 tokens a workgroup where both
+// fit: 4096 -> 4096 r1638 at 61 tokens 16.9 and 22.2 us, Q/K/V of 4096 21.4 and
+// 24.7, 1152 -> 6912 r768 at 200 17.3 and 18.6). Beyond, every workgroup reading
+// all of A costs more (2 x 12288 sign rows, 768 workgroups, at 24 tokens: 27 us
+// against 24). More than 48 K blocks go there up to 64 tokens of three planes
+// (against split K: 10240 -> 2560 r1536 at 24 tokens 23.1 and 26.9, at 61 22.1
+// and 26.2, 9000 -> 300 r240 19.6 and 21.6; five planes 28.8 and 26.8 at 17, 26.5
+// and 23.5 the other way).
+constexpr int64_t kFewWgs = 256, kFewBlocks = 48, kFewTokens = 64;
 constexpr double kCus = 256.0;
 constexpr int64_t kMinSliceBlocks = 4;
 constexpr double kReduceUs = 5.0;
@@ -855,11 +859,12 @@ Plan plan_phase(int count, const int64_t* k_blocks, const int64_t* n, const int6
     const int wide = planes == kPlanesSplit ? 1 : 0;
     int64_t kb_max = 1;
     for (int i = 0; i < count; ++i) kb_max = k_blocks[i] > kb_max ? k_blocks[i] : kb_max;
-    const bool few64 = tokens > 32 && planes == kPlanes;  // five planes of 64 rows would spill
     int64_t few_wgs = 0;
     for (int i = 0; i < count; ++i) few_wgs += (n[i] + 31) / 32;
-    few_wgs *= (tokens + (few64 ? 63 : 31)) / (few64 ? 64 : 32);
-    if (few_wgs <= kFewWgs && (kb_max <= kFewBlocks || (tokens <= 32 && planes == kPlanes))) {
+    const int64_t few32_wgs = few_wgs * ((tokens + 31) / 32);
+    const bool few64 = few32_wgs > kFewWgs && planes == kPlanes;  // five planes of 64 rows would spill
+    if ((few64 ? few_wgs * ((tokens + 63) / 64) : few32_wgs) <= kFewWgs &&
+        (kb_max <= kFewBlocks || (tokens <= kFewTokens && planes == kPlanes && !few64))) {
         best.shape = few64 ? kFew64 : kFew32;
         for (int i = 0; i < count; ++i) best.k_per_split[i] = k_blocks[i], best.slices[i] = 1;
         return best;
