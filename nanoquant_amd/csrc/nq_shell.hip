@@ -1287,9 +1287,9 @@ __global__ __launch_bounds__(HALVES * 256, 2) void k_prompt_attention(const Flas
                 for (int j = 0; j < 4; ++j)
                     o[d0 + i][j] = fmaf(o[d0 + i][j], keep, kOwnMax ? y[i][j] * join : y[i][j]);
         }
-        if (wild[half]) {
-            // The values that store_tile left out, for the tokens that see their rows: in every
-            // tile with rows past `first`, also one whose rows all of this unit's tokens see.
+        if (row0 + R - 1 > first && wild[half]) {
+            // The values that store_tile left out, for the tokens that see their rows (also in a
+            // tile whose rows all of this unit's tokens see).
             const int r_end = last < row0 + R - 1 ? last : row0 + R - 1;
             for (int r = row0 > first ? row0 : first + 1; r <= r_end; ++r) {
                 const int rr = r - row0;
@@ -1823,28 +1823,28 @@ struct FlashPlan {
 };
 
 // Fewer than 128 workgroups leave most of the chip idle: their cache goes to
-// several (64 rows each or more, as the workspace holds; up to 16 and to 512
-// workgroups in all) where it pays for the merge: from two tiles on up to 32
-// workgroups, from eight beyond. Not split and split, bf16, 32 / 8 heads of
-// 128 where not said: 17 tokens after 100 with 16 / 4 heads (8 workgroups) 10.8
-// and 9.5 us, after 300 (16) 15.8 and 10.5; 64 after 250 (32) 16.2 and 12.8;
-// 33 after 300 with 16 / 8 16.4 and 10.6; 100 after none (56, 300-row cache)
-// 10.7 and 11.4; 128 after 3000 (64) 75 and 39; 256 after 1000 (128) 35 either
-// way. Two tiles each or more lost where a split could have one (17 after 1000
-// 13.4 and 12.2). Below 512 workgroups that are not split, eight waves share a
-// workgroup's cache between them (17 after 1000: 30 us against 35 in four; 1024
-// tokens, 512 workgroups: 44 either way).
+// several, which pays for the merge where it is long enough: up to 32
+// workgroups 64 rows each or more (as the workspace holds), 256 workgroups in
+// all; from eight tiles on, up to 128 workgroups, two tiles each or more, 512 in
+// all; 16 parts at most. Not split and split, bf16, 32 / 8 heads of 128 where
+// not said: 17 tokens after 100 with 16 / 4 heads (8 workgroups) 10.8 and 9.5
+// us, after 300 (16) 15.8 and 10.5; 64 after 250 (32) 16.2 and 12.8; 33 after
+// 300 with 16 / 8 16.4 and 10.6; 100 after none (56, 300-row cache) 10.7 and
+// 11.4; 128 after 3000 (64) 75 and 39; 256 after 1000 (128) 35 either way. Two
+// tiles a part and one: 17 after 1000 with 16 / 4 13.4 and 12.2, but 33 after
+// 500 with 64 / 8 (48, of which 480) 15.5 and 18.3. Below 512 workgroups that
+// are not split, eight waves share a workgroup's cache between them where it
+// has two tiles (17 after 1000: 30 us against 35 in four; 1024 tokens, 512
+// workgroups: 44 either way; 17 of one tile 13.0 against 11.2).
 FlashPlan flash_plan(int64_t groups, int64_t tiles, int64_t rows) {
     FlashPlan p;
-    const bool split = groups <= 32 ? tiles >= 2 : groups < 128 && tiles >= 8;
-    const int64_t most = tiles * rows / kSeqBlock;
-    int64_t want = split ? 512 / groups : 1;
-    want = want < most ? want : most;
-    want = want < 16 ? want : 16;
-    want = want > 1 ? want : 1;
-    p.tiles_per_split = (tiles + want - 1) / want;
+    const auto least = [](int64_t a, int64_t b) { return a < b ? a : b; };
+    const int64_t ones = groups <= 32 ? least(256 / groups, tiles * rows / kSeqBlock) : 1;
+    const int64_t twos = groups < 128 && tiles >= 8 ? least(512 / groups, tiles / 2) : 1;
+    const int64_t want = least(ones > twos ? ones : twos, 16);
+    p.tiles_per_split = want > 1 ? (tiles + want - 1) / want : tiles;
     p.splits = (tiles + p.tiles_per_split - 1) / p.tiles_per_split;
-    p.halves = groups < 512 && p.splits == 1 ? 2 : 1;
+    p.halves = groups < 512 && p.splits == 1 && tiles > 1 ? 2 : 1;
     return p;
 }
 
@@ -1915,7 +1915,10 @@ int launch_attention(const float* q, const void* kc, const void* vc, int64_t tok
                      const int32_t* position, int64_t max_positions, float scaling, void* out, int odt, float* ml,
                      float* acc, hipStream_t st) {
     if constexpr (CT != NQ_DTYPE_F32) {
-        if (tokens > 1)
+        // One token, and two with heads of 256 (8 / 4 heads, after 40, 500 and
+        // 2000: 10.7, 16.3 and 20.8 us in one pass, 9.2, 15.9 and 17.6 in
+        // blocks; of 128, 32 / 8 heads, after 500 9.1 and 10.8), take the blocks.
+        if (tokens > (D == 256 ? 2 : 1))
             return launch_prompt_attention<D, CT>(q, kc, vc, tokens, q_heads, kv_heads, position, max_positions,
                                                   scaling, out, odt, ml, st);
     }

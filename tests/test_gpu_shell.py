@@ -235,6 +235,10 @@ def test_attention(tokens, start, q_heads, kv_heads, head_dim, cache_dtype):
         (30, 70, 8, 4, 256, 100),
         (18, 130, 8, 4, 256, 150),
         (17, 40, 16, 4, 128, 63),
+        # two and three tokens, in blocks (heads of 256) and in one pass
+        (2, 77, 8, 4, 256, 100),
+        (3, 77, 8, 4, 256, 100),
+        (2, 130, 16, 8, 128, 140),
         # enough tokens for one half per workgroup
         (1040, 37, 32, 8, 128, 1077),
         (1030, 5, 16, 16, 64, 1050),
