@@ -54,7 +54,7 @@ typedef enum nq_status {
                                 NQ_STATIC_SCRATCH_BYTES of workspace         */
 } nq_status;
 
-/* Size of the per-device static scratch array of nq_linear_static (4 MiB). */
+/* What nq_linear_static holds calls against (4 MiB); its array has three times as much. */
 #define NQ_STATIC_SCRATCH_BYTES (4 << 20)
 
 /* Launch structure of the tiled decode path (tokens <= 16).
@@ -62,6 +62,9 @@ typedef enum nq_status {
  *     intermediate, the kernel boundary publishes it, stage 2 reads it).
  *   NQ_DECODE_FUSED: one kernel; stage-2 workgroups wait on a grid-wide
  *     counter in the tiles header that stage-1 workgroups signal.
+ * From five tokens the split form has a kernel more, which forms x * s_in's
+ * operands; from nine both forms run the same three kernels (6-bit operand
+ * planes: FUSED is one kernel up to eight tokens only).
  * Both give bit-identical results. No reference counterpart (the reference
  * always launches two Triton kernels, cuda_kernels.py:816-874). */
 typedef enum nq_decode_launch {
@@ -72,11 +75,13 @@ typedef enum nq_decode_launch {
 /* Operands of the prefill path's MFMA GEMMs (tokens > 16): the activations
  * and the rank intermediate as sums of 6-bit planes of five bits each, with one
  * exponent for 32 columns of a row.
- *   NQ_PREFILL_FP16: three planes, an error of at most 2^-14 of the largest of
- *     the 32 values (about 6e-5 rel-L2 against the fp32 forward; never more
- *     than fp16 operands have, hence the name).
- *   NQ_PREFILL_FP16_SPLIT: five planes (about 1e-7), for callers whose errors
- *     compound (a decoder's prompt pass).
+ *   NQ_PREFILL_FP16: three planes, each value off by at most 2^-14 of the
+ *     largest of its 32 (about 6e-5 rel-L2 against the fp32 forward, 1.1e-4
+ *     beside a channel a thousand times the others; fp16 operands, after which
+ *     it is named, have 3e-4 to 5e-4, though a small value beside a large one
+ *     keeps fewer bits here).
+ *   NQ_PREFILL_FP16_SPLIT: five planes, 2^-24 (about 1e-7), for callers whose
+ *     errors compound (a decoder's prompt pass).
  * Batch members must agree. No reference counterpart (the reference's
  * kernels compute in the activation dtype, cuda_kernels.py:65-162). */
 typedef enum nq_prefill_operands {
@@ -229,14 +234,18 @@ int nq_linear(const nq_linear_desc* desc, const void* x, int32_t x_dtype,
 /* nq_linear without a workspace argument, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid allocation). No reference counterpart. The workspace is a
- * file-scope device array of NQ_STATIC_SCRATCH_BYTES per GPU, held until the
- * process ends; calls whose nq_linear_workspace_bytes exceeds it return
- * NQ_ERR_SCRATCH (decode token counts fit any Qwen3/Llama-sized layer;
- * larger prefill calls need nq_linear). The limit counts a prefill call's
- * operands as 16-bit values of the call's rows; where whole groups of 32 rows
- * make nq_linear_workspace_bytes larger than that, the array holds them too. Allocates nothing itself. All calls
- * on one GPU share the array: calls that overlap in time on one GPU race and
- * must not be issued (one stream, or streams ordered by the caller). */
+ * file-scope device array of 3 * NQ_STATIC_SCRATCH_BYTES (12 MiB) per GPU, held
+ * until the process ends. A call of up to 16 tokens is taken if its
+ * nq_linear_workspace_bytes are at most NQ_STATIC_SCRATCH_BYTES (any
+ * Qwen3/Llama-sized layer). A prefill call is held against the same limit with
+ * its operands counted as 16-bit values (two each when split) of its rows,
+ * beside an fp32 rank intermediate and split-K partials: at most
+ * nq_linear_workspace_bytes and at least a third of them, so a call whose
+ * nq_linear_workspace_bytes fit the limit is always taken and one that needs
+ * more than three times the limit never. Calls beyond return NQ_ERR_SCRATCH and
+ * launch nothing. Allocates nothing itself. All calls on one GPU share the
+ * array: calls that overlap in time on one GPU race and must not be issued (one
+ * stream, or streams ordered by the caller). */
 int nq_linear_static(const nq_linear_desc* desc, const void* x, int32_t x_dtype,
                      int64_t tokens, void* y, int32_t y_dtype, void* stream);
 

@@ -84,8 +84,10 @@ int64_t nq_attention_workspace_bytes(int64_t tokens, int32_t q_heads, int32_t he
  *   out[t, h, :] = softmax(scaling * q[t, h, :] · K[g, 0..p, :]) · V[g, 0..p, :]
  * q fp32 [tokens, q_heads, head_dim]; out F32/F16/BF16 [tokens, q_heads *
  * head_dim]. Softmax in fp32, in a fixed order (deterministic): a running
- * softmax over a 16-bit cache from two tokens on (three with heads of 256), otherwise 64-row blocks whose
- * partial results are merged in block order. Replaces
+ * softmax over a 16-bit cache from two tokens on (three with heads of 256),
+ * otherwise 64-row blocks whose partial results are merged in block order.
+ * Queries may have any magnitude; infinities and NaN in the cache do what fp32
+ * arithmetic does with them for the tokens that see their row. Replaces
  * launch_decode_attention (src/nanoquant/runtime/cuda_kernels.py:448-544),
  * generalised from its pinned one-kv-head, 64-row geometry. */
 int nq_attention(const float* q, const void* k_cache, const void* v_cache, int32_t cache_dtype,

@@ -219,9 +219,9 @@ constexpr int64_t kStage0Tokens = 5;
 bool stage0_path(int64_t tokens) { return tokens >= kStage0Tokens; }
 
 // Tokens from which both launches take the fp6 planes (nq_decode_planes.hip):
-// with three or four blocks of four tokens the int8 digits are 64 bytes a
-// column for each block against 60 for all sixteen rows, and a plane's MFMA
-// covers them at once. At 9 and 16 tokens (us a call, digits against planes): 4096 ->
+// with three or four blocks of four tokens the int8 digits take as many MFMAs
+// and 64 bytes a column, the planes 60 for all sixteen rows, which one MFMA a
+// plane covers. At 9 and 16 tokens (us a call, digits against planes): 4096 ->
 // 4096 r1638 20.8 / 14.1 and 28.5 / 14.4, 10240 -> 2560 r1536 21.4 / 18.2 and
 // 22.2 / 18.6. Five to eight tokens stay on digits (two blocks; planes would be
 // padded to twice their rows).

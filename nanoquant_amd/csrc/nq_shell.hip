@@ -887,7 +887,8 @@ __global__ __launch_bounds__(kMfmaHeads * kWave) void k_decode_attention_mfma(
 }
 
 // ---------------------------------------------------------------------------
-// Prompt attention on MFMA (16-bit cache, two tokens or more, any head_dim):
+// Prompt attention on MFMA (16-bit cache, two tokens or more, three with
+// heads of 256):
 // one pass over the cache with a running softmax, so no per-block partials
 // leave the chip. A unit is 16 tokens of one q head; a workgroup takes four
 // consecutive units of one kv head (the heads of a token tile, or, with fewer
@@ -907,14 +908,20 @@ __global__ __launch_bounds__(kMfmaHeads * kWave) void k_decode_attention_mfma(
 //   x 8 dimensions through registers), so an A fragment is one 16-byte read.
 // A tile's weighted values are summed on their own (small parts first) and
 // join the running output with one rounding: against 64 bits the output is
-// 1.1e-7 - 2.4e-7 off (rel-L2), 1.9e-7 - 4.0e-7 with per-block partials.
+// 0.9e-7 - 3.6e-7 off (rel-L2; fp16 cache 1.5e-7 - 4.3e-7), 2.6e-7 - 5.8e-7
+// with per-block partials.
+//   What the parts cannot do as fp32 does: an infinity in the cache (elements
+// that come out infinite or NaN are computed again at the end) and, with an
+// fp16 cache, magnitudes (the query and each tile's weights are brought to the
+// range where three fp16 parts hold 24 bits).
 // Bound by the matrix cores and the softmax beside them: 96 MFMAs (16 cycles)
 // and about 310 VALU instructions (four) per 16 tokens x 64 rows x 128
-// dimensions; 35% of the time is MFMA at 1531 tokens. Measured, 32 q heads,
-// 8 kv heads of 128, bf16 (per-block partials and a merge before): 512 tokens
-// 20 us (54), 1531 tokens after 517 cached 123 us (521), 16 / 8 heads 700
-// after 200 32 us (214), 8 / 4 heads of 256 700 tokens 51 us (181). Forming
-// the next tile's scores among this tile's softmax was slower (142 us): the
+// dimensions; 35% of the time is MFMA at 1531 tokens. Measured in a graph, 32 q
+// heads, 8 kv heads of 128, bf16 (per-block partials and a merge before): 512
+// tokens 21.5 us (56), 1531 tokens after 517 cached 116 us (520), 16 / 8 heads
+// 700 after 200 31 us (203), 8 / 4 heads of 256 700 tokens 43 us (176); with an
+// fp16 cache 22.6 (45), 124 (406), 32 (184) and 45 us (155). Forming the next
+// tile's scores among this tile's softmax was slower (142 against 123 us): the
 // registers spill. So were three waves a SIMD (241 us).
 constexpr int kFlashTokens = 16;      // tokens per unit (B columns)
 constexpr int kFlashUnits = 4;        // units per workgroup

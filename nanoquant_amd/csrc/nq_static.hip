@@ -1,9 +1,9 @@
 // nq_linear_static: nq_linear for callers that cannot allocate device memory
 // (code under HIP graph capture that may not call hipMalloc, tight serving
 // loops, harnesses that forbid allocation). The workspace nq_linear takes as
-// an argument is instead a file-scope device array of NQ_STATIC_SCRATCH_BYTES
-// bytes: every GPU the library runs on holds its own copy until the process
-// ends. Nothing in it needs to start at zero (every kernel writes the
+// an argument is instead a file-scope device array of three times
+// NQ_STATIC_SCRATCH_BYTES (12 MiB): every GPU the library runs on holds its own
+// copy until the process ends. Nothing in it needs to start at zero (every kernel writes the
 // workspace bytes it later reads), so no call clears it. Calls share the
 // array: two calls that overlap in time on one GPU (different streams without
 // ordering) race on it and must not be issued.

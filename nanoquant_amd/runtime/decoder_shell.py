@@ -259,11 +259,11 @@ class PackedDecoder:
         self.cache_dtype = cache_dtype
         # The prompt pass's errors reach every later token through the KV cache
         # and compound over the layers. With fp32 activations it takes split
-        # prefill operands (five 6-bit planes, all of fp32's 24 bits);
-        # with 16-bit activations, which the shell rounds to 8 (bf16) or 11
-        # (fp16) bits before every linear, three planes (14 bits below the
-        # largest of 32 values) add less than that rounding and take three
-        # fifths of the prompt's MFMA work.
+        # prefill operands (five 6-bit planes, 2^-24 of the largest of 32
+        # values); with 16-bit activations, which the shell rounds to 8 (bf16)
+        # or 11 (fp16) bits before every linear, three planes (2^-14 of it) add
+        # less than that rounding on hidden states and take three fifths of the
+        # prompt's MFMA work.
         operands = "split" if activation_dtype == torch.float32 else "fp16"
         self.backend = backend or HipPackedBackend(prefill_operands=operands)
         dev = self.device

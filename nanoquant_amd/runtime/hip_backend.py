@@ -154,12 +154,15 @@ class HipPackedBackend:
         """``tiled_decode`` prepares the MFMA tile layout (decode and prefill
         kernels); without it every call takes the canonical-word fp32 path.
         ``decode_launch``: ``"split"`` runs the two decode stages as two
-        kernels, ``"fused"`` as one kernel with an in-kernel grid handoff.
+        kernels (three from five tokens), ``"fused"`` as one kernel with an
+        in-kernel grid handoff up to eight tokens; from nine both run the same
+        three kernels.
         ``prefill_operands`` (above 16 tokens): ``"fp16"`` carries the
-        prefill GEMMs' activations and rank intermediate in three 6-bit planes
-        (about 6e-5 rel-L2 per linear, within what fp16 operands have);
-        ``"split"`` in five (about 1e-7), for callers whose errors compound
-        through many layers."""
+        prefill GEMMs' activations and rank intermediate in three 6-bit planes,
+        each value to 2^-14 of the largest of its 32 columns (about 6e-5 rel-L2
+        per linear, where fp16 operands have 3e-4); ``"split"`` in five, to
+        2^-24 (about 1e-7), for callers whose errors compound through many
+        layers."""
 
         if decode_launch not in _DECODE_LAUNCH:
             raise ValueError(f"decode_launch must be one of {sorted(_DECODE_LAUNCH)}")
