@@ -68,6 +68,23 @@ def test_static_entry_point_matches_nq_linear_on_shrinking_calls():
         assert torch.equal(again, ref)
 
 
+@pytest.mark.parametrize("in_f,out_f,rank,tokens", [(14336, 1024, 400, 33), (28000, 512, 600, 17)])
+def test_static_entry_point_holds_what_its_rule_takes(in_f, out_f, rank, tokens):
+    """Prefill calls whose workspace is beyond NQ_STATIC_SCRATCH_BYTES but whose 16-bit sizes are not:
+    taken, and the array holds them."""
+
+    _say("static", in_f, out_f, rank, tokens)
+    shape = syn.LinearShape("blocks.0.mlp.down_proj", in_f, out_f, rank)
+    layer = HipPackedBackend().prepare(syn.synthetic_packed_layer(shape, seed=syn.BASE_SEED + 320), "cuda")
+    need = int(_native.load().nq_linear_workspace_bytes(ctypes.byref(layer.payload.desc), tokens))
+    assert _native.NQ_STATIC_SCRATCH_BYTES < need <= 3 * _native.NQ_STATIC_SCRATCH_BYTES
+    x = syn.synthetic_activations(tokens, in_f, seed=320, device="cuda")
+    st_ref, ref = _call(layer, x, static=False)
+    st, got = _call(layer, x, static=True)
+    assert st_ref == _native.NQ_OK and st == _native.NQ_OK, (st_ref, st)
+    assert torch.equal(got, ref)
+
+
 def test_static_entry_point_rejects_calls_beyond_its_scratch():
     backend = HipPackedBackend()
     shape = syn.qwen3_8b_layer()[4]  # gate 4096 -> 12288 r3072 at 64 tokens: 16.6 MiB
